@@ -61,6 +61,9 @@ struct Member {
   int rk = 0;      // rotation kernel (RotKernel)
   bool tune_pending = false;  // rk to be measured at the start of the first solve
   int phase = 1;   // 0: mixed bulk, 1: FP64 (host view)
+  int pairs = 0;   // blocks per k that a rotation by pairs forms (0: the mesh has no pairing)
+  bool paired = false;  // the loaded M0 holds the pairs' identity
+  int* pair_flag = nullptr;  // device result of k_check_pairs
   int stage = 0;   // 0 idle, 1 queued, 2 running, 3 finished
   w90gpu_control ctl{};
   double wbtot = 0.0;
@@ -158,6 +161,7 @@ int max_panels(int nw) {
 // A contiguous range of an item list with the launch shape its kernels need.
 struct Seg {
   int off = 0, n = 0, nnmax = 0, npanmax = 0;
+  int nbmax = 0;             // most blocks per k that a rotation forms (nnmax, or half of it by pairs)
   int nwmin = 0, nwmax = 0;  // num_wann range of the items (0, 0 when empty)
 };
 
@@ -181,7 +185,7 @@ void one_group_lists(Lists& L, int g0, int q0, int n, int nn, int npan, int nw) 
         const bool after = c > kGroupClass[g0] || (c == kGroupClass[g0] && (q > q0 || (q == q0 && g > g0)));
         L.seg[g][q] = Seg{after ? n : 0, 0, 0, 0};
       }
-  L.seg[g0][q0] = Seg{0, n, nn, npan, nw, nw};
+  L.seg[g0][q0] = Seg{0, n, nn, npan, nn, nw, nw};
 }
 
 struct Pool {
@@ -320,7 +324,9 @@ struct Layout {
   }
 };
 
-size_t problem_layout(int nw, int nk, int nn, int num_iter, Layout& lay) {
+// pairs: with the tables of the rotation by pairs (not in the fixed scratch
+// of w90gpu_omega_noalloc, which never rotates).
+size_t problem_layout(int nw, int nk, int nn, int num_iter, Layout& lay, bool pairs = true) {
   const size_t nw2 = (size_t)nw * nw;
   const size_t mb = nw2 * nn * nk * sizeof(cplx);
   const size_t ub = nw2 * nk * sizeof(cplx);
@@ -358,6 +364,11 @@ size_t problem_layout(int nw, int nk, int nn, int num_iter, Layout& lay) {
   lay.add((size_t)nk * nn * sizeof(int));                   // nnl
   lay.add((size_t)nk * nn * 3 * sizeof(double));            // bk
   lay.add((size_t)nn * sizeof(double));                     // wb
+  if (pairs && wann_class(nw) >= 1) {
+    lay.add((size_t)nk * nn * sizeof(int));                 // bord
+    lay.add((size_t)nk * nn * sizeof(int));                 // mate
+    lay.add(sizeof(int));                                   // pair_flag
+  }
   return lay.total;
 }
 
@@ -595,6 +606,53 @@ void member_bind(Member* m, char* a, const Layout& lay) {
   p.nnl = (const int*)(a + lay.off[i++]);
   p.bk = (const double*)(a + lay.off[i++]);
   p.wb = (const double*)(a + lay.off[i++]);
+  p.npair = 0;
+  p.bord = p.mate = nullptr;
+  if (i < lay.n) {
+    p.bord = (const int*)(a + lay.off[i++]);
+    p.mate = (const int*)(a + lay.off[i++]);
+    m->pair_flag = (int*)(a + lay.off[i++]);
+  }
+}
+
+// Pairs of the k-mesh for the rotation by pairs: mate[k][b] = k' nn + b'
+// with k' = nnl(k, b), nnl(k', b') = k and bk(k', b') = -bk(k, b); bord
+// lists for each k the b whose vector points into the upper half space
+// first.  nnl as [k][b], 0-based.  Returns nntot/2, or 0 when some block has
+// no mate (an odd or one-sided set of neighbours).
+int find_pairs(int nk, int nn, const int* nnl, const double* bk, std::vector<int>& bord, std::vector<int>& mate) {
+  bord.assign((size_t)nk * nn, -1);
+  mate.assign((size_t)nk * nn, -1);
+  for (int k = 0; k < nk; ++k) {
+    int nfirst = 0, nlast = nn;
+    for (int b = 0; b < nn; ++b) {
+      const size_t kb = (size_t)k * nn + b;
+      const double* v = bk + 3 * kb;
+      const double tol = 1e-6 * std::sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+      const int k2 = nnl[kb];
+      for (int b2 = 0; b2 < nn; ++b2) {
+        const size_t kb2 = (size_t)k2 * nn + b2;
+        const double* v2 = bk + 3 * kb2;
+        if (nnl[kb2] != k || !(std::fabs(v[0] + v2[0]) <= tol && std::fabs(v[1] + v2[1]) <= tol &&
+                               std::fabs(v[2] + v2[2]) <= tol))
+          continue;
+        if (mate[kb] >= 0) return 0;  // two candidates
+        mate[kb] = (int)kb2;
+      }
+      if (mate[kb] < 0 || mate[kb] == (int)kb) return 0;
+      const int i = std::fabs(v[0]) > tol ? 0 : std::fabs(v[1]) > tol ? 1 : 2;
+      if (v[i] > 0) bord[(size_t)k * nn + nfirst++] = b;
+      else bord[(size_t)k * nn + --nlast] = b;
+    }
+    if (2 * nfirst != nn) return 0;
+  }
+  // exactly one block of each pair is formed
+  std::vector<char> first((size_t)nk * nn, 0);
+  for (int k = 0; k < nk; ++k)
+    for (int j = 0; j < nn / 2; ++j) first[(size_t)k * nn + bord[(size_t)k * nn + j]] = 1;
+  for (size_t kb = 0; kb < first.size(); ++kb)
+    if (mate[mate[kb]] != (int)kb || first[kb] == first[mate[kb]]) return 0;
+  return nn / 2;
 }
 
 State state_template(const Member* m, int first_pass, double omega_invariant) {
@@ -756,6 +814,18 @@ int engine_add(Engine* E, const w90gpu_problem* prob, const w90gpu_control* ctl,
   std::vector<int> hn((size_t)m->nk * m->nn);
   for (int k = 0; k < m->nk; ++k)
     for (int b = 0; b < m->nn; ++b) hn[(size_t)k * m->nn + b] = prob->nnlist[k + (size_t)m->nk * b] - 1;
+  std::vector<int> bord, mate;
+  if (m->p.bord) {
+    m->pairs = find_pairs(m->nk, m->nn, hn.data(), prob->bk, bord, mate);
+    if (m->pairs > 0 &&
+        (hipMemcpyAsync((void*)m->p.bord, bord.data(), bord.size() * sizeof(int), hipMemcpyHostToDevice, E->stream) !=
+             hipSuccess ||
+         hipMemcpyAsync((void*)m->p.mate, mate.data(), mate.size() * sizeof(int), hipMemcpyHostToDevice, E->stream) !=
+             hipSuccess)) {
+      set_error(ctx, "upload of the pair tables failed");
+      return fail(W90GPU_ERR_FATAL);
+    }
+  }
   const State s = state_template(m, 1, 0.0);
   if (hipMemcpyAsync((void*)m->p.nnl, hn.data(), hn.size() * sizeof(int), hipMemcpyHostToDevice, E->stream) !=
           hipSuccess ||
@@ -785,7 +855,16 @@ int member_upload(Engine* E, Member* m, const double* m_matrix, const double* u_
   const size_t ub = (size_t)m->nw * m->nw * m->nk * sizeof(cplx);
   HIPCHK(E->ctx, hipMemcpyAsync(m->M0, m_matrix, mb, hipMemcpyHostToDevice, E->copy));
   HIPCHK(E->ctx, hipMemcpyAsync(m->U0, u_matrix, ub, hipMemcpyHostToDevice, E->copy));
+  int flag = m->pairs > 0 ? 1 : 0;
+  if (flag) {
+    HIPCHK(E->ctx, hipMemcpyAsync(m->pair_flag, &flag, sizeof(int), hipMemcpyHostToDevice, E->copy));
+    hipLaunchKernelGGL(k_check_pairs, dim3((unsigned)(m->nk * m->pairs)), dim3(W90_NT), 0, E->copy, m->p, m->pairs,
+                       m->pair_flag);
+    HIPCHK(E->ctx, hipGetLastError());
+    HIPCHK(E->ctx, hipMemcpyAsync(&flag, m->pair_flag, sizeof(int), hipMemcpyDeviceToHost, E->copy));
+  }
   HIPCHK(E->ctx, hipStreamSynchronize(E->copy));
+  m->paired = flag != 0;
   return W90GPU_OK;
 }
 
@@ -817,6 +896,7 @@ void build_lists(const std::vector<Member*>& ms, F prec_of, std::vector<Item>& i
           for (int k = 0; k < m->nk; ++k) items.push_back(Item{m->slot, k});
           s.nnmax = std::max(s.nnmax, m->nn);
           s.npanmax = std::max(s.npanmax, rot_panels(m->rk, m->nw));
+          s.nbmax = std::max(s.nbmax, q == 0 && m->p.npair > 0 ? m->p.npair : m->nn);
           s.nwmin = s.nwmin ? std::min(s.nwmin, m->nw) : m->nw;
           s.nwmax = std::max(s.nwmax, m->nw);
         }
@@ -903,10 +983,11 @@ Seg class_prec_range(const Lists& L, int c, int q) {
 template <class T2>
 void launch_rot_kernel(hipStream_t s, const Prob* P, const Item* it, const Seg& g, int rk, int mode) {
   // MFMA GEMM tiles; gridDim.y covers b and the tiles of a block
-  const dim3 g2(g.n, g.nnmax * g.npanmax);
+  const int nb = mode == MODE_INIT ? g.nnmax : g.nbmax;
+  const dim3 g2(g.n, nb * g.npanmax);
   // one tile per block: both products in one launch, XCD-aware
   // one-dimensional grid (see k_rot_fused)
-  const dim3 gb((unsigned)(8 * ((g.n + 7) / 8) * g.nnmax));
+  const dim3 gb((unsigned)(8 * ((g.n + 7) / 8) * nb));
   if (rk == RK_W16) {
     hipLaunchKernelGGL(k_rotate_w16<T2>, dim3(g.n), dim3(64 * g.nnmax), rotate_w16_lds<T2>(g.nnmax), s, P, it, g.n,
                        mode);
@@ -920,16 +1001,16 @@ void launch_rot_kernel(hipStream_t s, const Prob* P, const Item* it, const Seg& 
   }
   switch (rk) {
     case RK_FUSED32:
-      hipLaunchKernelGGL((k_rot_fused<T2, 32>), gb, dim3(256), 0, s, P, it, g.n, g.nnmax, mode);
+      hipLaunchKernelGGL((k_rot_fused<T2, 32>), gb, dim3(256), 0, s, P, it, g.n, nb, mode);
       break;
     case RK_FUSED64:
-      hipLaunchKernelGGL((k_rot_fused<T2, 64>), gb, dim3(256), 0, s, P, it, g.n, g.nnmax, mode);
+      hipLaunchKernelGGL((k_rot_fused<T2, 64>), gb, dim3(256), 0, s, P, it, g.n, nb, mode);
       break;
     case RK_FUSED48:
-      hipLaunchKernelGGL((k_rot_fused<T2, 48>), gb, dim3(FusedWaves<48>::NT), 0, s, P, it, g.n, g.nnmax, mode);
+      hipLaunchKernelGGL((k_rot_fused<T2, 48>), gb, dim3(FusedWaves<48>::NT), 0, s, P, it, g.n, nb, mode);
       break;
     case RK_DIRECT64:
-      hipLaunchKernelGGL(k_rot_direct<T2>, gb, dim3(256), 0, s, P, it, g.n, g.nnmax, mode);
+      hipLaunchKernelGGL(k_rot_direct<T2>, gb, dim3(256), 0, s, P, it, g.n, nb, mode);
       break;
     case RK_GEMM64:
       hipLaunchKernelGGL((k_rot_gemm<T2, 1, 64>), g2, dim3(256), 0, s, P, it, g.n, mode);
@@ -1172,6 +1253,13 @@ int tune_pending(Engine* E, const std::vector<Member*>& ms) {
 int enqueue_start(Engine* E, const std::vector<Member*>& ms) {
   int rc = tune_pending(E, ms);
   if (rc) return rc;
+  // rotation by pairs or block by block, as the loaded overlaps allow
+  for (Member* m : ms) {
+    const int np = m->paired ? m->pairs : 0;
+    if (np == m->p.npair) continue;
+    m->p.npair = np;
+    HIPCHK(E->ctx, hipMemcpyAsync(E->d_probs + m->slot, &m->p, sizeof(Prob), hipMemcpyHostToDevice, E->stream));
+  }
   Lists L;
   rc = aux_lists(E, ms, L);
   if (rc) return rc;
@@ -1535,7 +1623,7 @@ ScratchLayout scratch_layout(int nw, int nk, int nn, Layout& lay) {
   s.plist = s.items + align_up(sizeof(Item) * (size_t)nk);
   s.raw = s.plist + align_up(sizeof(int));
   s.arena = s.raw + align_up(sizeof(int) * (size_t)nk * nn);
-  s.total = s.arena + problem_layout(nw, nk, nn, 0, lay);
+  s.total = s.arena + problem_layout(nw, nk, nn, 0, lay, false);
   return s;
 }
 

@@ -71,6 +71,7 @@ __device__ __forceinline__ cplx c_div(cplx a, cplx b) {
 __device__ __forceinline__ double c_abs2(cplx a) { return a.x * a.x + a.y * a.y; }
 
 // FP32 complex (storage of the mixed bulk phase)
+__device__ __forceinline__ float2 c_conj(float2 a) { return make_float2(a.x, -a.y); }
 __device__ __forceinline__ float2 c_add(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 c_mul(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
@@ -216,6 +217,12 @@ struct Prob {
                               // (0: the final reduction sums the per-k vectors itself)
   // npan: tiles of the MFMA rotation per block M(k,b) (num_wann > 16)
   const int* nnl;     // [k][b] 0-based neighbour
+  // FP64 rotation by pairs (see rot_pairs): npair blocks (k, b) per k are
+  // rotated, b = bord[k][j] for j < npair, and each writes block mate[k][b]
+  // too; npair = 0: every block is rotated by itself
+  int npair, pad2;
+  const int* bord;    // [k][j] the b of k that are rotated first, then the others
+  const int* mate;    // [k][b] k' nn + b' with k' = k + b and k' + b' = k
   const double* bk;   // [k][b][3]
   const double* wb;   // [b]
   cplx* M[2];         // [k][b][nw*nw] column-major blocks, FP64
@@ -517,6 +524,78 @@ __device__ __forceinline__ const T2* rot_src(const Prob& p, int mode, int cur) {
 __device__ __forceinline__ const cplx* rot_factor(const Prob& p, int, int) { return p.E; }
 
 // --------------------------------------------------------- M rotation
+
+// Overlaps come in adjoint pairs, M(k+b, -b) = M(k, b)^+, and the rotation
+// keeps them so: E_{k+b}^+ M(k,b)^+ E_k = (E_k^+ M(k,b) E_{k+b})^+.  Where
+// the loaded M holds the identity to rounding (k_check_pairs), the FP64
+// rotation above 16 bands forms one block of each pair and stores it twice,
+// the second time conjugate-transposed with its phases negated: half of the
+// MFMA products, which bound the kernel, and half of the reads of M.
+// Measured per rotation, every block formed -> by pairs: 64 bands, 800 k,
+// nntot 12 690 -> 419 us; 44, 343 k, 8 115 -> 78; 27, 216 k, 12 49 -> 38; 91,
+// 216 k, 6 372 -> 220.  FP32 storage (the mixed bulk phase) rotates every
+// block; up to 16 bands one workgroup forms all blocks of a k and its sums.
+template <class T2>
+__device__ __forceinline__ int rot_pairs(const Prob& p) {
+  return std::is_same<T2, cplx>::value ? p.npair : 0;
+}
+// Block of slot j of item k, or -1 past the blocks this rotation forms;
+// *mate is the block that receives the adjoint (-1: none).
+template <class T2>
+__device__ __forceinline__ int rot_slot(const Prob& p, int k, int j, int* mate) {
+  const int np = rot_pairs<T2>(p);
+  *mate = -1;
+  if (np == 0) return j < p.nn ? j : -1;
+  if (j >= np) return -1;
+  const int b = p.bord[(size_t)k * p.nn + j];
+  *mate = p.mate[(size_t)k * p.nn + b];
+  return b;
+}
+
+// Whether M0 holds M(mate) = M(k,b)^+ for every pair: workgroup (k, j) of a
+// problem compares one pair and clears *flag when an element differs by more
+// than 2 num_wann eps of the block's largest modulus, the rounding bound of
+// the products that formed the overlaps and of one rotation (so taking one
+// block of the pair for the other moves the result no more than a rotation
+// does).  NaN fails the test.  One pass over M0 through 32 x 32 tiles (the
+// transposed element of each comes from LDS): 0.2 ms for 64 bands, 800 k,
+// nntot 12, once per load.
+__global__ void __launch_bounds__(W90_NT) k_check_pairs(Prob p, int npair, int* flag) {
+  constexpr int TS = 32, RS = W90_NT / TS;
+  const int nw = p.nw, nn = p.nn;
+  const int k = blockIdx.x / npair, j = blockIdx.x % npair;
+  if (k >= p.nk) return;
+  const size_t b = p.bord[(size_t)k * nn + j];
+  const cplx* X = p.M0 + ((size_t)k * nn + b) * p.nw2;
+  const cplx* Y = p.M0 + (size_t)p.mate[(size_t)k * nn + b] * p.nw2;
+  __shared__ cplx ty[TS][TS + 1];
+  __shared__ double red[W90_NT];
+  const int tr = threadIdx.x % TS, tc = threadIdx.x / TS;
+  double top = 0.0, off = 0.0;
+  bool bad = false;
+  const int nt = (nw + TS - 1) / TS;
+  for (int t = 0; t < nt * nt; ++t) {
+    const int r0 = (t % nt) * TS, c0 = (t / nt) * TS;
+    __syncthreads();
+    for (int i = 0; i < TS; i += RS) {
+      const int r = c0 + tr, c = r0 + tc + i;  // tile (J, I) of Y
+      if (r < nw && c < nw) ty[tc + i][tr] = Y[r + (size_t)c * nw];
+    }
+    __syncthreads();
+    for (int i = 0; i < TS; i += RS) {
+      const int r = r0 + tr, c = c0 + tc + i;
+      if (r >= nw || c >= nw) continue;
+      const cplx x = X[r + (size_t)c * nw], y = ty[tr][tc + i];
+      const double d = fmax(fabs(x.x - y.x), fabs(x.y + y.y)), a = fmax(fabs(x.x), fabs(x.y));
+      if (!(d <= 1e300) || !(a <= 1e300)) bad = true;
+      off = fmax(off, d);
+      top = fmax(top, a);
+    }
+  }
+  off = block_max(off, red);
+  top = block_max(top, red);
+  if (bad || !(off <= 2.0 * nw * 2.220446049250313e-16 * top)) *flag = 0;
+}
 
 // Tiles per block M(k,b) of the MFMA rotation at most: 32 x 32 panels over
 // 256 bands.

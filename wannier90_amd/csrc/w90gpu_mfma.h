@@ -174,8 +174,8 @@ __host__ __device__ __forceinline__ int gemm_tiles(int nw) {
 // block (k, b) by the workgroup (256 threads): operands and scratch as in
 // k_rot_gemm, LDS passed in.
 template <class T2, int STAGE, int GT>
-__device__ __forceinline__ void rot_gemm_tile(const Prob& p, int k, int b, int tile, int row0, int col0, int mode,
-                                              int cur, typename Real<T2>::type (*As)[W90_GK][GT + 1],
+__device__ __forceinline__ void rot_gemm_tile(const Prob& p, int k, int b, int mate, int tile, int row0, int col0,
+                                              int mode, int cur, typename Real<T2>::type (*As)[W90_GK][GT + 1],
                                               typename Real<T2>::type (*Bs)[W90_GK][GT + 1], double* red) {
   constexpr int FR = GT / 32;  // fragments per wavefront along rows and columns
   typedef typename Real<T2>::type R;
@@ -272,6 +272,7 @@ __device__ __forceinline__ void rot_gemm_tile(const Prob& p, int k, int b, int t
 
   double od = 0.0, all = 0.0;
   T2* out = (STAGE == 1) ? Tm : mbuf<T2>(p, dst) + kb * nw2;
+  T2* outm = mbuf<T2>(p, dst) + (mate >= 0 ? (size_t)mate * nw2 : 0);
 #pragma unroll
   for (int fi = 0; fi < FR; ++fi)
 #pragma unroll
@@ -286,14 +287,20 @@ __device__ __forceinline__ void rot_gemm_tile(const Prob& p, int k, int b, int t
           v.y = C[fi][fj].im(i);
           out[r + (size_t)c * nw] = v;
           if (STAGE == 2) {
+            if (mate >= 0) outm[c + (size_t)r * nw] = c_conj(v);
             const cplx vw = c_wide(v);
             const double a2 = c_abs2(vw);
             all += a2;
             if (r != c) {
               od += a2;
             } else {
-              p.ln[dst][kb * nw + r] = atan2(vw.y, vw.x);
+              const double l = atan2(vw.y, vw.x);
+              p.ln[dst][kb * nw + r] = l;
               p.d2[kb * nw + r] = a2;
+              if (mate >= 0) {
+                p.ln[dst][(size_t)mate * nw + r] = -l;
+                p.d2[(size_t)mate * nw + r] = a2;
+              }
             }
           }
         }
@@ -303,6 +310,12 @@ __device__ __forceinline__ void rot_gemm_tile(const Prob& p, int k, int b, int t
     if (tid == 0) {
       p.part_od[kb * p.npan + tile] = od;
       p.part_all[kb * p.npan + tile] = all;
+      if (mate >= 0) {  // tile (J, I) of the adjoint block
+        const int nt1 = (nw + GT - 1) / GT;
+        const size_t q = (size_t)mate * p.npan + tile / nt1 + (tile % nt1) * nt1;
+        p.part_od[q] = od;
+        p.part_all[q] = all;
+      }
     }
   }
 }
@@ -322,12 +335,15 @@ __global__ void __launch_bounds__(256, 2) k_rot_gemm(const Prob* probs, const It
   const int ntl = nt1 * nt1;
   const int by = blockIdx.y;
   if (by >= nn * ntl) return;
-  const int b = by / ntl, tile = by % ntl;
+  const int tile = by % ntl;
+  int mate;
+  const int b = rot_slot<T2>(p, it.k, by / ntl, &mate);
+  if (b < 0) return;
   const int row0 = (tile % nt1) * GT, col0 = (tile / nt1) * GT;
   __shared__ R As[2][W90_GK][GT + 1];  // [re/im][k][row]
   __shared__ R Bs[2][W90_GK][GT + 1];  // [re/im][k][col]
   __shared__ double red[256];
-  rot_gemm_tile<T2, STAGE, GT>(p, it.k, b, tile, row0, col0, mode, cur, As, Bs, red);
+  rot_gemm_tile<T2, STAGE, GT>(p, it.k, b, mate, tile, row0, col0, mode, cur, As, Bs, red);
 }
 
 // K chunk of the second product of k_rot_fused (T held in LDS).
@@ -364,7 +380,7 @@ __host__ __device__ constexpr int rot_fused_elems() {
 // fragments from there and its B operand in chunks of W90_GK2 rows of
 // E_{k+b}, loaded one chunk ahead.  The epilogue is that of stage 2.
 template <class T2, int GT>
-__device__ __forceinline__ void rot_fused_tile(const Prob& p, int k, int b, int mode, int cur,
+__device__ __forceinline__ void rot_fused_tile(const Prob& p, int k, int b, int mate, int mode, int cur,
                                                typename Real<T2>::type* lds, double* red) {
   typedef FusedWaves<GT> WL;
   constexpr int FRR = WL::FRR, FRC = WL::FRC, FRM = FRR > FRC ? FRR : FRC, NT = WL::NT;
@@ -378,6 +394,7 @@ __device__ __forceinline__ void rot_fused_tile(const Prob& p, int k, int b, int 
   const cplx* Ekb = p.E + (size_t)p.nnl[kb] * nw2;
   const T2* src = rot_src<T2>(p, mode, cur) + kb * nw2;
   T2* out = mbuf<T2>(p, dst) + kb * nw2;
+  T2* outm = mbuf<T2>(p, dst) + (mate >= 0 ? (size_t)mate * nw2 : 0);
   double* lnd = p.ln[dst] + kb * nw;
   double* d2d = p.d2 + kb * nw;
   double* pod = p.part_od + kb * p.npan;
@@ -532,14 +549,20 @@ __device__ __forceinline__ void rot_fused_tile(const Prob& p, int k, int b, int 
           v.x = C[fi][fj].re(i);
           v.y = C[fi][fj].im(i);
           out[r + (size_t)c * nw] = v;
+          if (mate >= 0) outm[c + (size_t)r * nw] = c_conj(v);
           const cplx vw = c_wide(v);
           const double a2 = c_abs2(vw);
           all += a2;
           if (r != c) {
             od += a2;
           } else {
-            lnd[r] = atan2(vw.y, vw.x);
+            const double l = atan2(vw.y, vw.x);
+            lnd[r] = l;
             d2d[r] = a2;
+            if (mate >= 0) {
+              p.ln[dst][(size_t)mate * nw + r] = -l;
+              p.d2[(size_t)mate * nw + r] = a2;
+            }
           }
         }
       }
@@ -547,6 +570,10 @@ __device__ __forceinline__ void rot_fused_tile(const Prob& p, int k, int b, int 
   if (tid == 0) {
     pod[0] = od;
     pall[0] = all;
+    if (mate >= 0) {
+      p.part_od[(size_t)mate * p.npan] = od;
+      p.part_all[(size_t)mate * p.npan] = all;
+    }
   }
 }
 
@@ -564,17 +591,18 @@ __global__ void __launch_bounds__(FusedWaves<GT>::NT, FusedWaves<GT>::MINB) k_ro
   const int w = blockIdx.x;
   const int r = w >> 3;
   const int item = 8 * (r / nnmax) + (w & 7);
-  const int b = r % nnmax;
   if (item >= nitems) return;
   const Item it = items[item];
   const Prob& p = probs[it.prob];
   const State* st = p.st;
   const int cur = gate_cur(st, mode);
   if (cur < 0) return;
-  if (b >= p.nn) return;
+  int mate;
+  const int b = rot_slot<T2>(p, it.k, r % nnmax, &mate);
+  if (b < 0) return;
   __shared__ R lds[rot_fused_elems<R, GT>()];
   __shared__ double red[256];
-  rot_fused_tile<T2, GT>(p, it.k, b, mode, cur, lds, red);
+  rot_fused_tile<T2, GT>(p, it.k, b, mate, mode, cur, lds, red);
 }
 
 // ------------------------------------------------ rotation, direct operands
@@ -598,7 +626,7 @@ __global__ void __launch_bounds__(FusedWaves<GT>::NT, FusedWaves<GT>::MINB) k_ro
 // Epilogue as k_rot_fused: Im ln M_nn, |M_nn|^2, sum |M_mn|^2 and the
 // off-diagonal sum of the block.
 template <class T2>
-__device__ __forceinline__ void rot_direct_tile(const Prob& p, int k, int b, int mode, int cur,
+__device__ __forceinline__ void rot_direct_tile(const Prob& p, int k, int b, int mate, int mode, int cur,
                                                 typename Real<T2>::type* Ps, double* red) {
   constexpr int GT = 64, LD = GT + 1, FR = 2, PF = W90_RD_PF;
   typedef typename Real<T2>::type R;
@@ -610,6 +638,7 @@ __device__ __forceinline__ void rot_direct_tile(const Prob& p, int k, int b, int
   const cplx* ETkb = p.ET + (size_t)p.nnl[kb] * nw2;
   const T2* src = rot_src<T2>(p, mode, cur) + kb * nw2;
   T2* out = mbuf<T2>(p, dst) + kb * nw2;
+  T2* outm = mbuf<T2>(p, dst) + (mate >= 0 ? (size_t)mate * nw2 : 0);
   double* lnd = p.ln[dst] + kb * nw;
   double* d2d = p.d2 + kb * nw;
 
@@ -756,11 +785,17 @@ __device__ __forceinline__ void rot_direct_tile(const Prob& p, int k, int b, int
           const cplx vw = c_wide(v);
           const double a2 = c_abs2(vw);
           all += a2;
+          if (mate >= 0) outm[c + (size_t)r * nw] = c_conj(v);
           if (r != c) {
             od += a2;
           } else {
-            lnd[r] = atan2(vw.y, vw.x);
+            const double l = atan2(vw.y, vw.x);
+            lnd[r] = l;
             d2d[r] = a2;
+            if (mate >= 0) {
+              p.ln[dst][(size_t)mate * nw + r] = -l;
+              p.d2[(size_t)mate * nw + r] = a2;
+            }
           }
         }
       }
@@ -788,6 +823,10 @@ __device__ __forceinline__ void rot_direct_tile(const Prob& p, int k, int b, int
   if (tid == 0) {
     p.part_od[kb * p.npan] = od;
     p.part_all[kb * p.npan] = all;
+    if (mate >= 0) {
+      p.part_od[(size_t)mate * p.npan] = od;
+      p.part_all[(size_t)mate * p.npan] = all;
+    }
   }
 }
 
@@ -801,17 +840,18 @@ __global__ void __launch_bounds__(256, 2) k_rot_direct(const Prob* probs, const 
   const int w = blockIdx.x;
   const int r = w >> 3;
   const int item = 8 * (r / nnmax) + (w & 7);
-  const int b = r % nnmax;
   if (item >= nitems) return;
   const Item it = items[item];
   const Prob& p = probs[it.prob];
   const State* st = p.st;
   const int cur = gate_cur(st, mode);
   if (cur < 0) return;
-  if (b >= p.nn) return;
+  int mate;
+  const int b = rot_slot<T2>(p, it.k, r % nnmax, &mate);
+  if (b < 0) return;
   __shared__ R Ps[2 * 64 * 65];
   __shared__ double red[256];
-  rot_direct_tile<T2>(p, it.k, b, mode, cur, Ps, red);
+  rot_direct_tile<T2>(p, it.k, b, mate, mode, cur, Ps, red);
 }
 
 // Omega partial sums of the current M by GEMM tile (MODE_INIT of the MFMA
