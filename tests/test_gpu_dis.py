@@ -208,3 +208,19 @@ def test_disentangle_errors_follow_the_reference(ctx):
     for c, msg in bad:
         with pytest.raises(capi.W90Error, match=msg):
             ctx.disentangle(km, nb, c, e, np.asfortranarray(z["a"]), np.asfortranarray(z["m"]))
+
+
+# orders of the extraction's eigenproblem at the edges of its workgroup
+# sizes and of the memory that holds it (16, 32, 48, 64, 96), and the smallest
+# ones, where a round has one block or none (2 to 5 bands)
+@pytest.mark.parametrize("nb,nw", [(2, 1), (3, 2), (4, 2), (5, 3), (15, 8), (16, 9), (17, 9), (32, 14), (33, 14),
+                                   (48, 20), (49, 20), (63, 24), (64, 24), (65, 24), (96, 30), (97, 30)])
+def test_disentangle_orders_match_oracle(ctx, nb, nw):
+    from wannier90_amd import synth
+
+    print(f"[dis order] {nb} -> {nw}", flush=True)
+    p, ctl = synth.make_dis_problem(1700 + nb, kind="sc", num_bands=nb, num_wann=nw, mp=(2, 2, 2), decay=2.0)
+    ctl["num_iter"] = 12
+    g = ctx.disentangle(p.kmesh, nb, ctl, p.eig, p.amat_dis, p.m_orig)
+    o = po.dis_main(nb, nw, p.kmesh, ctl, p.eig, p.amat_dis, p.m_orig)
+    check_against(g, o, nw, well_posed=True)

@@ -31,11 +31,12 @@
 // Hermitian eigenproblems (of Z, Q P Q and the subspace Hamiltonian) are
 // solved in the workgroup by a two-sided cyclic Jacobi method with
 // round-robin (tournament) ordering: n/2 disjoint complex rotations per
-// round, applied to A (by 2 x 2 blocks) and to the basis in one parallel
-// pass; the polar factors (of A and of U_opt^+ A) by the one-sided Jacobi
-// SVD with the same ordering.  A workgroup's matrices live in LDS up to 64
-// bands (two 64 x 65 complex blocks) and in its own area of global memory
-// above that, up to 256 bands (the same code, instantiated for each).  The
+// round, applied to A (by 2 x 2 blocks) and to the basis between two
+// barriers; the polar factors (of A and of U_opt^+ A) by the one-sided Jacobi
+// SVD with the same ordering.  A workgroup's matrices live in LDS up to order
+// 64 (two 64 x 65 complex blocks); up to 96 the matrix does and the basis is
+// in the workgroup's own area of global memory, which holds both above that,
+// up to 256 bands (the same code, instantiated for each).  The
 // extraction only uses the spanned subspaces and the eigenvalue sums, which
 // do not depend on the eigenvector phases; the final U_opt and U do, so they
 // agree with the reference up to the phase of each Hamiltonian eigenvector
@@ -48,6 +49,7 @@
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/w90gpu.h"
@@ -79,14 +81,24 @@ __device__ __forceinline__ void zcfma(zd& a, zd b, zd c) {
   a.y = fma(b.x, c.y, fma(-b.y, c.x, a.y));
 }
 
-constexpr int kNT = 256;             // threads per workgroup
+// (x, y) J for J = [[c, s], [-conj(s), c]]: c x - conj(s) y and s x + c y
+__device__ __forceinline__ zd zrot_a(zd x, zd y, double c, zd s) {
+  return make_double2(fma(c, x.x, -fma(s.x, y.x, s.y * y.y)), fma(c, x.y, -fma(s.x, y.y, -s.y * y.x)));
+}
+__device__ __forceinline__ zd zrot_b(zd x, zd y, double c, zd s) {
+  return make_double2(fma(c, y.x, fma(s.x, x.x, -s.y * x.y)), fma(c, y.y, fma(s.x, x.y, s.y * x.x)));
+}
+
+constexpr int kNT = 256;             // threads per workgroup (the eigenproblem kernels choose theirs)
 constexpr int kMaxN = W90GPU_DIS_MAX_BANDS;
 // Largest matrix order of the LDS kernels: two kLdsN x (kLdsN + 1) complex
-// blocks fill 133 KB of a workgroup's 160 KB.  Above it the same kernels
-// run with their blocks in a per-workgroup area of global memory
-// (instantiated with N = kMaxN), launched in chunks of kGwsBlocks
-// workgroups that share those areas.
+// blocks fill 133 KB of a workgroup's 160 KB.  Above it, up to kHalfN, the
+// eigenproblem kernels keep the matrix in LDS (149 KB at 96) and the basis
+// in a per-workgroup area of global memory, which holds both above kHalfN
+// (and the blocks of the other kernels above kLdsN); such launches run in
+// chunks of kGwsBlocks workgroups that share those areas.
 constexpr int kLdsN = 64;
+constexpr int kHalfN = 96;
 constexpr size_t kLdsBytes = 2 * (size_t)kLdsN * (kLdsN + 1) * sizeof(double2);
 constexpr int kGwsBlocks = 1024;
 
@@ -119,10 +131,12 @@ enum : int {
 };
 
 struct DisProb {
-  int nb, nw, nk, nn, ld;  // ld: leading dimension of the workgroup matrices (nb + 1)
+  int nb, nw, nk, nn;
   int ntri;                // nb (nb + 1) / 2
-  int ldc;                 // k_dis_zmat: LDS leading dimension (odd, >= every ndim)
-  int nzmax, ldz;          // k_dis_update: largest ndim - nfroz, leading dimension (odd)
+  int ldc;                 // blocks of ndim rows: leading dimension (odd, >= every ndim)
+  int ldw;                 // num_wann x num_wann blocks of k_dis_find_u (odd)
+  int mz, mq, mh;          // eigenproblems of k_dis_update, k_dis_proj_froz and k_dis_ham:
+                           // largest order, rounded up to even (leading dimension one more)
   double wbtot;
   const int* nnl;      // [k * nn + b], 0-based
   const double* wb;    // [nn]
@@ -149,12 +163,25 @@ struct DisProb {
 };
 
 // The workgroup's matrix area (LDS, or its slice of gws above kLdsN) and
-// its block index (the launch's offset added above kLdsN).
+// its block index (the launch's offset added above kLdsN).  The
+// eigenproblem kernels with kLdsN < N <= kHalfN hold the matrix in LDS and
+// the basis in gws.
 extern __shared__ zd dis_lds[];
 template <int N>
 __device__ __forceinline__ zd* dis_ws(const DisProb& p) {
   if constexpr (N > kLdsN) return p.gws + (size_t)blockIdx.x * p.gws_stride;
   else return dis_lds;
+}
+template <int N>
+__device__ __forceinline__ zd* dis_mat(const DisProb& p) {
+  if constexpr (N > kHalfN) return p.gws + (size_t)blockIdx.x * p.gws_stride;
+  else return dis_lds;
+}
+template <int N>
+__device__ __forceinline__ zd* dis_basis(const DisProb& p, size_t matrix) {
+  if constexpr (N > kHalfN) return p.gws + (size_t)blockIdx.x * p.gws_stride + matrix;
+  else if constexpr (N > kLdsN) return p.gws + (size_t)blockIdx.x * p.gws_stride;
+  else return dis_lds + matrix;
 }
 template <int N>
 __device__ __forceinline__ int dis_blk(const DisProb& p) {
@@ -165,14 +192,15 @@ __device__ __forceinline__ int dis_blk(const DisProb& p) {
 // window row of the i-th non-frozen state
 __device__ __forceinline__ int nf_row(const Win& w, int i) { return i < w.fmin ? i : i + w.nfroz; }
 
-// Deterministic block reductions (wavefront butterflies, then the four
-// wavefront results in order); red holds kNT / 64 doubles.
+// Deterministic block reductions (wavefront butterflies, then the
+// wavefront results in order); red holds NT / 64 doubles.
+template <int NT = kNT>
 __device__ __forceinline__ double block_sum(double v, double* red) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
   double r = 0.0;
-  for (int i = 0; i < kNT / 64; ++i) r += red[i];
+  for (int i = 0; i < NT / 64; ++i) r += red[i];
   __syncthreads();
   return r;
 }
@@ -188,15 +216,30 @@ struct JRot {
   zd s;
 };
 
+// The rotation of a slot of the two-sided method in the slot's own order
+// (a, b) of its indices, and the diagonal entries it leaves at a and b.
+struct JSlot {
+  double c;
+  zd s;
+  double la, lb;
+};
+
 template <int N>
 struct JacobiLds {
   static constexpr int kN = N;
-  JRot rot[N / 2];
-  int count;
-  double red[kNT / 64];
+  JSlot slot[2][N / 2];  // the rotations of this round and of the next
+  double red[16];
   double lam[N];
   int perm[N];
   int rank[N];
+};
+
+template <int N>
+struct PolarLds {
+  JRot rot[N / 2];
+  int count;
+  double red[16];
+  double lam[N];
 };
 
 // Position (r, c), r <= c, of entry x = c (c + 1) / 2 + r of a packed upper
@@ -226,14 +269,6 @@ __device__ __forceinline__ void rr_pair(int s, int r, int m, int& p, int& q) {
   q = max(a, b);
 }
 
-// rows of E per lane and chunk in a rotation pass; n <= 64 takes one chunk
-// (at least 8 lanes a slot), n <= 256 up to eight
-constexpr int kRowsPerLane = 8;
-template <int N>
-constexpr int row_chunks() {
-  return (N + (kNT / (N / 2)) * kRowsPerLane - 1) / ((kNT / (N / 2)) * kRowsPerLane);
-}
-
 // The rotation of pair (p, q) is skipped when |a_pq| <= 1e-15 sqrt(|a_pp
 // a_qq|) (relative to the diagonal) or <= 1e-16 ||A||_F (without this floor
 // the rounding noise among the zero eigenvalues of a rank-deficient matrix
@@ -242,177 +277,292 @@ __device__ __forceinline__ bool jacobi_rotates(double b2, double app, double aqq
   return b2 > floor2 && b2 > 1e-30 * fabs(app * aqq);
 }
 
-// Whether some off-diagonal pair of A still rotates (all lanes, one pass).
-__device__ __forceinline__ bool jacobi_pending(const zd* A, int n, int ld, double floor2) {
+// Off-diagonal entries left in A (all lanes, one pass): with theta, whether
+// some pair that rotates has an angle above 1e-8 (see jacobi_run), else
+// whether any pair rotates.
+template <int NT>
+__device__ __forceinline__ bool jacobi_pending(const zd* A, int n, int ld, double floor2, bool theta) {
   int any = 0;
-  for (int e = threadIdx.x; e < n * n; e += kNT) {
+  for (int e = threadIdx.x; e < n * n; e += NT) {
     const int i = e % n, j = e / n;
-    if (i < j && jacobi_rotates(zabs2(A[i + j * ld]), A[i + i * ld].x, A[j + j * ld].x, floor2)) any = 1;
+    if (i >= j) continue;
+    const double b2 = zabs2(A[i + j * ld]), aii = A[i + i * ld].x, ajj = A[j + j * ld].x;
+    const double h = ajj - aii;
+    if (jacobi_rotates(b2, aii, ajj, floor2) && !(theta && b2 <= 1e-16 * h * h)) any = 1;
   }
   return __syncthreads_or(any) != 0;
 }
 
-// The rotation that zeroes a_pq: with D = diag(1, a_pq/|a_pq|) the 2 x 2
-// block D^+ A D is real, and its rotation by the smaller angle (tan 2t =
-// 2|a_pq| / (a_qq - a_pp)) gives J = D R D^+:
-//   t = sign(h) 2|a_pq| / (|h| + sqrt(h^2 + 4|a_pq|^2)), h = a_qq - a_pp,
-//   c = 1 / sqrt(1 + t^2), s = t c a_pq / |a_pq|.
-__device__ __forceinline__ JRot jacobi_rotation(int p, int q, const zd* A, int n, int ld, double floor2) {
-  JRot R;
-  R.p = p;
-  R.q = q;
+// 1 / sqrt(x) to rounding for normal x > 0: the hardware estimate and one
+// third-order step (the library's form adds the handling of zero, infinity
+// and subnormals, in the middle of the chain that bounds a Jacobi round).
+__device__ __forceinline__ double rsqrt_step(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// The rotation that zeroes a_pq (p < q): with D = diag(1, a_pq/|a_pq|) the
+// 2 x 2 block D^+ A D is real, and its rotation by the smaller angle t (tan
+// 2t = 2|a_pq| / (a_qq - a_pp)) gives J = D R D^+.  With h = a_qq - a_pp and
+// r = sqrt(h^2 + 4|a_pq|^2): c^2 = (1 + |h|/r) / 2, s = sign(h) a_pq / (r c),
+// and the diagonal moves by sign(h) |a_pq|^2 / (r c^2); two reciprocal square
+// roots, no division.  Stored in the order (a, b) of the slot's indices:
+// flip when a is the larger.
+__device__ __forceinline__ JSlot jacobi_rotation(zd aab, double laa, double lbb, bool flip, double floor2) {
+  JSlot R;
   R.c = 1.0;
   R.s = zmk(0.0, 0.0);
-  if (q < n) {
-    const zd apq = A[p + q * ld];
-    const double app = A[p + p * ld].x, aqq = A[q + q * ld].x;
-    const double b2 = zabs2(apq);
-    if (jacobi_rotates(b2, app, aqq, floor2)) {
-      const double rb = rsqrt(b2);
-      const double h = aqq - app;
-      const double den = fabs(h) + sqrt(fma(h, h, 4.0 * b2));
-      const double tt = copysign(2.0 * b2 * rb, h) / den;
-      const double c = rsqrt(fma(tt, tt, 1.0));
-      const double sr = tt * c * rb;
-      R.c = c;
-      R.s = zmk(sr * apq.x, sr * apq.y);
-    }
+  R.la = laa;
+  R.lb = lbb;
+  const double b2 = zabs2(aab);
+  if (jacobi_rotates(b2, laa, lbb, floor2)) {
+    const double h = flip ? laa - lbb : lbb - laa;  // a_qq - a_pp
+    const double u = rsqrt_step(fma(h, h, 4.0 * b2));
+    const double c2 = fma(0.5 * fabs(h), u, 0.5);
+    const double rc = rsqrt_step(c2);
+    // sign(h) of the order (p, q); s of (b, a) is minus the conjugate
+    const double sg = copysign(1.0, h), so = flip ? -sg : sg;
+    R.c = c2 * rc;
+    R.s = zscale(aab, so * u * rc);
+    const double d = so * b2 * u * rc * rc;
+    R.la = laa - d;
+    R.lb = lbb + d;
   }
   return R;
 }
 
-// Eigen-decomposition of the Hermitian n x n matrix A (LDS, column-major,
-// leading dimension ld, stored whole) by the two-sided cyclic Jacobi method
-// with round-robin (tournament) ordering: each round rotates n/2 disjoint
-// pairs at once; the rotations go into J.rot, and one parallel pass then
-// applies A <- J^+ A J by 2 x 2 blocks (one lane per block of the upper
-// block triangle, which writes the block and its mirror) and E <- E J to
-// the rows of E (LDS, leading dimension ld).  On return A is diagonal to the
-// tolerance of jacobi_rotates and the columns of E (as it came in) times the
+// Index of slot s's first (a) and second (b) member in round r of the
+// round-robin schedule of rr_pair, and the same one round later.
+__device__ __forceinline__ int rr_a(int s, int r, int m) {
+  if (s == 0) return 0;
+  int a = s - 1 + r;
+  if (a >= m - 1) a -= m - 1;
+  return a + 1;
+}
+__device__ __forceinline__ int rr_b(int s, int r, int m) {
+  int b = m - 2 - s + r;
+  if (b >= m - 1) b -= m - 1;
+  return b + 1;
+}
+// (inc 0 for the index that stays, 1 for the others)
+__device__ __forceinline__ int rr_next(int x, int inc, int m) { return x == m - 1 ? 1 : x + inc; }
+
+// Slots (r1, r2) of work item x of a round: x < half are the blocks that
+// hold the pivot of slot x of the next round (its pair is (a of slot x + 1,
+// b of slot x - 1), at the ends (a of 0, a of 1) and (b of half - 1, b of
+// half - 2)); then the other off-diagonal blocks; then the diagonal ones.
+__device__ __forceinline__ void jacobi_item(int x, int half, int& r1, int& r2) {
+  const int noff = half * (half - 1) / 2;
+  if (x >= noff) {
+    r1 = r2 = x - noff;
+  } else if (x < half) {
+    r1 = x == 0 ? 0 : x == half - 1 ? half - 2 : x - 1;
+    r2 = x == 0 ? 1 : x == half - 1 ? half - 1 : x + 1;
+  } else if (x < 2 * half - 3) {
+    r1 = x - half + 1;
+    r2 = r1 + 1;
+  } else {
+    tri_decode(x - (2 * half - 3), r1, r2);
+    r2 += 3;
+  }
+}
+
+// Eigen-decomposition of the Hermitian n x n matrix A (column-major, leading
+// dimension ld >= n + (n odd), stored whole) by the two-sided cyclic Jacobi
+// method with round-robin (tournament) ordering: each round rotates n/2
+// disjoint pairs at once, A <- J^+ A J by 2 x 2 blocks (one lane per block of
+// the upper block triangle, which writes the block and its mirror) and
+// E <- E J by rows.  On return the columns of E (as it came in) times the
 // rotations are the eigenvectors: E = I gives those of A, E = V for A = V^+
-// Z V those of Z.  The sweeps end when no pair rotates (checked before each
-// sweep in one parallel pass).  Returns the number of sweeps, or -1 if
-// kMaxSweeps were not enough.  A warm start (a nearly diagonal A) leaves
-// off-diagonal entries just below the skip bounds, so they are kept tight:
-// the selected subspace moves by their size over the eigenvalue gap at the
-// selection.
-template <class JL>
-__device__ __forceinline__ int jacobi_run(zd* A, zd* E, int n, int ld, JL& J) {
-  constexpr int CH = row_chunks<JL::kN>();
+// Z V those of Z.  Odd n is padded by a zero row and column (A and E hold
+// n + 1 columns).
+//
+// One barrier per round.  The wavefronts are split: the first AW lanes take
+// the blocks of A, the others the rows of E.  The pair of slot s in round
+// r + 1 lies in one block of round r, so the lane of that block forms the
+// next rotation from its new entry and the two diagonal entries, which the
+// rotations carry along; nothing waits for a separate pass over the pivots.
+// What bounds a round: the chain of the pivot blocks (LDS reads, the block's
+// products, two reciprocal square roots, LDS write, barrier) where a CU holds
+// one workgroup, 0.85 us at order 11; the LDS traffic of the blocks and rows
+// with two per CU, 1.1 us at order 39 (1.66 us when the rotations had a pass
+// of their own between two barriers and every wavefront did both parts).
+// k_dis_update per launch, before -> now: 48 bands to 24, 11 frozen, 512 k
+// 385 -> 250 us; 12 to 8, 64 k 68 -> 43 us; 80 to 40, 64 k, whose matrices
+// were both in global memory, 4.34 -> 0.87 ms.
+//
+// theta false: sweeps until no pair rotates.  theta true: sweeps until every
+// angle left is at most 1e-8, where the rest of the method is the first-order
+// step E (1 + T), T_ij = a_ij / (a_jj - a_ii), to rounding (products of two
+// angles are below 1e-16); the caller applies it with its own product.  The
+// sweeps are checked in one parallel pass before each.  Returns the number
+// of sweeps, or -1 if kMaxSweeps were not enough.  A warm start (a nearly
+// diagonal A) leaves off-diagonal entries just below the skip bounds, so they
+// are kept tight: the selected subspace moves by their size over the
+// eigenvalue gap at the selection.
+template <int NT, class JL>
+__device__ __forceinline__ int jacobi_run(zd* A, zd* E, int n, int ld, int lde, JL& J, bool theta) {
   const int t = threadIdx.x;
   double fro = 0.0;
-  for (int e = t; e < n * n; e += kNT) fro += zabs2(A[(e % n) + (e / n) * ld]);
-  const double floor2 = block_sum(fro, J.red) * 1e-32;
+  for (int e = t; e < n * n; e += NT) fro += zabs2(A[(e % n) + (e / n) * ld]);
   const int m = n + (n & 1), half = m / 2;
-  const int nblk = half * (half + 1) / 2;
-  // this lane's first block of the upper block triangle, and its share of
-  // the rows of E: slot es (g lanes per slot), rows eg, eg + g, ...
-  int bs1 = 0, bs2 = 0;
-  if (t < nblk) tri_decode(t, bs1, bs2);
-  const int g = kNT / half, es = t / g, eg = t % g;
-  int sweeps = 0;
-  while (jacobi_pending(A, n, ld, floor2)) {
+  if (m > n)
+    for (int i = t; i < m; i += NT) {
+      A[i + n * ld] = A[n + i * ld] = zmk(0.0, 0.0);
+      if (i < n) E[i + n * lde] = zmk(0.0, 0.0);
+    }
+  const double floor2 = block_sum<NT>(fro, J.red) * 1e-32;
+  const int nitem = half * (half + 1) / 2, noff = nitem - half;
+  // lanes: [0, SW) the blocks with the next round's pivots, one each, in
+  // wavefronts of their own (theirs is the chain that bounds a round);
+  // [SW, AW) the other blocks; [AW, NT) the rows of E
+  const int nsp = min(half, noff), SW = (half + 63) & ~63;
+  const int AW = min(SW + ((nitem - nsp + 63) & ~63), JL::kN > kHalfN ? NT / 2 : NT * 3 / 4 / 64 * 64);
+  const bool erole = t >= AW;
+  int b1 = 0, b2 = 0;
+  const int x0 = t < SW ? t : nsp + t - SW;
+  const bool mine = t < SW ? t < nsp : !erole && x0 < nitem;
+  if (mine) jacobi_item(x0, half, b1, b2);
+  // rows of E: slot es (g lanes each), rows eg, eg + g, ...
+  const int u = t - AW, g = max(1, (NT - AW) / half), nes = (NT - AW) / g;
+  const int es0 = erole ? u / g : 0, eg = erole ? u % g : 0;
+  // the rotations of the first round
+  for (int sl = t; sl < half; sl += NT) {
+    const int a = rr_a(sl, 0, m), b = rr_b(sl, 0, m);
+    J.slot[0][sl] = jacobi_rotation(A[a + b * ld], A[a + a * ld].x, A[b + b * ld].x, a > b, floor2);
+  }
+  // A <- J^+ A J on the block of slots s1 < s2 (members i1, j1 and i2, j2),
+  // which this lane owns in this round with its mirror
+  auto block = [&](const JSlot* cur, int s1, int s2, int i1, int j1, int i2, int j2, zd& naa, zd& nab, zd& nba, zd& nbb) {
+    const int ci1 = __mul24(i1, ld), cj1 = __mul24(j1, ld), ci2 = __mul24(i2, ld), cj2 = __mul24(j2, ld);
+    naa = A[i1 + ci2];
+    nab = A[i1 + cj2];
+    nba = A[j1 + ci2];
+    nbb = A[j1 + cj2];
+    const double k1 = cur[s1].c, k2 = cur[s2].c;
+    const zd q1 = cur[s1].s, q2 = cur[s2].s;
+    if (q1.x != 0.0 || q1.y != 0.0 || q2.x != 0.0 || q2.y != 0.0) {
+      // Y = X J2, then J1^+ Y
+      const zd yaa = zrot_a(naa, nab, k2, q2), yab = zrot_b(naa, nab, k2, q2);
+      const zd yba = zrot_a(nba, nbb, k2, q2), ybb = zrot_b(nba, nbb, k2, q2);
+      const zd p1 = zconj(q1);
+      naa = zrot_a(yaa, yba, k1, p1);
+      nba = zrot_b(yaa, yba, k1, p1);
+      nab = zrot_a(yab, ybb, k1, p1);
+      nbb = zrot_b(yab, ybb, k1, p1);
+      A[i1 + ci2] = naa;
+      A[i2 + ci1] = zconj(naa);
+      A[i1 + cj2] = nab;
+      A[j2 + ci1] = zconj(nab);
+      A[j1 + ci2] = nba;
+      A[i2 + cj1] = zconj(nba);
+      A[j1 + cj2] = nbb;
+      A[j2 + cj1] = zconj(nbb);
+    }
+  };
+  const int inc = (erole ? es0 : b1) == 0 ? 0 : 1;
+  const int nfull = (n - 1) / g;  // rows eg + j g with j < nfull are all below n
+  int sweeps = 0, par = 0;
+  while (jacobi_pending<NT>(A, n, ld, floor2, theta)) {
     if (sweeps == kMaxSweeps) return -1;
     ++sweeps;
+    // members of this lane's block, or (E) of its first slot
+    int a1 = rr_a(erole ? es0 : b1, 0, m), c1 = rr_b(erole ? es0 : b1, 0, m);
+    int a2 = rr_a(b2, 0, m), c2 = rr_b(b2, 0, m);
     for (int r = 0; r < m - 1; ++r) {
-      if (t < half) {
-        int p, q;
-        rr_pair(t, r, m, p, q);
-        J.rot[t] = jacobi_rotation(p, q, A, n, ld, floor2);
-      }
-      __syncthreads();
-      for (int x = t; x < nblk; x += kNT) {
-        int r1 = bs1, r2 = bs2;
-        if (x != t) tri_decode(x, r1, r2);
-        int p1, q1, p2, q2;
-        rr_pair(r1, r, m, p1, q1);
-        rr_pair(r2, r, m, p2, q2);
-        const bool v1 = q1 < n, v2 = q2 < n;
-        // the block's entries requested with the rotations
-        const zd z0 = zmk(0.0, 0.0);
-        const zd xpp = A[p1 + p2 * ld];
-        const zd xpq = v2 ? A[p1 + q2 * ld] : z0;
-        const zd xqp = v1 ? A[q1 + p2 * ld] : z0;
-        const zd xqq = (v1 && v2) ? A[q1 + q2 * ld] : z0;
-        const double c1 = J.rot[r1].c, c2 = J.rot[r2].c;
-        const zd s1 = J.rot[r1].s, s2 = J.rot[r2].s;
-        if (s1.x == 0.0 && s1.y == 0.0 && s2.x == 0.0 && s2.y == 0.0) continue;
-        // Y = X J2, then J1^+ Y
-        const zd s2c = zconj(s2), s1c = zconj(s1);
-        const zd ypp = zsub(zscale(xpp, c2), zmul(s2c, xpq)), ypq = zadd(zmul(s2, xpp), zscale(xpq, c2));
-        const zd yqp = zsub(zscale(xqp, c2), zmul(s2c, xqq)), yqq = zadd(zmul(s2, xqp), zscale(xqq, c2));
-        const zd npp = zsub(zscale(ypp, c1), zmul(s1, yqp)), nqp = zadd(zmul(s1c, ypp), zscale(yqp, c1));
-        const zd npq = zsub(zscale(ypq, c1), zmul(s1, yqq)), nqq = zadd(zmul(s1c, ypq), zscale(yqq, c1));
-        if (r1 != r2) {
-          A[p1 + p2 * ld] = npp;
-          A[p2 + p1 * ld] = zconj(npp);
-          if (v2) {
-            A[p1 + q2 * ld] = npq;
-            A[q2 + p1 * ld] = zconj(npq);
-          }
-          if (v1) {
-            A[q1 + p2 * ld] = nqp;
-            A[p2 + q1 * ld] = zconj(nqp);
-          }
-          if (v1 && v2) {
-            A[q1 + q2 * ld] = nqq;
-            A[q2 + q1 * ld] = zconj(nqq);
-          }
-        } else {
-          A[p1 + p1 * ld] = zmk(npp.x, 0.0);
-          if (v1) {
-            A[q1 + q1 * ld] = zmk(nqq.x, 0.0);
-            A[p1 + q1 * ld] = npq;
-            A[q1 + p1 * ld] = zconj(npq);
-          }
+      const JSlot* cur = J.slot[par];
+      JSlot* nxt = J.slot[par ^ 1];
+      if (t < SW) {
+        if (mine) {
+          zd naa, nab, nba, nbb;
+          block(cur, b1, b2, a1, c1, a2, c2, naa, nab, nba, nbb);
+          // slot t of the next round: its pair and its pivot in the order (a, b)
+          const bool lo = t == 0, hi = t == half - 1;
+          const zd v = lo ? naa : zconj(hi ? nbb : nba);
+          const double la = lo ? cur[0].la : hi ? cur[b2].lb : cur[b2].la;
+          const double lb = lo ? cur[1].la : cur[b1].lb;
+          const int na = lo ? a1 : hi ? c2 : a2, nb = lo ? a2 : c1;
+          nxt[t] = jacobi_rotation(v, la, lb, na > nb, floor2);
+          // two slots: the one off-diagonal block holds both pivots
+          if (half == 2) nxt[1] = jacobi_rotation(zconj(nbb), cur[1].lb, cur[0].lb, c2 > c1, floor2);
         }
-      }
-      if (es < half) {
-        int p, q;
-        rr_pair(es, r, m, p, q);
-        if (q < n) {
-#pragma unroll 1
-          for (int ch = 0; ch < CH; ++ch) {
-            const int row0 = eg + ch * kRowsPerLane * g;
-            zd ep[kRowsPerLane], eq[kRowsPerLane];
-#pragma unroll
-            for (int j = 0; j < kRowsPerLane; ++j) {
-              const int row = row0 + j * g;
-              if (row < n) {
-                ep[j] = E[row + p * ld];
-                eq[j] = E[row + q * ld];
-              }
-            }
-            const double c = J.rot[es].c;
-            const zd sv = J.rot[es].s, sc = zconj(sv);
-            if (sv.x != 0.0 || sv.y != 0.0) {
-#pragma unroll
-              for (int j = 0; j < kRowsPerLane; ++j) {
-                const int row = row0 + j * g;
-                if (row < n) {
-                  E[row + p * ld] = zsub(zscale(ep[j], c), zmul(sc, eq[j]));
-                  E[row + q * ld] = zadd(zmul(sv, ep[j]), zscale(eq[j], c));
-                }
-              }
+      } else if (!erole) {
+        for (int x = x0; x < nitem; x += AW - SW) {
+          int s1 = b1, s2 = b2, i1 = a1, j1 = c1, i2 = a2, j2 = c2;
+          if (x != x0) {
+            jacobi_item(x, half, s1, s2);
+            i1 = rr_a(s1, r, m);
+            j1 = rr_b(s1, r, m);
+            i2 = rr_a(s2, r, m);
+            j2 = rr_b(s2, r, m);
+          }
+          if (x < noff) {
+            zd naa, nab, nba, nbb;
+            block(cur, s1, s2, i1, j1, i2, j2, naa, nab, nba, nbb);
+          } else {  // diagonal block: the rotation carries its entries
+            const JSlot R = cur[s1];
+            if (R.s.x != 0.0 || R.s.y != 0.0) {
+              A[i1 + i1 * ld] = zmk(R.la, 0.0);
+              A[j1 + j1 * ld] = zmk(R.lb, 0.0);
+              A[i1 + j1 * ld] = zmk(0.0, 0.0);
+              A[j1 + i1 * ld] = zmk(0.0, 0.0);
             }
           }
         }
+      } else if (u < nes * g) {
+        for (int es = es0; es < half; es += nes) {
+          int p = a1, q = c1;
+          if (es != es0) {
+            p = rr_a(es, r, m);
+            q = rr_b(es, r, m);
+          }
+          const double c = cur[es].c;
+          const zd sv = cur[es].s;
+          if (sv.x == 0.0 && sv.y == 0.0) continue;
+          zd* Ep = E + __mul24(p, lde);
+          zd* Eq = E + __mul24(q, lde);
+          auto rows = [&](auto two, int row) {
+            constexpr int R = decltype(two)::value ? 2 : 1;
+            zd ep[R], eq[R];
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+              ep[j] = Ep[row + j * g];
+              eq[j] = Eq[row + j * g];
+            }
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+              Ep[row + j * g] = zrot_a(ep[j], eq[j], c, sv);
+              Eq[row + j * g] = zrot_b(ep[j], eq[j], c, sv);
+            }
+          };
+          int row = eg, j = 0;
+          for (; j + 2 <= nfull; j += 2, row += 2 * g) rows(std::true_type{}, row);
+          for (; j < nfull; ++j, row += g) rows(std::false_type{}, row);
+          if (row < n) rows(std::false_type{}, row);
+        }
       }
+      a1 = rr_next(a1, inc, m);
+      c1 = rr_next(c1, 1, m);
+      a2 = rr_next(a2, 1, m);  // (a diagonal block uses a1, c1 only)
+      c2 = rr_next(c2, 1, m);
+      par ^= 1;
       __syncthreads();
     }
   }
   return sweeps;
 }
 
-// jacobi_run from E = I into V (the eigenvectors of A itself).
-template <class JL>
-__device__ __forceinline__ int jacobi_eigh(zd* A, zd* V, int n, int ld, JL& J) {
-  for (int e = threadIdx.x; e < n * n; e += kNT) {
+// jacobi_run from E = I into V (the eigenvectors of A itself), A diagonal on
+// return to the tolerance of jacobi_rotates.
+template <int NT, class JL>
+__device__ __forceinline__ int jacobi_eigh(zd* A, zd* V, int n, int ld, int ldv, JL& J) {
+  for (int e = threadIdx.x; e < n * n; e += NT) {
     const int r = e % n, c = e / n;
-    V[r + c * ld] = zmk(r == c ? 1.0 : 0.0, 0.0);
+    V[r + c * ldv] = zmk(r == c ? 1.0 : 0.0, 0.0);
   }
   __syncthreads();
-  return jacobi_run(A, V, n, ld, J);
+  return jacobi_run<NT>(A, V, n, ld, ldv, J, false);
 }
 
 // ------------------------------------------------------------ products
@@ -421,10 +571,10 @@ __device__ __forceinline__ int jacobi_eigh(zd* A, zd* V, int n, int ld, JL& J) {
 // register tiles, one tile per lane and pass: op(A)(i, l) = A[i + l * lda],
 // or conj(A[l + i * lda]) when ADJ; B(l, j) = B[l + j * ldb].  Rows and
 // columns past the edge are read clamped and not stored.
-template <int RT, int CT, bool ADJ, int UNR = 2, class Out>
+template <int NT, int RT, int CT, bool ADJ, int UNR = 2, class Out>
 __device__ void zgemm_tiles(int M, int N, int K, const zd* A, int lda, const zd* B, int ldb, Out out) {
   const int tr = (M + RT - 1) / RT, tc = (N + CT - 1) / CT;
-  for (int x = threadIdx.x; x < tr * tc; x += kNT) {
+  for (int x = threadIdx.x; x < tr * tc; x += NT) {
     const int i0 = (x % tr) * RT, j0 = (x / tr) * CT;
     int ii[RT], jj[CT];
 #pragma unroll
@@ -465,28 +615,27 @@ __device__ void zgemm_tiles(int M, int N, int K, const zd* A, int lda, const zd*
 // when A is in global memory, to request its loads ahead).
 template <bool ADJ, int UNR, class Out>
 __device__ void zgemm_small(int M, int N, int K, const zd* A, int lda, const zd* B, int ldb, Out out) {
-  if (((M + 1) / 2) * ((N + 1) / 2) <= kNT) zgemm_tiles<2, 2, ADJ, UNR>(M, N, K, A, lda, B, ldb, out);
-  else zgemm_tiles<2, 3, ADJ, UNR>(M, N, K, A, lda, B, ldb, out);
+  if (((M + 1) / 2) * ((N + 1) / 2) <= kNT) zgemm_tiles<kNT, 2, 2, ADJ, UNR>(M, N, K, A, lda, B, ldb, out);
+  else zgemm_tiles<kNT, 2, 3, ADJ, UNR>(M, N, K, A, lda, B, ldb, out);
 }
 
-// zgemm_tiles with the smallest tile that needs at most one pass (M, N <=
-// 64 fit 4 x 4 tiles; larger results take several passes of them).
-template <bool ADJ, class Out>
+// zgemm_tiles with the smallest tile that needs at most one pass, or 3 x 3
+// over several: the eigenproblem kernels have a lane for every 2 x 3 tile up
+// to kLdsN, and larger tiles would take the registers of a second workgroup.
+template <int NT, bool ADJ, class Out>
 __device__ void zgemm(int M, int N, int K, const zd* A, int lda, const zd* B, int ldb, Out out) {
-  auto fits = [&](int r, int c) { return ((M + r - 1) / r) * ((N + c - 1) / c) <= kNT; };
-  if (fits(2, 2)) zgemm_tiles<2, 2, ADJ>(M, N, K, A, lda, B, ldb, out);
-  else if (fits(2, 3)) zgemm_tiles<2, 3, ADJ>(M, N, K, A, lda, B, ldb, out);
-  else if (fits(3, 3)) zgemm_tiles<3, 3, ADJ>(M, N, K, A, lda, B, ldb, out);
-  else if (fits(3, 4)) zgemm_tiles<3, 4, ADJ>(M, N, K, A, lda, B, ldb, out);
-  else zgemm_tiles<4, 4, ADJ>(M, N, K, A, lda, B, ldb, out);
+  auto fits = [&](int r, int c) { return ((M + r - 1) / r) * ((N + c - 1) / c) <= NT; };
+  if (fits(2, 2)) zgemm_tiles<NT, 2, 2, ADJ>(M, N, K, A, lda, B, ldb, out);
+  else if (fits(2, 3)) zgemm_tiles<NT, 2, 3, ADJ>(M, N, K, A, lda, B, ldb, out);
+  else zgemm_tiles<NT, 3, 3, ADJ>(M, N, K, A, lda, B, ldb, out);
 }
 
 // The upper triangle (i <= j) of a Hermitian N x N product A^+ B by T x T
 // tiles of the upper block triangle: out(i, j, C(i, j)) for i <= j only.
-template <int T, class Out>
+template <int NT, int T, class Out>
 __device__ void zgemm_herm_tiles(int N, int K, const zd* A, int lda, const zd* B, int ldb, Out out) {
   const int nt = (N + T - 1) / T;
-  for (int x = threadIdx.x; x < nt * (nt + 1) / 2; x += kNT) {
+  for (int x = threadIdx.x; x < nt * (nt + 1) / 2; x += NT) {
     int ib, jb;
     tri_decode(x, ib, jb);
     const int i0 = ib * T, j0 = jb * T;
@@ -522,15 +671,14 @@ __device__ void zgemm_herm_tiles(int N, int K, const zd* A, int lda, const zd* B
   }
 }
 
-template <class Out>
+template <int NT, class Out>
 __device__ void zgemm_herm(int N, int K, const zd* A, int lda, const zd* B, int ldb, Out out) {
   auto fits = [&](int tl) {
     const int nt = (N + tl - 1) / tl;
-    return nt * (nt + 1) / 2 <= kNT;
+    return nt * (nt + 1) / 2 <= NT;
   };
-  if (fits(2)) zgemm_herm_tiles<2>(N, K, A, lda, B, ldb, out);
-  else if (fits(3)) zgemm_herm_tiles<3>(N, K, A, lda, B, ldb, out);
-  else zgemm_herm_tiles<4>(N, K, A, lda, B, ldb, out);
+  if (fits(2)) zgemm_herm_tiles<NT, 2>(N, K, A, lda, B, ldb, out);
+  else zgemm_herm_tiles<NT, 3>(N, K, A, lda, B, ldb, out);
 }
 
 // Eigenvalues (the diagonal of A after jacobi_run) into J.lam, their
@@ -561,12 +709,12 @@ __device__ __forceinline__ void eig_order(const zd* A, int n, int ld, JL& J) {
 // X, where the polar factor is not unique, as with the SVD) are completed
 // by Gram-Schmidt from unit vectors.  U goes to global memory (leading
 // dimension ldu).  LDS: G (rows x nw, leading dimension ld), V.
-template <class JL>
+template <int NT, class JL>
 __device__ __forceinline__ void polar_factor(const zd* X, int ldx, int rows, int nw, zd* U, int ldu, zd* G, zd* V,
                                              int ld, JL& J, int* flags) {
   const int t = threadIdx.x;
   double fro = 0.0;
-  for (int e = t; e < rows * nw; e += kNT) {
+  for (int e = t; e < rows * nw; e += NT) {
     const int r = e % rows, c = e / rows;
     const zd x = X[r + (size_t)c * ldx];
     G[r + c * ld] = x;
@@ -574,8 +722,8 @@ __device__ __forceinline__ void polar_factor(const zd* X, int ldx, int rows, int
   }
   // columns below 1e-15 ||X||_F are numerically zero: rotating their
   // rounding noise against the others would never end
-  const double zero2 = 1e-30 * block_sum(fro, J.red);
-  for (int e = t; e < nw * nw; e += kNT) {
+  const double zero2 = 1e-30 * block_sum<NT>(fro, J.red);
+  for (int e = t; e < nw * nw; e += NT) {
     const int r = e % nw, c = e / nw;
     V[r + c * ld] = zmk(r == c ? 1.0 : 0.0, 0.0);
   }
@@ -586,8 +734,8 @@ __device__ __forceinline__ void polar_factor(const zd* X, int ldx, int rows, int
     if (t == 0) J.count = 0;
     __syncthreads();
     for (int r = 0; r < m - 1; ++r) {
-      // Gram entries of each pair, 8 lanes per pair (kNT / 8 pairs a pass)
-      for (int pb = 0; pb < half; pb += kNT / 8) {
+      // Gram entries of each pair, 8 lanes per pair (NT / 8 pairs a pass)
+      for (int pb = 0; pb < half; pb += NT / 8) {
         const int pi = pb + (t >> 3), lane = t & 7;
         double al = 0.0, be = 0.0;
         zd ga = zmk(0.0, 0.0);
@@ -632,7 +780,7 @@ __device__ __forceinline__ void polar_factor(const zd* X, int ldx, int rows, int
         }
       }
       __syncthreads();
-      for (int e = t; e < half * (rows + nw); e += kNT) {
+      for (int e = t; e < half * (rows + nw); e += NT) {
         const int i = e / (rows + nw), row = e % (rows + nw);
         const JRot R = J.rot[i];
         if (R.s.x == 0.0 && R.s.y == 0.0) continue;
@@ -658,7 +806,7 @@ __device__ __forceinline__ void polar_factor(const zd* X, int ldx, int rows, int
   double smax = 0.0;
   for (int i = 0; i < nw; ++i) smax = fmax(smax, J.lam[i]);
   auto good = [&](int i) { return J.lam[i] > 1e-12 * smax && J.lam[i] > 0.0; };
-  for (int e = t; e < rows * nw; e += kNT) {
+  for (int e = t; e < rows * nw; e += NT) {
     const int r = e % rows, i = e / rows;
     G[r + i * ld] = good(i) ? zscale(G[r + i * ld], 1.0 / J.lam[i]) : zmk(0.0, 0.0);
   }
@@ -688,7 +836,7 @@ __device__ __forceinline__ void polar_factor(const zd* X, int ldx, int rows, int
   }
   __syncthreads();
   // U = Z V^+
-  for (int e = t; e < rows * nw; e += kNT) {
+  for (int e = t; e < rows * nw; e += NT) {
     const int r = e % rows, j = e / rows;
     zd u = zmk(0.0, 0.0);
     for (int i = 0; i < nw; ++i) zfma(u, G[r + i * ld], zconj(V[j + i * ld]));
@@ -701,21 +849,22 @@ __device__ __forceinline__ void polar_factor(const zd* X, int ldx, int rows, int
 //
 // Each kernel with matrices per workgroup is a template on the largest
 // matrix order N: N = kLdsN keeps them in LDS, N = kMaxN in the
-// workgroup's area of global memory (dis_ws, dis_blk).
+// workgroup's area of global memory (dis_ws, dis_blk); the eigenproblem
+// kernels also on the workgroup size, with a form in between (kHalfN).
 
 // dis_project: U_opt(k) = polar factor of A(window rows, :); its unitarity
 // checked to 1e-5; rows below the window zero.
 template <int N>
 __global__ void __launch_bounds__(kNT) k_dis_project(DisProb p) {
-  __shared__ JacobiLds<N> J;
+  __shared__ PolarLds<N> J;
   const int k = dis_blk<N>(p);
   const Win w = p.win[k];
-  const int nb = p.nb, nw = p.nw, ld = p.ld;
+  const int nb = p.nb, nw = p.nw, ld = p.ldc;
   zd* S = dis_ws<N>(p);
-  zd* V = S + nb * ld;
+  zd* V = S + nw * ld;
   zd* U = p.Uopt + (size_t)k * nb * nw;
   const zd* X = p.A + (size_t)k * nb * nw + w.first;
-  polar_factor(X, nb, w.ndim, nw, U, nb, S, V, ld, J, p.flags);
+  polar_factor<kNT>(X, nb, w.ndim, nw, U, nb, S, V, ld, J, p.flags);
   for (int e = threadIdx.x; e < nb * nw; e += kNT)
     if (e % nb >= w.ndim) U[e] = zmk(0.0, 0.0);
   // unitarity of U_opt (dis_project, :1384-1410)
@@ -736,21 +885,21 @@ __global__ void __launch_bounds__(kNT) k_dis_project(DisProb p) {
 // order of eigenvalue; when some of those eigenvalues are below 1e-8 the
 // reference's ortho-fix picks, from the top down, eigenvectors orthogonal
 // to the frozen columns.
-template <int N>
-__global__ void __launch_bounds__(kNT) k_dis_proj_froz(DisProb p) {
+template <int N, int NT>
+__global__ void __launch_bounds__(NT) k_dis_proj_froz(DisProb p) {
   __shared__ JacobiLds<N> J;
   __shared__ int vmap[N];
   __shared__ int fix_ok;
   const int k = dis_blk<N>(p);
   const Win w = p.win[k];
-  const int nb = p.nb, nw = p.nw, ld = p.ld, nd = w.ndim, t = threadIdx.x;
-  zd* Aq = dis_ws<N>(p);
-  zd* V = Aq + nb * ld;
+  const int nb = p.nb, nw = p.nw, ld = p.mq + 1, nd = w.ndim, t = threadIdx.x;
+  zd* Aq = dis_mat<N>(p);
+  zd* V = dis_basis<N>(p, (size_t)ld * p.mq);
   zd* U = p.Uopt + (size_t)k * nb * nw;
   const int r = nw - w.nfroz;
   auto frozen = [&](int i) { return i >= w.fmin && i < w.fmin + w.nfroz; };
   if (r > 0) {
-    for (int e = t; e < nd * nd; e += kNT) {
+    for (int e = t; e < nd * nd; e += NT) {
       const int i = e % nd, j = e / nd;
       if (i > j) continue;
       zd s = zmk(0.0, 0.0);
@@ -761,7 +910,7 @@ __global__ void __launch_bounds__(kNT) k_dis_proj_froz(DisProb p) {
       Aq[j + i * ld] = zconj(s);
     }
     __syncthreads();
-    if (jacobi_eigh(Aq, V, nd, ld, J) < 0 && t == 0) atomicOr(p.flags, F_JACOBI);
+    if (jacobi_eigh<NT>(Aq, V, nd, ld, ld, J) < 0 && t == 0) atomicOr(p.flags, F_JACOBI);
     eig_order(Aq, nd, ld, J);
     if (t == 0) {
       fix_ok = 1;
@@ -813,14 +962,14 @@ __global__ void __launch_bounds__(kNT) k_dis_proj_froz(DisProb p) {
     }
     __syncthreads();
     if (fix_ok) {
-      for (int e = t; e < nd * r; e += kNT) {
+      for (int e = t; e < nd * r; e += NT) {
         const int i = e % nd, l = e / nd;
         U[i + (size_t)(w.nfroz + l) * nb] = V[i + vmap[l] * ld];
       }
     }
   }
   __syncthreads();
-  for (int e = t; e < nb * w.nfroz; e += kNT) {
+  for (int e = t; e < nb * w.nfroz; e += NT) {
     const int i = e % nb, l = e / nb;
     U[i + (size_t)l * nb] = zmk(i == w.fmin + l ? 1.0 : 0.0, 0.0);
   }
@@ -967,16 +1116,17 @@ __global__ void __launch_bounds__(kNT) k_dis_zmat(DisProb p) {
 // diagonal and the Jacobi rotations go straight into E.  One Newton-Schulz
 // step E <- E (3 I - E^+ E) / 2 then keeps the product of the iterations'
 // rotations orthonormal to rounding (without it the basis drifts by ~n eps
-// per iteration).  LDS: A and E (nd x nd, leading dimension ldz); Z E
+// per iteration), and the same product takes the rotations that the sweeps
+// left to first order.  A and E: nd x nd, leading dimension mz + 1; Z E
 // passes through the Vprev area of global memory.
-template <int N>
-__global__ void __launch_bounds__(kNT) k_dis_update(DisProb p) {
+template <int N, int NT>
+__global__ void __launch_bounds__(NT) k_dis_update(DisProb p) {
   __shared__ JacobiLds<N> J;
   DisState* st = p.st;
   if (st->done) return;
   const int k = dis_blk<N>(p), t = threadIdx.x;
   const Win w = p.win[k];
-  const int nb = p.nb, nw = p.nw, ld = p.ldz, nn = p.nn;
+  const int nb = p.nb, nw = p.nw, ld = p.mz + 1, nn = p.nn;
   const int nd = w.ndim - w.nfroz, r = nw - w.nfroz;
   double fz = 0.0;
   if (t == 0)
@@ -989,10 +1139,10 @@ __global__ void __launch_bounds__(kNT) k_dis_update(DisProb p) {
   const double mix = st->mix;
   zd* Zi = p.Zin + (size_t)k * nb * nb;
   zd* Vp = p.Vprev + (size_t)k * nb * nb;
-  zd* A = dis_ws<N>(p);
-  zd* E = A + ld * p.nzmax;
+  zd* A = dis_mat<N>(p);
+  zd* E = dis_basis<N>(p, (size_t)ld * p.mz);
   const zd* Zp = p.Zpart + (size_t)k * nn * p.ntri;
-  for (int e = t; e < nd * nd; e += kNT) {
+  for (int e = t; e < nd * nd; e += NT) {
     const int i = e % nd, j = e / nd;
     E[i + j * ld] = first ? zmk(i == j ? 1.0 : 0.0, 0.0) : Vp[i + (size_t)j * nb];
     if (i > j) continue;
@@ -1007,16 +1157,16 @@ __global__ void __launch_bounds__(kNT) k_dis_update(DisProb p) {
   __syncthreads();
   if (!first) {
     // Z E into the Vprev area (E holds its contents), then A = E^+ (Z E)
-    zgemm<false>(nd, nd, nd, A, ld, E, ld, [&](int i, int j, zd v) { Vp[i + (size_t)j * nb] = v; });
+    zgemm<NT, false>(nd, nd, nd, A, ld, E, ld, [&](int i, int j, zd v) { Vp[i + (size_t)j * nb] = v; });
     __threadfence_block();
     __syncthreads();
-    zgemm_herm(nd, nd, E, ld, Vp, nb, [&](int i, int j, zd v) {
+    zgemm_herm<NT>(nd, nd, E, ld, Vp, nb, [&](int i, int j, zd v) {
       A[i + j * ld] = i == j ? zmk(v.x, 0.0) : v;
       A[j + i * ld] = zconj(v);
     });
     __syncthreads();
   }
-  const int sweeps = jacobi_run(A, E, nd, ld, J);
+  const int sweeps = jacobi_run<NT>(A, E, nd, ld, ld, J, true);
   if (t == 0) {
     if (sweeps < 0) {
       atomicOr(p.flags, F_JACOBI);
@@ -1027,23 +1177,33 @@ __global__ void __launch_bounds__(kNT) k_dis_update(DisProb p) {
     }
   }
   eig_order(A, nd, ld, J);
-  // E^+ E into the A area (the eigenvalues are in J.lam), then the
-  // Newton-Schulz step to Vprev and the selected columns to U_opt
-  zgemm_herm(nd, nd, E, ld, E, ld, [&](int i, int j, zd v) {
-    A[i + j * ld] = i == j ? zmk(v.x, 0.0) : v;
-    A[j + i * ld] = zconj(v);
+  // E^+ E and the first-order step T of the angles left in A (jacobi_run),
+  // as E^+ E - 2 T into the A area (the eigenvalues are in J.lam; each entry
+  // of A is read by the lane that replaces it).  Then the Newton-Schulz step
+  // and the angles in one product, E (3 - E^+ E + 2 T) / 2, to Vprev, and the
+  // selected columns to U_opt
+  zgemm_herm<NT>(nd, nd, E, ld, E, ld, [&](int i, int j, zd v) {
+    if (i == j) {
+      A[i + i * ld] = zmk(v.x, 0.0);
+      return;
+    }
+    const zd a = A[i + j * ld];
+    const double h = J.lam[j] - J.lam[i];
+    const zd T = h != 0.0 && zabs2(a) <= 1e-16 * h * h ? zscale(a, 1.0 / h) : zmk(0.0, 0.0);
+    A[i + j * ld] = zsub(v, zscale(T, 2.0));
+    A[j + i * ld] = zconj(zadd(v, zscale(T, 2.0)));
   });
   __syncthreads();
   zd* U = p.Uopt + (size_t)k * nb * nw;
   const int lead = nd - r;
-  zgemm<false>(nd, nd, nd, E, ld, A, ld, [&](int i, int j, zd v) {
+  zgemm<NT, false>(nd, nd, nd, E, ld, A, ld, [&](int i, int j, zd v) {
     const zd s = zsub(zscale(E[i + j * ld], 1.5), zscale(v, 0.5));
     Vp[i + (size_t)j * nb] = s;
     const int c = J.rank[j] - lead;
     if (c >= 0) U[nf_row(w, i) + (size_t)(w.nfroz + c) * nb] = s;
   });
   // the frozen rows of the non-frozen columns
-  for (int e = t; e < w.nfroz * r; e += kNT)
+  for (int e = t; e < w.nfroz * r; e += NT)
     U[w.fmin + e % w.nfroz + (size_t)(w.nfroz + e / w.nfroz) * nb] = zmk(0.0, 0.0);
   if (t == 0) {
     double s = (double)nw * p.wbtot;
@@ -1090,17 +1250,18 @@ __global__ void __launch_bounds__(kNT) k_dis_reduce(DisProb p) {
 
 // The Hamiltonian in the optimal subspace, H = U_opt^+ diag(e) U_opt, its
 // eigenvalues into eigopt(1:nw) and U_opt <- U_opt V (ascending order).
-template <int N>
-__global__ void __launch_bounds__(kNT) k_dis_ham(DisProb p) {
+template <int N, int NT>
+__global__ void __launch_bounds__(NT) k_dis_ham(DisProb p) {
   __shared__ JacobiLds<N> J;
   const int k = dis_blk<N>(p), t = threadIdx.x;
   const Win w = p.win[k];
-  const int nb = p.nb, nw = p.nw, ld = p.ld;
+  const int nb = p.nb, nw = p.nw, ld = p.mh + 1;
   zd* U = p.Uopt + (size_t)k * nb * nw;
   const double* e = p.eig + (size_t)k * nb + w.first;
-  zd* H = dis_ws<N>(p);
-  zd* V = H + nb * ld;
-  for (int q = t; q < nw * nw; q += kNT) {
+  zd* H = dis_mat<N>(p);
+  zd* V = dis_basis<N>(p, (size_t)ld * p.mh);
+  zd* W = p.W + (size_t)k * nb * nw;
+  for (int q = t; q < nw * nw; q += NT) {
     const int i = q % nw, j = q / nw;
     if (i > j) continue;
     zd s = zmk(0.0, 0.0);
@@ -1110,21 +1271,22 @@ __global__ void __launch_bounds__(kNT) k_dis_ham(DisProb p) {
     H[j + i * ld] = zconj(s);
   }
   __syncthreads();
-  if (jacobi_eigh(H, V, nw, ld, J) < 0 && t == 0) atomicOr(p.flags, F_JACOBI);
+  if (jacobi_eigh<NT>(H, V, nw, ld, ld, J) < 0 && t == 0) atomicOr(p.flags, F_JACOBI);
   eig_order(H, nw, ld, J);
   if (t < nw) p.eigopt[(size_t)k * nb + t] = J.lam[J.perm[t]];
-  // U_opt V into the H area, then back
-  for (int q = t; q < w.ndim * nw; q += kNT) {
+  // U_opt V into the W area (formed after this kernel), then back
+  for (int q = t; q < w.ndim * nw; q += NT) {
     const int i = q % w.ndim, j = q / w.ndim;
     zd s = zmk(0.0, 0.0);
     const int c = J.perm[j];
     for (int l = 0; l < nw; ++l) zfma(s, U[i + (size_t)l * nb], V[l + c * ld]);
-    H[i + j * ld] = s;
+    W[i + (size_t)j * nb] = s;
   }
+  __threadfence_block();
   __syncthreads();
-  for (int q = t; q < w.ndim * nw; q += kNT) {
+  for (int q = t; q < w.ndim * nw; q += NT) {
     const int i = q % w.ndim, j = q / w.ndim;
-    U[i + (size_t)j * nb] = H[i + j * ld];
+    U[i + (size_t)j * nb] = W[i + (size_t)j * nb];
   }
 }
 
@@ -1132,10 +1294,10 @@ __global__ void __launch_bounds__(kNT) k_dis_ham(DisProb p) {
 // the Zin area, free after the extraction), then W(k) = U_opt(k) U(k).
 template <int N>
 __global__ void __launch_bounds__(kNT) k_dis_find_u(DisProb p) {
-  __shared__ JacobiLds<N> J;
+  __shared__ PolarLds<N> J;
   const int k = dis_blk<N>(p), t = threadIdx.x;
   const Win w = p.win[k];
-  const int nb = p.nb, nw = p.nw, ld = p.ld;
+  const int nb = p.nb, nw = p.nw, ld = p.ldw;
   const zd* Uo = p.Uopt + (size_t)k * nb * nw;
   const zd* A = p.A + (size_t)k * nb * nw + w.first;
   zd* X = p.Zin + (size_t)k * nb * nb;  // nw x nw, leading dimension nw
@@ -1149,7 +1311,7 @@ __global__ void __launch_bounds__(kNT) k_dis_find_u(DisProb p) {
   __syncthreads();
   zd* U = p.U + (size_t)k * nw * nw;
   zd* G = dis_ws<N>(p);
-  polar_factor(X, nw, nw, nw, U, nw, G, G + nb * ld, ld, J, p.flags);
+  polar_factor<kNT>(X, nw, nw, nw, U, nw, G, G + nw * ld, ld, J, p.flags);
   __threadfence_block();
   __syncthreads();
   zd* W = p.W + (size_t)k * nb * nw;
@@ -1167,12 +1329,12 @@ template <int N>
 __global__ void __launch_bounds__(kNT) k_dis_rotate(DisProb p) {
   const int blk = dis_blk<N>(p);
   const int k = blk / p.nn, b = blk % p.nn, t = threadIdx.x;
-  const int nb = p.nb, nw = p.nw, ld = p.ld, nn = p.nn;
+  const int nb = p.nb, nw = p.nw, ld = p.ldc, nn = p.nn;
   const Win w = p.win[k];
   const int k2 = p.nnl[k * nn + b];
   const Win w2 = p.win[k2];
   zd* P = dis_ws<N>(p);  // ndim(k) x nw
-  zd* W2 = P + nb * ld;   // ndim(k+b) x nw
+  zd* W2 = P + nw * ld;   // ndim(k+b) x nw
   const zd* Wk = p.W + (size_t)k * nb * nw;
   const zd* Wkb = p.W + (size_t)k2 * nb * nw;
   for (int e = t; e < w2.ndim * nw; e += kNT) {
@@ -1287,50 +1449,89 @@ struct DevBuf {
   }
 };
 
-// Once per process (calls from several host threads are serialised).
-int set_lds_limits(w90gpu_ctx* ctx, size_t bytes) {
+// Dynamic LDS bytes of an eigenproblem of order m (even): matrix and basis
+// up to kLdsN, the matrix alone up to kHalfN, none above.
+size_t eig_lds(int m) {
+  const size_t one = (size_t)(m + 1) * m * sizeof(zd);
+  return m <= kLdsN ? 2 * one : m <= kHalfN ? one : 0;
+}
+
+// Instantiations of the eigenproblem kernels by largest order: the workgroup
+// that gives the blocks of A one lane each and the rows of E the rest (see
+// jacobi_run), in the memory that holds the matrices.
+template <template <int, int> class K>
+void eig_kernel(int m, void (**fn)(DisProb), int* nt) {
+  if (m <= 16) *fn = K<kLdsN, 192>::fn, *nt = 192;
+  else if (m <= 32) *fn = K<kLdsN, 320>::fn, *nt = 320;
+  else if (m <= 48) *fn = K<kLdsN, 512>::fn, *nt = 512;
+  else if (m <= kLdsN) *fn = K<kLdsN, 1024>::fn, *nt = 1024;
+  else if (m <= kHalfN) *fn = K<kHalfN, 1024>::fn, *nt = 1024;
+  else *fn = K<kMaxN, 1024>::fn, *nt = 1024;
+}
+template <int N, int NT> struct KProjFroz { static constexpr void (*fn)(DisProb) = k_dis_proj_froz<N, NT>; };
+template <int N, int NT> struct KUpdate { static constexpr void (*fn)(DisProb) = k_dis_update<N, NT>; };
+template <int N, int NT> struct KHam { static constexpr void (*fn)(DisProb) = k_dis_ham<N, NT>; };
+
+// One kernel over nblocks workgroups: in one launch where no global area is
+// used, else in launches of at most kGwsBlocks workgroups (each launch
+// reuses the workgroup areas of gws; the stream orders them).
+struct Kern {
+  void (*fn)(DisProb) = nullptr;
+  int nt = kNT;
+  size_t lds = 0;
+  size_t area = 0;  // complex elements of gws per workgroup
+};
+
+void launch(const Kern& K, int nblocks, hipStream_t sm, DisProb p) {
+  const int step = K.area ? kGwsBlocks : nblocks;
+  for (int b0 = 0; b0 < nblocks; b0 += step) {
+    p.blk0 = b0;
+    hipLaunchKernelGGL(K.fn, dim3(std::min(step, nblocks - b0)), dim3(K.nt), K.lds, sm, p);
+  }
+}
+
+template <template <int, int> class K>
+Kern eig_kern(int m) {
+  Kern r;
+  eig_kernel<K>(m, &r.fn, &r.nt);
+  r.lds = eig_lds(m);
+  const size_t one = (size_t)(m + 1) * m;
+  r.area = m <= kLdsN ? 0 : m <= kHalfN ? one : 2 * one;
+  return r;
+}
+
+// A kernel of two blocks of rows x cols (leading dimension ld), in LDS when
+// they fit and its per-column arrays hold them.
+Kern block_kern(void (*in_lds)(DisProb), void (*in_gws)(DisProb), int ld, int cols, bool arrays) {
+  Kern r;
+  const size_t elems = 2 * (size_t)ld * cols;
+  if (elems * sizeof(zd) <= kLdsBytes && (!arrays || cols <= kLdsN)) {
+    r.fn = in_lds;
+    r.lds = elems * sizeof(zd);
+  } else {
+    r.fn = in_gws;
+    r.area = elems;
+  }
+  return r;
+}
+
+// Dynamic LDS above 64 KiB, once per process (calls from several host
+// threads are serialised).
+int set_lds_limits(w90gpu_ctx* ctx) {
   static std::mutex mu;
   static bool done = false;
   std::lock_guard<std::mutex> lock(mu);
   if (done) return W90GPU_OK;
-  const void* ks[] = {(const void*)k_dis_project<kLdsN>, (const void*)k_dis_proj_froz<kLdsN>,
-                      (const void*)k_dis_zmat<kLdsN>,    (const void*)k_dis_update<kLdsN>,
-                      (const void*)k_dis_ham<kLdsN>,     (const void*)k_dis_find_u<kLdsN>,
-                      (const void*)k_dis_rotate<kLdsN>};
-  for (const void* f : ks)
-    DCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+  std::vector<std::pair<void (*)(DisProb), size_t>> ks = {
+      {k_dis_project<kLdsN>, kLdsBytes}, {k_dis_zmat<kLdsN>, kLdsBytes},
+      {k_dis_find_u<kLdsN>, kLdsBytes},  {k_dis_rotate<kLdsN>, kLdsBytes}};
+  for (int m : {16, 32, 48, kLdsN, kHalfN})
+    for (const Kern& K : {eig_kern<KProjFroz>(m), eig_kern<KUpdate>(m), eig_kern<KHam>(m)}) ks.push_back({K.fn, K.lds});
+  for (const auto& f : ks)
+    DCHK(hipFuncSetAttribute((const void*)f.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)f.second));
   done = true;
   return W90GPU_OK;
 }
-
-// A kernel over nblocks workgroups: the LDS instantiation in one launch,
-// the global-memory one in launches of at most kGwsBlocks workgroups (each
-// launch reuses the workgroup areas of gws; the stream orders them).
-template <int N>
-void launch_blocks(void (*kern)(DisProb), int nblocks, size_t lds, hipStream_t sm, DisProb p) {
-  if constexpr (N <= kLdsN) {
-    hipLaunchKernelGGL(kern, dim3(nblocks), dim3(kNT), lds, sm, p);
-  } else {
-    for (int b0 = 0; b0 < nblocks; b0 += kGwsBlocks) {
-      p.blk0 = b0;
-      hipLaunchKernelGGL(kern, dim3(std::min(kGwsBlocks, nblocks - b0)), dim3(kNT), 0, sm, p);
-    }
-  }
-}
-
-// The instantiation that holds a kernel's matrices: LDS when they fit.
-template <template <int> class K>
-void launch_sized(bool global, int nblocks, size_t lds, hipStream_t sm, const DisProb& p) {
-  if (global) launch_blocks<kMaxN>(K<kMaxN>::fn, nblocks, 0, sm, p);
-  else launch_blocks<kLdsN>(K<kLdsN>::fn, nblocks, lds, sm, p);
-}
-template <int N> struct KProject { static constexpr void (*fn)(DisProb) = k_dis_project<N>; };
-template <int N> struct KProjFroz { static constexpr void (*fn)(DisProb) = k_dis_proj_froz<N>; };
-template <int N> struct KZmat { static constexpr void (*fn)(DisProb) = k_dis_zmat<N>; };
-template <int N> struct KUpdate { static constexpr void (*fn)(DisProb) = k_dis_update<N>; };
-template <int N> struct KHam { static constexpr void (*fn)(DisProb) = k_dis_ham<N>; };
-template <int N> struct KFindU { static constexpr void (*fn)(DisProb) = k_dis_find_u<N>; };
-template <int N> struct KRotate { static constexpr void (*fn)(DisProb) = k_dis_rotate<N>; };
 
 }  // namespace
 
@@ -1377,27 +1578,28 @@ int w90gpu_disentangle(w90gpu_ctx* ctx, const w90gpu_problem* prob, int num_band
   int rc = windows(ctx, nb, nw, nk, ctl, eigval, win, eigopt, &linner);
   if (rc) return rc;
   DCHK(hipSetDevice(ctx->device));
-  const int ld = nb + 1;
-  const size_t lds = 2 * (size_t)nb * ld * sizeof(zd);
-  // the per-iteration kernels size their LDS by the windows: k_dis_zmat
-  // holds two ndim x nw blocks, k_dis_update two (ndim - nfroz)^2 blocks
-  // (odd leading dimensions: rows and columns of complex doubles both
-  // spread over the banks)
+  // the kernels size their matrices by the windows (odd leading dimensions:
+  // rows and columns of complex doubles both spread over the banks): two
+  // ndim x nw blocks in the projection, the Z pass and the rotation, two nw x
+  // nw blocks in k_dis_find_u, and the eigenproblems of order ndim - nfroz
+  // (extraction), ndim (frozen projection) and nw (Hamiltonian)
   int ndmax = 1, nzmax = 1;
   for (const Win& wk : win) {
     ndmax = std::max(ndmax, wk.ndim);
     if (nw > wk.nfroz) nzmax = std::max(nzmax, wk.ndim - wk.nfroz);
   }
-  const int ldc = ndmax | 1, ldz = nzmax | 1;
-  const size_t lds_zmat = 2 * (size_t)ldc * nw * sizeof(zd), lds_update = 2 * (size_t)ldz * nzmax * sizeof(zd);
-  if ((rc = set_lds_limits(ctx, kLdsBytes))) return rc;
-  // matrices beyond the LDS go to per-workgroup areas of global memory:
-  // those of the one-time kernels (two nb x (nb + 1) blocks) above kLdsN
-  // bands, those of the extraction kernels when their window blocks do not
-  // fit
-  const bool g_once = nb > kLdsN, g_zmat = lds_zmat > kLdsBytes, g_update = nzmax > kLdsN;
-  const size_t gws_stride = 2 * (size_t)nb * ld;
-  const size_t gws_blocks = (g_once || g_zmat || g_update) ? std::min<size_t>(kGwsBlocks, (size_t)nk * nn) : 0;
+  auto even = [](int n) { return n + (n & 1); };
+  const int ldc = ndmax | 1, ldw = nw | 1, mz = even(nzmax), mq = even(ndmax), mh = even(nw);
+  if ((rc = set_lds_limits(ctx))) return rc;
+  const Kern k_project = block_kern(k_dis_project<kLdsN>, k_dis_project<kMaxN>, ldc, nw, true);
+  const Kern k_zmat = block_kern(k_dis_zmat<kLdsN>, k_dis_zmat<kMaxN>, ldc, nw, false);
+  const Kern k_find_u = block_kern(k_dis_find_u<kLdsN>, k_dis_find_u<kMaxN>, ldw, nw, true);
+  const Kern k_rotate = block_kern(k_dis_rotate<kLdsN>, k_dis_rotate<kMaxN>, ldc, nw, false);
+  const Kern k_proj_froz = eig_kern<KProjFroz>(mq), k_update = eig_kern<KUpdate>(mz), k_ham = eig_kern<KHam>(mh);
+  size_t gws_stride = 0;
+  for (const Kern* K : {&k_project, &k_zmat, &k_find_u, &k_rotate, &k_proj_froz, &k_update, &k_ham})
+    gws_stride = std::max(gws_stride, K->area);
+  const size_t gws_blocks = gws_stride ? std::min<size_t>(kGwsBlocks, (size_t)nk * nn) : 0;
 
   const size_t zb = sizeof(zd);
   const int nlog = std::max(ctl->num_iter, 1);
@@ -1440,7 +1642,6 @@ int w90gpu_disentangle(w90gpu_ctx* ctx, const w90gpu_problem* prob, int num_band
   p.nw = nw;
   p.nk = nk;
   p.nn = nn;
-  p.ld = ld;
   p.wbtot = prob->wbtot;
   p.nnl = (const int*)(base + o_nnl);
   p.wb = (const double*)(base + o_wb);
@@ -1454,8 +1655,10 @@ int w90gpu_disentangle(w90gpu_ctx* ctx, const w90gpu_problem* prob, int num_band
   p.Vprev = (zd*)(base + o_Vprev);
   p.ntri = nb * (nb + 1) / 2;
   p.ldc = ldc;
-  p.nzmax = nzmax;
-  p.ldz = ldz;
+  p.ldw = ldw;
+  p.mz = mz;
+  p.mq = mq;
+  p.mh = mh;
   p.U = (zd*)(base + o_U);
   p.W = (zd*)(base + o_W);
   p.Mw = (zd*)(base + o_Mw);
@@ -1478,8 +1681,8 @@ int w90gpu_disentangle(w90gpu_ctx* ctx, const w90gpu_problem* prob, int num_band
   s0.done = ctl->num_iter == 0 ? 1 : 0;
   hipStream_t sm = nullptr;
   hipLaunchKernelGGL(k_dis_init_state, dim3(1), dim3(1), 0, sm, p.st, s0);
-  launch_sized<KProject>(g_once, nk, lds, sm, p);
-  if (linner) launch_sized<KProjFroz>(g_once, nk, lds, sm, p);
+  launch(k_project, nk, sm, p);
+  if (linner) launch(k_proj_froz, nk, sm, p);
   hipLaunchKernelGGL(k_dis_orthonorm, dim3(nk), dim3(kNT), 0, sm, p);
   DCHK(hipGetLastError());
   int flags = 0;
@@ -1504,14 +1707,14 @@ int w90gpu_disentangle(w90gpu_ctx* ctx, const w90gpu_problem* prob, int num_band
   // the extraction: Z of the initial U_opt, then (update, Z, reduce) per
   // iteration, polled every kPoll iterations
   constexpr int kPoll = 16;
-  launch_sized<KZmat>(g_zmat, nk * nn, lds_zmat, sm, p);
+  launch(k_zmat, nk * nn, sm, p);
   DisState st;
   int launched = 0;
   while (launched < ctl->num_iter) {
     const int n = std::min(kPoll, ctl->num_iter - launched);
     for (int i = 0; i < n; ++i) {
-      launch_sized<KUpdate>(g_update, nk, lds_update, sm, p);
-      launch_sized<KZmat>(g_zmat, nk * nn, lds_zmat, sm, p);
+      launch(k_update, nk, sm, p);
+      launch(k_zmat, nk * nn, sm, p);
       hipLaunchKernelGGL(k_dis_reduce, dim3(1), dim3(kNT), 0, sm, p);
     }
     DCHK(hipGetLastError());
@@ -1519,9 +1722,9 @@ int w90gpu_disentangle(w90gpu_ctx* ctx, const w90gpu_problem* prob, int num_band
     DCHK(hipMemcpy(&st, p.st, sizeof(DisState), hipMemcpyDeviceToHost));
     if (st.done) break;
   }
-  launch_sized<KHam>(g_once, nk, lds, sm, p);
-  launch_sized<KFindU>(g_once, nk, lds, sm, p);
-  launch_sized<KRotate>(g_once, nk * nn, lds, sm, p);
+  launch(k_ham, nk, sm, p);
+  launch(k_find_u, nk, sm, p);
+  launch(k_rotate, nk * nn, sm, p);
   DCHK(hipGetLastError());
   DCHK(hipMemcpy(&st, p.st, sizeof(DisState), hipMemcpyDeviceToHost));
   DCHK(hipMemcpy(&flags, p.flags, sizeof(int), hipMemcpyDeviceToHost));
