@@ -278,7 +278,7 @@ __device__ __forceinline__ bool jacobi_rotates(double b2, double app, double aqq
 }
 
 // Off-diagonal entries left in A (all lanes, one pass): with theta, whether
-// some pair that rotates has an angle above 1e-8 (see jacobi_run), else
+// some pair that rotates has an angle above 5e-9 (see jacobi_run), else
 // whether any pair rotates.
 template <int NT>
 __device__ __forceinline__ bool jacobi_pending(const zd* A, int n, int ld, double floor2, bool theta) {
@@ -288,7 +288,7 @@ __device__ __forceinline__ bool jacobi_pending(const zd* A, int n, int ld, doubl
     if (i >= j) continue;
     const double b2 = zabs2(A[i + j * ld]), aii = A[i + i * ld].x, ajj = A[j + j * ld].x;
     const double h = ajj - aii;
-    if (jacobi_rotates(b2, aii, ajj, floor2) && !(theta && b2 <= 1e-16 * h * h)) any = 1;
+    if (jacobi_rotates(b2, aii, ajj, floor2) && !(theta && b2 <= 2.5e-17 * h * h)) any = 1;
   }
   return __syncthreads_or(any) != 0;
 }
@@ -393,9 +393,9 @@ __device__ __forceinline__ void jacobi_item(int x, int half, int& r1, int& r2) {
 // were both in global memory, 4.34 -> 0.87 ms.
 //
 // theta false: sweeps until no pair rotates.  theta true: sweeps until every
-// angle left is at most 1e-8, where the rest of the method is the first-order
+// angle left is at most 5e-9, where the rest of the method is the first-order
 // step E (1 + T), T_ij = a_ij / (a_jj - a_ii), to rounding (products of two
-// angles are below 1e-16); the caller applies it with its own product.  The
+// angles are below 2.5e-17); the caller applies it with its own product.  The
 // sweeps are checked in one parallel pass before each.  Returns the number
 // of sweeps, or -1 if kMaxSweeps were not enough.  A warm start (a nearly
 // diagonal A) leaves off-diagonal entries just below the skip bounds, so they
@@ -1189,7 +1189,7 @@ __global__ void __launch_bounds__(NT) k_dis_update(DisProb p) {
     }
     const zd a = A[i + j * ld];
     const double h = J.lam[j] - J.lam[i];
-    const zd T = h != 0.0 && zabs2(a) <= 1e-16 * h * h ? zscale(a, 1.0 / h) : zmk(0.0, 0.0);
+    const zd T = h != 0.0 && zabs2(a) <= 2.5e-17 * h * h ? zscale(a, 1.0 / h) : zmk(0.0, 0.0);
     A[i + j * ld] = zsub(v, zscale(T, 2.0));
     A[j + i * ld] = zconj(zadd(v, zscale(T, 2.0)));
   });
