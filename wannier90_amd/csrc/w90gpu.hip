@@ -64,6 +64,7 @@ struct Member {
   int pairs = 0;   // blocks per k that a rotation by pairs forms (0: the mesh has no pairing)
   bool paired = false;  // the loaded M0 holds the pairs' identity
   int* pair_flag = nullptr;  // device result of k_check_pairs
+  int issued = 0;  // iterations enqueued since the start of the solve (corrected from every status)
   int stage = 0;   // 0 idle, 1 queued, 2 running, 3 finished
   w90gpu_control ctl{};
   double wbtot = 0.0;
@@ -243,8 +244,8 @@ struct Engine {
   int cap_items = 0, cap_plist = 0;
   Status* h_status = nullptr;     // [2][cap_plist] pinned
   Status* hd_status = nullptr;    // device address of h_status: k_status writes it directly
-  Final* d_final = nullptr;       // [cap_plist]
-  Final* h_final = nullptr;       // pinned
+  Final* h_final = nullptr;       // [cap_plist] pinned, behind h_status in its allocation
+  Final* hd_final = nullptr;      // device address of h_final: k_gather_final writes it directly
   // run lists of the current epoch
   long epoch = 0, lists_epoch = -1;
   Lists run;
@@ -264,6 +265,7 @@ struct Engine {
   int graph_block = kGraphBlock;  // iterations per block
   hipEvent_t blk_ev[2] = {nullptr, nullptr};
   std::vector<int> blk_slots[2];
+  int blk_iters[2] = {0, 0};      // iterations of the block in each status slot
   hipEvent_t t0 = nullptr, t1 = nullptr;
   std::vector<int> finished_ids;  // retired since the last report
 };
@@ -430,21 +432,20 @@ int grow_tables(Engine* E, int nprob, int nitems) {
   if (nprob > E->cap_plist) {
     const int cap = std::max(nprob, 2 * E->cap_plist);
     HIPCHK(ctx, hipStreamSynchronize(E->stream));
-    for (void* q : {(void*)E->d_plist, (void*)E->d_aux_plist, (void*)E->d_final})
+    for (void* q : {(void*)E->d_plist, (void*)E->d_aux_plist})
       if (q) HIPCHK(ctx, hipFree(q));
     if (E->h_status) HIPCHK(ctx, hipHostFree(E->h_status));
-    if (E->h_final) HIPCHK(ctx, hipHostFree(E->h_final));
     E->d_plist = E->d_aux_plist = nullptr;
-    E->hd_status = nullptr;
-    E->d_final = nullptr;
-    E->h_status = nullptr;
-    E->h_final = nullptr;
+    E->h_status = E->hd_status = nullptr;
+    E->h_final = E->hd_final = nullptr;
     HIPCHK(ctx, hipMalloc(&E->d_plist, sizeof(int) * cap));
     HIPCHK(ctx, hipMalloc(&E->d_aux_plist, sizeof(int) * cap));
-    HIPCHK(ctx, hipMalloc(&E->d_final, sizeof(Final) * cap));
-    HIPCHK(ctx, hipHostMalloc((void**)&E->h_status, sizeof(Status) * 2 * cap, hipHostMallocDefault));
+    // one pinned allocation for both tables the kernels write
+    HIPCHK(ctx, hipHostMalloc((void**)&E->h_status, (sizeof(Status) * 2 + sizeof(Final)) * cap, hipHostMallocDefault));
     HIPCHK(ctx, hipHostGetDevicePointer((void**)&E->hd_status, E->h_status, 0));
-    HIPCHK(ctx, hipHostMalloc((void**)&E->h_final, sizeof(Final) * cap, hipHostMallocDefault));
+    static_assert(sizeof(Status) % alignof(Final) == 0, "Final rows follow the Status rows");
+    E->h_final = reinterpret_cast<Final*>(E->h_status + 2 * cap);
+    E->hd_final = reinterpret_cast<Final*>(E->hd_status + 2 * cap);
     E->cap_plist = cap;
     E->epoch++;  // run lists must be uploaded again
   }
@@ -485,7 +486,9 @@ void engine_destroy(Engine* E);
 
 void tune_refresh();
 
-int engine_create(w90gpu_ctx* ctx, size_t pool_bytes, Engine** out) {
+// own_copy: uploads on a stream of their own, beside the running problems (a
+// batch); else on the compute stream (a session, which has one problem).
+int engine_create(w90gpu_ctx* ctx, size_t pool_bytes, bool own_copy, Engine** out) {
   tune_refresh();
   *out = nullptr;
   HIPCHK(ctx, hipSetDevice(ctx->device));
@@ -494,17 +497,18 @@ int engine_create(w90gpu_ctx* ctx, size_t pool_bytes, Engine** out) {
   E->ctx = ctx;
   auto fail = [&](int code) {
     // partial engine: release what was made
+    if (E->copy && E->copy != E->stream) (void)hipStreamDestroy(E->copy);
     if (E->stream) (void)hipStreamDestroy(E->stream);
-    if (E->copy) (void)hipStreamDestroy(E->copy);
     if (E->pool.base) (void)hipFree(E->pool.base);
     delete E;
     return code;
   };
   if (hipStreamCreateWithFlags(&E->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipStreamCreateWithFlags(&E->copy, hipStreamNonBlocking) != hipSuccess) {
+      (own_copy && hipStreamCreateWithFlags(&E->copy, hipStreamNonBlocking) != hipSuccess)) {
     set_error(ctx, "hipStreamCreate failed");
     return fail(W90GPU_ERR_FATAL);
   }
+  if (!own_copy) E->copy = E->stream;
   pool_bytes = align_up(std::max<size_t>(pool_bytes, 256));
   hipError_t e = hipMalloc((void**)&E->pool.base, pool_bytes);
   if (e != hipSuccess) {
@@ -542,12 +546,11 @@ void engine_destroy(Engine* E) {
   for (hipEvent_t ev : {E->t0, E->t1, E->blk_ev[0], E->blk_ev[1]})
     if (ev) (void)hipEventDestroy(ev);
   for (void* q : {(void*)E->d_probs, (void*)E->d_items, (void*)E->d_plist, (void*)E->d_aux_items,
-                  (void*)E->d_aux_plist, (void*)E->d_final, (void*)E->pool.base})
+                  (void*)E->d_aux_plist, (void*)E->pool.base})
     if (q) (void)hipFree(q);
   if (E->h_status) (void)hipHostFree(E->h_status);
-  if (E->h_final) (void)hipHostFree(E->h_final);
+  if (E->copy && E->copy != E->stream) (void)hipStreamDestroy(E->copy);
   if (E->stream) (void)hipStreamDestroy(E->stream);
-  if (E->copy) (void)hipStreamDestroy(E->copy);
   delete E;
 }
 
@@ -814,27 +817,28 @@ int engine_add(Engine* E, const w90gpu_problem* prob, const w90gpu_control* ctl,
   std::vector<int> hn((size_t)m->nk * m->nn);
   for (int k = 0; k < m->nk; ++k)
     for (int b = 0; b < m->nn; ++b) hn[(size_t)k * m->nn + b] = prob->nnlist[k + (size_t)m->nk * b] - 1;
+  // state, state template, k-mesh and pair tables are neighbours in the arena:
+  // one upload from a staged image of that range
+  const State s = state_template(m, 1, 0.0);
+  char* t0 = (char*)m->p.st;
+  const char* t1 = (const char*)(m->p.wb + m->nn);
   std::vector<int> bord, mate;
   if (m->p.bord) {
     m->pairs = find_pairs(m->nk, m->nn, hn.data(), prob->bk, bord, mate);
-    if (m->pairs > 0 &&
-        (hipMemcpyAsync((void*)m->p.bord, bord.data(), bord.size() * sizeof(int), hipMemcpyHostToDevice, E->stream) !=
-             hipSuccess ||
-         hipMemcpyAsync((void*)m->p.mate, mate.data(), mate.size() * sizeof(int), hipMemcpyHostToDevice, E->stream) !=
-             hipSuccess)) {
-      set_error(ctx, "upload of the pair tables failed");
-      return fail(W90GPU_ERR_FATAL);
-    }
+    if (m->pairs > 0) t1 = (const char*)(m->p.mate + mate.size());
   }
-  const State s = state_template(m, 1, 0.0);
-  if (hipMemcpyAsync((void*)m->p.nnl, hn.data(), hn.size() * sizeof(int), hipMemcpyHostToDevice, E->stream) !=
-          hipSuccess ||
-      hipMemcpyAsync((void*)m->p.bk, prob->bk, (size_t)m->nk * m->nn * 3 * sizeof(double), hipMemcpyHostToDevice,
-                     E->stream) != hipSuccess ||
-      hipMemcpyAsync((void*)m->p.wb, prob->wb, (size_t)m->nn * sizeof(double), hipMemcpyHostToDevice,
-                     E->stream) != hipSuccess ||
-      hipMemcpyAsync(m->st_init, &s, sizeof(State), hipMemcpyHostToDevice, E->stream) != hipSuccess ||
-      hipMemcpyAsync(m->p.st, &s, sizeof(State), hipMemcpyHostToDevice, E->stream) != hipSuccess ||
+  std::vector<char> img(t1 - t0, 0);
+  auto put = [&](const void* dst, const void* src, size_t n) { std::memcpy(img.data() + ((const char*)dst - t0), src, n); };
+  put(m->p.st, &s, sizeof(State));
+  put(m->st_init, &s, sizeof(State));
+  put(m->p.nnl, hn.data(), hn.size() * sizeof(int));
+  put(m->p.bk, prob->bk, (size_t)m->nk * m->nn * 3 * sizeof(double));
+  put(m->p.wb, prob->wb, (size_t)m->nn * sizeof(double));
+  if (m->pairs > 0) {
+    put(m->p.bord, bord.data(), bord.size() * sizeof(int));
+    put(m->p.mate, mate.data(), mate.size() * sizeof(int));
+  }
+  if (hipMemcpyAsync(t0, img.data(), img.size(), hipMemcpyHostToDevice, E->stream) != hipSuccess ||
       hipMemcpyAsync(E->d_probs + slot, &m->p, sizeof(Prob), hipMemcpyHostToDevice, E->stream) != hipSuccess ||
       hipStreamSynchronize(E->stream) != hipSuccess) {
     set_error(ctx, "upload of k-mesh tables failed");
@@ -1281,6 +1285,7 @@ int enqueue_start(Engine* E, const std::vector<Member*>& ms) {
     m->stage = 2;
     m->phase = (m->ctl.precision == W90GPU_PREC_MIXED) ? 0 : 1;
     m->t_start = t;
+    m->issued = 0;
   }
   E->epoch++;
   return W90GPU_OK;
@@ -1311,9 +1316,8 @@ int retire(Engine* E, const std::vector<Member*>& ms) {
   hipLaunchKernelGGL(k_unitarity, dim3(n), dim3(W90_NT), 0, E->stream, E->d_probs, L.items, n);
   HIPCHK(E->ctx, hipGetLastError());
   hipLaunchKernelGGL(k_gather_final, dim3(L.np), dim3(W90_NT), 0, E->stream, E->d_probs, L.plist, L.np,
-                     E->d_final);
+                     E->hd_final);
   HIPCHK(E->ctx, hipGetLastError());
-  HIPCHK(E->ctx, hipMemcpyAsync(E->h_final, E->d_final, sizeof(Final) * L.np, hipMemcpyDeviceToHost, E->stream));
   HIPCHK(E->ctx, hipStreamSynchronize(E->stream));
   const double t = now_s();
   for (size_t i = 0; i < ms.size(); ++i) {
@@ -1404,25 +1408,50 @@ int capture_block(Engine* E, bool lean) {
   return W90GPU_OK;
 }
 
-int enqueue_block(Engine* E, int slot) {
+// Iterations that the running members still need beyond those already
+// enqueued, at most one block: the size of the next block.
+int next_block_iters(const Engine* E) {
+  int n = 0;
+  for (int sl : E->run_slots) {
+    const Member* m = E->slots[sl];
+    if (m && m->stage == 2) n = std::max(n, m->ctl.num_iter - m->issued);
+  }
+  return std::min(n, E->graph_block);
+}
+
+// A block of n iterations over the run lists and its status.  Short of a
+// whole block (the end of a solve) the iterations are launched directly, and
+// a graph is captured only for at least two blocks: a capture costs about as
+// much host time as launching its kernels once, and an iteration past a
+// problem's last one still pays its launches (a 12-iteration solve of 27
+// bands, 216 k: 3.8 ms with the 32 iterations of two fixed blocks, 2.4 ms).
+// n = 0 only reads the status.
+int enqueue_block(Engine* E, int slot, int n) {
   int rc;
   // the first block of an epoch is launched directly; the graph is
   // captured when the membership has stayed the same for a block
-  const bool graph = E->use_graph && !E->graph_failed && E->epoch_blocks >= 1;
+  const bool graph = E->use_graph && !E->graph_failed && E->epoch_blocks >= 1 && n == E->graph_block;
   // without second-step kernels after a processed block in which no problem
   // took a parabolic step (a problem that asks for one then waits for the
   // host, which launches it and returns to full blocks)
   const bool lean = E->use_lean && E->run.any_second && E->clean_blocks >= 1;
   hipGraphExec_t& ge = lean ? E->gexec_lean : E->gexec;
   if (graph && !ge) {
-    if ((rc = capture_block(E, lean))) return rc;
+    int rem = 0;
+    for (int sl : E->run_slots) {
+      const Member* m = E->slots[sl];
+      if (m && m->stage == 2) rem = std::max(rem, m->ctl.num_iter - m->issued);
+    }
+    if (rem >= 2 * E->graph_block && (rc = capture_block(E, lean))) return rc;
   }
   if (graph && ge) {
     HIPCHK(E->ctx, hipGraphLaunch(ge, E->stream));
   } else {
-    for (int i = 0; i < E->graph_block; ++i)
+    for (int i = 0; i < n; ++i)
       if ((rc = enqueue_iteration(E, E->run, lean))) return rc;
   }
+  for (int sl : E->run_slots)
+    if (Member* m = E->slots[sl]) m->issued += n;
   E->epoch_blocks++;
   const int np = E->run.np;
   // the status rows go straight to pinned host memory; the event after the
@@ -1432,6 +1461,7 @@ int enqueue_block(Engine* E, int slot) {
   HIPCHK(E->ctx, hipGetLastError());
   HIPCHK(E->ctx, hipEventRecord(E->blk_ev[slot], E->stream));
   E->blk_slots[slot] = E->run_slots;
+  E->blk_iters[slot] = n;
   return W90GPU_OK;
 }
 
@@ -1451,7 +1481,7 @@ int enqueue_seconds(Engine* E, const std::vector<Member*>& ms) {
   return launch_omega(E, L, MODE_SECOND);
 }
 
-int process_block(Engine* E, int slot, std::vector<Member*>& remix) {
+int process_block(Engine* E, int slot, int ahead, std::vector<Member*>& remix) {
   HIPCHK(E->ctx, hipEventSynchronize(E->blk_ev[slot]));
   const Status* st = E->h_status + (size_t)slot * E->cap_plist;
 
@@ -1462,6 +1492,9 @@ int process_block(Engine* E, int slot, std::vector<Member*>& remix) {
     Member* m = E->slots[sl[i]];
     if (!m || m->stage != 2) continue;
     if (st[i].nsecond > 0) any_second = true;
+    // iterations reached, and those of the blocks still in flight (too many
+    // for a member that holds: corrected when they have been read)
+    m->issued = st[i].iter + ahead;
     if (st[i].done) {
       done.push_back(m);
     } else if (st[i].second) {
@@ -1471,7 +1504,7 @@ int process_block(Engine* E, int slot, std::vector<Member*>& remix) {
       remix.push_back(m);
     }
   }
-  E->clean_blocks = any_second ? 0 : E->clean_blocks + 1;
+  if (E->blk_iters[slot] > 0) E->clean_blocks = any_second ? 0 : E->clean_blocks + 1;
   int rc;
   if (!seconds.empty() && (rc = enqueue_seconds(E, seconds))) return rc;
   if (!done.empty()) return retire(E, done);
@@ -1493,6 +1526,13 @@ int engine_advance(Engine* E, int max_blocks) {
   int issued = 0;
   int inflight = 0, head = 0;  // blocks in flight: slots head, head^1
   std::vector<Member*> remix;
+  // read the status of the oldest block in flight
+  auto process = [&]() -> int {
+    const int slot = head;
+    head ^= 1;
+    --inflight;
+    return process_block(E, slot, inflight ? E->blk_iters[head] : 0, remix);
+  };
   while (true) {
     std::vector<Member*> queued;
     for (Member* m : E->slots)
@@ -1506,30 +1546,26 @@ int engine_advance(Engine* E, int max_blocks) {
     if (max_blocks >= 0 && issued >= max_blocks) break;
     if (E->lists_epoch != E->epoch) {
       // a new epoch: let the blocks in flight finish with the old lists
-      while (inflight > 0) {
-        if ((rc = process_block(E, head, remix))) return rc;
-        head ^= 1;
-        --inflight;
-      }
+      while (inflight > 0)
+        if ((rc = process())) return rc;
       if (!remix.empty()) continue;
       if (running_count(E) == 0) break;
       if ((rc = build_run_lists(E))) return rc;
     }
-    const int slot = (head + inflight) & 1;
-    if ((rc = enqueue_block(E, slot))) return rc;
+    // every iteration of the running members is enqueued: read the blocks in
+    // flight before issuing more
+    const int n = next_block_iters(E);
+    if (n <= 0 && inflight > 0) {
+      if ((rc = process())) return rc;
+      continue;
+    }
+    if ((rc = enqueue_block(E, (head + inflight) & 1, std::max(n, 0)))) return rc;
     ++inflight;
     ++issued;
-    if (inflight == 2) {
-      if ((rc = process_block(E, head, remix))) return rc;
-      head ^= 1;
-      --inflight;
-    }
+    if (inflight == 2 && (rc = process())) return rc;
   }
-  while (inflight > 0) {
-    if ((rc = process_block(E, head, remix))) return rc;
-    head ^= 1;
-    --inflight;
-  }
+  while (inflight > 0)
+    if ((rc = process())) return rc;
   if (!remix.empty() && (rc = enqueue_remix(E, remix))) return rc;
   HIPCHK(E->ctx, hipStreamSynchronize(E->stream));
   reap_graphs(E);
@@ -1543,10 +1579,17 @@ int read_member_state(Engine* E, Member* m, State* out) {
 }
 
 int member_fetch(Engine* E, Member* m, double* m_matrix, double* u_matrix, double* centres, double* spreads) {
+  // the loop state and the centres and <r^2> of both buffers (neighbours in
+  // the arena) in one round
   State st;
+  const char* c0 = (const char*)m->p.rave[0];
+  std::vector<char> cen((const char*)(m->p.r2ave[1] + m->nw) - c0);
+  HIPCHK(E->ctx, hipMemcpyAsync(cen.data(), c0, cen.size(), hipMemcpyDeviceToHost, E->stream));
   int rc = read_member_state(E, m, &st);
   if (rc) return rc;
   const int cur = st.cur;
+  const double* rave = (const double*)(cen.data() + ((const char*)m->p.rave[cur] - c0));
+  const double* r2 = (const double*)(cen.data() + ((const char*)m->p.r2ave[cur] - c0));
   const size_t mb = (size_t)m->nw * m->nw * m->nn * m->nk * sizeof(cplx);
   const size_t ub = (size_t)m->nw * m->nw * m->nk * sizeof(cplx);
   if (m_matrix) {
@@ -1557,13 +1600,8 @@ int member_fetch(Engine* E, Member* m, double* m_matrix, double* u_matrix, doubl
     HIPCHK(E->ctx, hipMemcpyAsync(m_matrix, m->p.M[cur], mb, hipMemcpyDeviceToHost, E->stream));
   }
   if (u_matrix) HIPCHK(E->ctx, hipMemcpyAsync(u_matrix, m->p.U[cur], ub, hipMemcpyDeviceToHost, E->stream));
-  std::vector<double> rave(3 * m->nw), r2(m->nw);
-  HIPCHK(E->ctx, hipMemcpyAsync(rave.data(), m->p.rave[cur], 3 * m->nw * sizeof(double), hipMemcpyDeviceToHost,
-                                E->stream));
-  HIPCHK(E->ctx, hipMemcpyAsync(r2.data(), m->p.r2ave[cur], m->nw * sizeof(double), hipMemcpyDeviceToHost,
-                                E->stream));
   HIPCHK(E->ctx, hipStreamSynchronize(E->stream));
-  if (centres) std::memcpy(centres, rave.data(), 3 * m->nw * sizeof(double));
+  if (centres) std::memcpy(centres, rave, 3 * m->nw * sizeof(double));
   if (spreads)
     for (int n = 0; n < m->nw; ++n) {
       const double rx = rave[3 * n], ry = rave[3 * n + 1], rz = rave[3 * n + 2];
@@ -1767,7 +1805,7 @@ int w90gpu_session_create(w90gpu_ctx* ctx, const w90gpu_problem* prob, const w90
   Layout lay;
   const size_t bytes = problem_layout(prob->num_wann, prob->num_kpts, prob->nntot, ctl->num_iter, lay);
   Engine* E = nullptr;
-  if ((rc = engine_create(ctx, bytes, &E))) return rc;
+  if ((rc = engine_create(ctx, bytes, false, &E))) return rc;
   Member* m = nullptr;
   if ((rc = engine_add(E, prob, ctl, &m))) {
     engine_destroy(E);
@@ -1939,7 +1977,7 @@ int w90gpu_batch_create(w90gpu_ctx* ctx, size_t pool_bytes, w90gpu_batch** out) 
   if (!ctx || !out) return W90GPU_ERR_INPUT;
   *out = nullptr;
   Engine* E = nullptr;
-  int rc = engine_create(ctx, pool_bytes, &E);
+  int rc = engine_create(ctx, pool_bytes, true, &E);
   if (rc) return rc;
   w90gpu_batch* b = new (std::nothrow) w90gpu_batch();
   if (!b) {
