@@ -587,6 +587,7 @@ void member_bind(Member* m, char* a, const Layout& lay) {
   p.W1 = (cplx*)(a + lay.off[i++]);
   p.W2 = (cplx*)(a + lay.off[i++]);
   p.ET = p.W1;
+  p.want_et = m->rk == RK_DIRECT64;
   p.ln[0] = (double*)(a + lay.off[i++]);
   p.ln[1] = (double*)(a + lay.off[i++]);
   p.d2 = (double*)(a + lay.off[i++]);
@@ -1074,19 +1075,14 @@ int launch_step(Engine* E, const Lists& L, int mode) {
   hipStream_t s = E->stream;
   const Seg a = class_range(L, 0, 0), b = class_range(L, 1, 1), c = class_range(L, 2, 2),
             d = class_range(L, 3, 3);
-  if (a.n)
-    hipLaunchKernelGGL(k_step_k<16>, dim3(a.n), dim3(W90_NT), 0, s, E->d_probs, L.items + a.off, a.n, mode);
-  if (b.n)
-    hipLaunchKernelGGL(k_step_k<kLdsMaxWann>, dim3(b.n), dim3(W90_NT), 0, s, E->d_probs, L.items + b.off, b.n,
-                       mode);
-  // num_wann up to 48 on the 48 layout, above on the 64 one (each launch
-  // covers the class; workgroups of the other's items return at once)
+  // one wavefront per 16 columns; 33-64 bands are one class, so both launches
+  // may cover its items and the workgroups of the other's return at once
+  if (a.n) hipLaunchKernelGGL(k_step_panel<1>, dim3(a.n), dim3(64), 0, s, E->d_probs, L.items + a.off, a.n, mode);
+  if (b.n) hipLaunchKernelGGL(k_step_panel<2>, dim3(b.n), dim3(128), 0, s, E->d_probs, L.items + b.off, b.n, mode);
   if (c.n && c.nwmin <= 48)
-    hipLaunchKernelGGL(k_step_mfma<48>, dim3(c.n), dim3(StepWaves<48>::NT), step_mfma_lds<48>(), s, E->d_probs,
-                       L.items + c.off, c.n, mode);
+    hipLaunchKernelGGL(k_step_panel<3>, dim3(c.n), dim3(192), 0, s, E->d_probs, L.items + c.off, c.n, mode);
   if (c.n && c.nwmax > 48)
-    hipLaunchKernelGGL(k_step_mfma<64>, dim3(c.n), dim3(StepWaves<64>::NT), step_mfma_lds<64>(), s, E->d_probs,
-                       L.items + c.off, c.n, mode);
+    hipLaunchKernelGGL(k_step_panel<4>, dim3(c.n), dim3(256), 0, s, E->d_probs, L.items + c.off, c.n, mode);
   if (d.n)
     hipLaunchKernelGGL(k_step, dim3(d.n), dim3(W90_STEP_NT), 0, s, E->d_probs, L.items + d.off, d.n, mode);
   HIPCHK(E->ctx, hipGetLastError());
@@ -1212,6 +1208,7 @@ int tune_member(Engine* E, Member* m) {
   if (pick != d && !(t[pick] <= 0.97 * t[d])) pick = d;
   m->rk = pick;
   m->p.npan = rot_panels(pick, nw);
+  m->p.want_et = pick == RK_DIRECT64;
   HIPCHK(E->ctx, hipMemcpyAsync(E->d_probs + m->slot, &m->p, sizeof(Prob), hipMemcpyHostToDevice, E->stream));
   HIPCHK(E->ctx, hipStreamSynchronize(E->stream));
   TuneCache& tc = tune_cache();
@@ -1240,6 +1237,7 @@ int tune_pending(Engine* E, const std::vector<Member*>& ms) {
       if (rk != m->rk) {
         m->rk = rk;
         m->p.npan = rot_panels(rk, m->nw);
+        m->p.want_et = rk == RK_DIRECT64;
         HIPCHK(E->ctx,
                hipMemcpyAsync(E->d_probs + m->slot, &m->p, sizeof(Prob), hipMemcpyHostToDevice, E->stream));
       }
@@ -1712,8 +1710,6 @@ int w90gpu_create(int device, w90gpu_ctx** ctx) {
   } lds[] = {
       {(const void*)k_rotate_w16<cplx>, rotate_w16_lds<cplx>(W90GPU_NUM_NNMAX)},
       {(const void*)k_rotate_w16<float2>, rotate_w16_lds<float2>(W90GPU_NUM_NNMAX)},
-      {(const void*)k_step_mfma<48>, step_mfma_lds<48>()},
-      {(const void*)k_step_mfma<64>, step_mfma_lds<64>()},
       {(const void*)k_domega_k<16, cplx>, domega_lds<16, cplx>()},
       {(const void*)k_domega_k<16, float2>, domega_lds<16, float2>()},
       {(const void*)k_domega_k<kLdsMaxWann, cplx>, domega_lds<kLdsMaxWann, cplx>()},

@@ -213,8 +213,9 @@ struct State {
 // Device view of one problem: sizes and pointers into its HBM arena.
 struct Prob {
   int nw, nk, nn, npan;
-  int psz, nw2, ngroup, pad;  // psz: per-k partial vector length; ngroup: first-level k-ranges
-                              // (0: the final reduction sums the per-k vectors itself)
+  int psz, nw2, ngroup, want_et;  // psz: per-k partial vector length; ngroup: first-level k-ranges
+                                  // (0: the final reduction sums the per-k vectors itself);
+                                  // want_et: the rotation kernel reads ET
   // npan: tiles of the MFMA rotation per block M(k,b) (num_wann > 16)
   const int* nnl;     // [k][b] 0-based neighbour
   // FP64 rotation by pairs (see rot_pairs): npair blocks (k, b) per k are
@@ -664,13 +665,6 @@ __global__ void __launch_bounds__(W90_NT) k_kpart(const Prob* probs, const Item*
     kpart_bmat(wbL, bkL, nn, out + 8 * nw);
   }
 }
-
-// C = A B (with ident: I + scale A B) of n x n column-major complex
-// matrices in LDS with leading dimension n + 1 (n <= NWM, NWM a multiple of
-// 16), on FP64 MFMA tiles; defined with the other matrix-core code.
-template <int NWM>
-__device__ void lds_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, double scale = 1.0,
-                              bool ident = false);
 
 // ---------------------------------------------------------- omega / control
 
@@ -1442,8 +1436,8 @@ __device__ void search_control(State* st, double gg, double gd) {
 // workgroup sums Re<G,G> and Re<G,D_old> over k in a fixed order (every
 // workgroup of a problem gets the same sums), runs the scalar part on a copy
 // of the state in LDS and forms its D from the result; the workgroup of
-// k = 0 stores the results.  Called by all threads of the block; blockDim
-// must be W90_NT (the summation order depends on it).
+// k = 0 stores the results.  Called by all threads of the block; the
+// summation order depends on blockDim (up to W90_NT).
 __device__ void search_in_step(const Prob& p, int k, State* lst, double* red) {
   constexpr int NSD = sizeof(State) / sizeof(double);
   // the partial sums are requested first, the state copy overlaps them;
@@ -1454,17 +1448,17 @@ __device__ void search_in_step(const Prob& p, int k, State* lst, double* red) {
   const int nsplit = min((int)blockDim.x, W90_NT);
   const int per = (p.nk + nsplit - 1) / nsplit;
   const int kb = threadIdx.x * per, ke = min(p.nk, kb + per);
-  // chunks of 4: the loads of a chunk are issued together, then added in
+  // chunks of 8: the loads of a chunk are issued together, then added in
   // k order
-  for (int q = kb; q < ke; q += 4) {
-    double xg[4], xd[4];
+  for (int q = kb; q < ke; q += 8) {
+    double xg[8], xd[8];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < 8; ++u) {
       xg[u] = (q + u < ke) ? p.part_gg[q + u] : 0.0;
       xd[u] = (q + u < ke) ? p.part_gd[q + u] : 0.0;
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 8; ++u)
       if (q + u < ke) {
         gg += xg[u];
         gd += xd[u];
@@ -1658,145 +1652,6 @@ __global__ void __launch_bounds__(W90_STEP_NT) k_step(const Prob* probs, const I
   for (int e = threadIdx.x; e < nw2; e += blockDim.x) Ek[e] = a[e];
   __syncthreads();
   wg_gemm_mfma(p.U[1 - cur] + (size_t)k * nw2, p.U[cur] + (size_t)k * nw2, Ek, nw);
-}
-
-// Retraction of one (problem, k) with every matrix in LDS (num_wann <= NWM):
-// forms D (trial step), X = scale D, E = exp(X) and U_new = U E.  Padded
-// column-major LDS matrices (leading dimension nw + 1).
-template <int NWM>
-__global__ void __launch_bounds__(W90_NT) k_step_k(const Prob* probs, const Item* items, int nitems, int mode) {
-  if (blockIdx.x >= (unsigned)nitems) return;
-  const Item it = items[blockIdx.x];
-  const Prob& p = probs[it.prob];
-  const State* st = p.st;
-  const int cur = gate_cur(st, mode);
-  if (cur < 0) return;
-  const int nw = p.nw, nw2 = p.nw2;
-  const int ld = nw + 1;
-  const int k = it.k;
-  const int tid = threadIdx.x;
-  __shared__ cplx X[NWM * (NWM + 1)];
-  __shared__ cplx P[NWM * (NWM + 1)];
-  __shared__ cplx T[NWM * (NWM + 1)];
-  __shared__ double red[W90_NT];
-  cplx* Dk = p.D + (size_t)k * nw2;
-  // G, D and U of the k are loaded before the search and the exponential,
-  // so their latency overlaps that work
-  constexpr int SL = (NWM * NWM + W90_NT - 1) / W90_NT;
-  cplx gpre[SL], dpre[SL], upre[SL];
-  {
-    const cplx* Gk = p.G + (size_t)k * nw2;
-    const cplx* Uc = p.U[cur] + (size_t)k * nw2;
-#pragma unroll
-    for (int i = 0; i < SL; ++i) {
-      const int e = tid + i * W90_NT;
-      cplx g = c_make(0.0, 0.0), d = g, u = g;
-      if (e < nw2) {
-        if (mode == MODE_TRIAL) g = Gk[e];
-        d = Dk[e];
-        u = Uc[e];
-      }
-      gpre[i] = g;
-      dpre[i] = d;
-      upre[i] = u;
-    }
-  }
-  __shared__ State lst;
-  const State* ss = st;
-  if (mode == MODE_TRIAL) {
-    search_in_step(p, k, &lst, red);
-    ss = &lst;
-  }
-  const double scale = ss->scale;
-  // X, and the moduli of its elements for the 1-norm (into T, free until
-  // the Taylor products)
-  double* absx = reinterpret_cast<double*>(T);
-  if (mode == MODE_TRIAL) {
-    const double beta = ss->beta, sign = ss->dir_sign;
-#pragma unroll
-    for (int i = 0; i < SL; ++i) {
-      const int e = tid + i * W90_NT;
-      if (e < nw2) {
-        cplx d = c_scale(c_add(gpre[i], c_scale(dpre[i], beta)), sign);
-        st_stream(&Dk[e], d);
-        const int q = (e % nw) + (e / nw) * ld;
-        const cplx x = c_scale(d, scale);
-        X[q] = x;
-        absx[q] = sqrt(c_abs2(x));
-      }
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < SL; ++i) {
-      const int e = tid + i * W90_NT;
-      if (e < nw2) {
-        const int q = (e % nw) + (e / nw) * ld;
-        const cplx x = c_scale(dpre[i], scale);
-        X[q] = x;
-        absx[q] = sqrt(c_abs2(x));
-      }
-    }
-  }
-  __syncthreads();
-  // column j < nw <= 64 is summed by lane j of wavefront 0, whose maximum
-  // is formed by lane exchange and passed on through LDS
-  double cs = 0.0;
-  if (tid < 64) {
-    if (tid < nw) {
-#pragma unroll 4
-      for (int i = 0; i < nw; ++i) cs += absx[i + tid * ld];
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) cs = fmax(cs, __shfl_xor(cs, o));
-    if (tid == 0) red[0] = cs;
-  }
-  __syncthreads();
-  cs = red[0];
-  int sq, m;
-  taylor_plan(cs, &sq, &m);
-  const double f = ldexp(1.0, -sq);
-  const double invm = 1.0 / (double)m;
-  for (int e = tid; e < nw2; e += W90_NT) {
-    const int q = (e % nw) + (e / nw) * ld;
-    const cplx x = c_scale(X[q], f);
-    X[q] = x;
-    cplx v = c_scale(x, invm);
-    if (e % nw == e / nw) v.x += 1.0;
-    P[q] = v;
-  }
-  __syncthreads();
-  // Horner: P <- I + X P / j, the scale and the identity applied as each
-  // product is stored; P and T take turns holding the polynomial
-  cplx* pc = P;
-  cplx* pn = T;
-  for (int j = m - 1; j >= 1; --j) {
-    lds_gemm_mfma<NWM>(pn, X, pc, nw, 1.0 / (double)j, true);
-    cplx* t = pc;
-    pc = pn;
-    pn = t;
-  }
-  cplx* a = pc;
-  cplx* b = pn;
-  for (int s = 0; s < sq; ++s) {
-    lds_gemm_mfma<NWM>(b, a, a, nw);
-    cplx* t = a;
-    a = b;
-    b = t;
-  }
-  cplx* Ek = p.E + (size_t)k * nw2;
-#pragma unroll
-  for (int i = 0; i < SL; ++i) {
-    const int e = tid + i * W90_NT;
-    if (e < nw2) {
-      const int q = (e % nw) + (e / nw) * ld;
-      st_stream(&Ek[e], a[q]);
-      X[q] = upre[i];
-    }
-  }
-  __syncthreads();
-  lds_gemm_mfma<NWM>(b, X, a, nw);
-  cplx* Un = p.U[1 - cur] + (size_t)k * nw2;
-  for (int e = tid; e < nw2; e += W90_NT) st_stream(&Un[e], b[(e % nw) + (e / nw) * ld]);
 }
 
 // ---------------------------------------------------------- projection

@@ -2,7 +2,7 @@
 // M(k,b) <- E_k^+ M(k,b) E_{k+b} as two complex products on
 // v_mfma_*_16x16x4 tiles (FP64 for the plain path, FP32 with FP32
 // accumulation for the mixed bulk phase), and the products of the
-// retraction above num_wann 16.
+// retraction (k_step_panel up to num_wann 64).
 //
 // num_wann <= 16 (k_rotate_w16): one 16 x 16 tile per block, one wavefront
 // per neighbour b.  num_wann 17-64 (k_rot_fused): a workgroup computes both
@@ -91,75 +91,6 @@ struct Real<float2> {
   typedef float type;
 };
 
-
-// C = A B for the LDS retraction (k_step_k): n x n column-major complex
-// matrices in LDS, leading dimension n + 1, n <= NWM.  The product is
-// (NWM/16)^2 tiles of 16 x 16; each (tile, real or imaginary part) is one
-// job of a wavefront: K in steps of 4 on FP64 MFMA 16x16x4, operand
-// fragments read from LDS (zero outside n), the result part written to its
-// half of the complex elements of C.  With ident, C = I + scale A B (one
-// Taylor step, applied as the product is stored).  C must not overlap A or
-// B; the workgroup is synchronised before return.
-template <int NWM>
-__device__ void lds_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, double scale, bool ident) {
-  static_assert(NWM % 16 == 0, "whole 16 x 16 tiles");
-  constexpr int TN = NWM / 16;
-  constexpr int JOBS = 2 * TN * TN;
-  // the job index lives in a scalar register, and operands outside n are
-  // read through a clamped index and a select: no lane branches in the K
-  // loop, so its LDS reads are issued together
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  const int lr = lane & 15, lk = lane >> 4;
-  const int ld = n + 1;
-  const int nwaves = blockDim.x >> 6;
-  double* Cd = reinterpret_cast<double*>(C);
-  for (int job = wave; job < JOBS; job += nwaves) {
-    const int part = job & 1;  // 0: real part, 1: imaginary part
-    const int t = job >> 1;
-    const int ti = t % TN, tj = t / TN;
-    const int i = 16 * ti + lr, j = 16 * tj + lr;
-    double ax[NWM / 4], ay[NWM / 4], bx[NWM / 4], by[NWM / 4];
-#pragma unroll
-    for (int s = 0; s < NWM / 4; ++s) {
-      const int l = 4 * s + lk;
-      const bool oka = i < n && l < n, okb = l < n && j < n;
-      const cplx a = A[oka ? i + l * ld : 0];
-      const cplx bv = B[okb ? l + j * ld : 0];
-      ax[s] = oka ? a.x : 0.0;
-      ay[s] = oka ? a.y : 0.0;
-      bx[s] = okb ? bv.x : 0.0;
-      by[s] = okb ? bv.y : 0.0;
-    }
-    Mfma<double>::acc acc = {0.0, 0.0, 0.0, 0.0};
-    if (part == 0) {
-#pragma unroll
-      for (int s = 0; s < NWM / 4; ++s) {
-        acc = Mfma<double>::mma(ax[s], bx[s], acc);
-        acc = Mfma<double>::mma(-ay[s], by[s], acc);
-      }
-    } else {
-#pragma unroll
-      for (int s = 0; s < NWM / 4; ++s) {
-        acc = Mfma<double>::mma(ax[s], by[s], acc);
-        acc = Mfma<double>::mma(ay[s], bx[s], acc);
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int r = 16 * ti + Mfma<double>::row(lk, q), c = 16 * tj + lr;
-      if (r < n && c < n) {
-        double v = acc[q];
-        if (ident) {
-          v = v * scale;
-          if (part == 0 && r == c) v += 1.0;
-        }
-        Cd[2 * (r + c * ld) + part] = v;
-      }
-    }
-  }
-  __syncthreads();
-}
 
 // output tile edge of a workgroup: 32 up to num_wann 32, 64 above
 __host__ __device__ __forceinline__ int gemm_edge(int nw) { return nw <= 32 ? 32 : 64; }
@@ -898,279 +829,299 @@ __global__ void __launch_bounds__(256) k_reduce_tiles(const Prob* probs, const I
 
 // ---------------------------------------------------------- retraction
 
-// Square complex matrices of edge N in LDS for k_step_mfma<N> (N = 64 for
-// num_wann 49-64, 48 up to 48): planar re/im, column-major with leading
-// dimension N + 1 (MFMA fragment loads of A along a column and of B along
-// a row are both conflict-free with this padding).  Wavefront layout: a 64
-// matrix in 32 x 16 blocks over eight wavefronts (two per SIMD, so one
-// covers the other's LDS waits; the matrices fill the CU's LDS, so there
-// is no second workgroup), a 48 matrix in three 48 x 16 column strips over
-// three (3 x 3 fragments do not split evenly over four), which leaves room
-// in LDS for two workgroups per CU.
 #define W90_STEP_N 64
-template <int N>
-struct StepWaves {
-  static constexpr int LD = N + 1, MAT = N * LD;
-  static constexpr int WR = N == 48 ? 1 : 2, WC = N == 48 ? 3 : 4;
-  static constexpr int NT = 64 * WR * WC;
-  static constexpr int FRR = N / (16 * WR), FRC = N / (16 * WC), FRM = FRR > FRC ? FRR : FRC;
-  static constexpr int MINB = N == 48 ? 2 : 1;  // workgroups per CU (LDS: 75 KB at 48, 133 KB at 64)
-};
 
-// LDS bytes of k_step_mfma<N>: X and P (re, im each) and a reduction buffer.
-template <int N>
-__host__ __device__ constexpr size_t step_mfma_lds() {
-  return sizeof(double) * (4 * StepWaves<N>::MAT + 256);
+// exp(X) as its Taylor polynomial of degree 8 in three products (Bader,
+// Blanes and Casas, Mathematics 7 (2019) 1174, eq. 11):
+//   A4 = X2 (x1 X + x2 X2), X2 = X X,
+//   T8 = 1 + X + y2 X2 + (x3 X2 + A4)(x4 + x5 X + x6 X2 + x7 A4).
+// The remainder is at most r^9 / 9! for ||X||_2 <= r (X is anti-Hermitian, so
+// the scalar bound holds on its spectrum): kTayl8 is the r where that is
+// 1e-18, far below the FP64 rounding of the result, a unitary matrix.
+constexpr double kT8x1 = 0.10836465678522780852, kT8x2 = 0.027091164196306952131, kT8x3 = 0.66666666666666666667,
+                 kT8x4 = 0.54676145797072405251, kT8x5 = 0.16112557339541759283, kT8x6 = 0.014090917158378207731,
+                 kT8x7 = 0.033792797010870504140, kT8y2 = 0.13549236135285063166;
+constexpr double kTayl8 = 0.0414;
+
+// Squarings of exp(X) for ||X||_2 <= r: X is scaled by 2^-s to r <= kTayl8.
+__device__ __forceinline__ int squarings(double r) {
+  if (!isfinite(r)) return 0;  // a non-finite step yields a non-finite U
+  int s = 0;
+  while (r > kTayl8 && s < 64) {
+    r *= 0.5;
+    ++s;
+  }
+  return s;
 }
 
-// C = A B for the 64 x 64 LDS matrices (planar at Ar/Ai, Br/Bi) over the
-// first 4 KS columns of A (rows of B): each wavefront accumulates its 32 x 32 quadrant as 2 x 2 complex
-// FP64 MFMA fragments (three real products per K step, Cfrag).  The rows
-// and columns beyond num_wann are zero in every operand, so all fragments
-// are formed and the K steps past num_wann (up to KS) add zeros.  The K
-// steps are unrolled without branches and the operands of step ks + 1 are
-// read from LDS before the products of step ks are issued: with one
-// wavefront per SIMD nothing else covers the LDS latency.
-template <int KS, int N>
-__device__ __forceinline__ void step_gemm(Cfrag<double> (&C)[StepWaves<N>::FRR][StepWaves<N>::FRC], const double* Ar,
-                                          const double* Ai, const double* Br, const double* Bi) {
-  typedef StepWaves<N> SW;
-  constexpr int FRR = SW::FRR, FRC = SW::FRC, LD = SW::LD;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wr = (w / SW::WC) * (N / SW::WR), wc = (w % SW::WC) * (N / SW::WC);
-  const int lr = lane & 15, lk = lane >> 4;
+// Matrices of 16 TN x 16 TN in k_step_panel: column panel w (16 columns) is
+// held by wavefront w in the result layout of the MFMA, element q of row
+// tile t = row 16 t + 4 q + l / 16, column 16 w + l % 16, which is also the
+// layout of the B operand of K step 4 t + q; a matrix that is an A operand
+// goes to LDS as 16 x 16 tiles, row-major with the column XORed by the row
+// (the store runs along rows and the operand load along columns, both
+// without bank conflicts).
+template <int TN>
+struct Panel {
+  double r[TN][4], i[TN][4];
+};
+constexpr int kStepWaves(int tn) { return tn == 1 ? 4 : tn == 2 ? 3 : 2; }  // wavefronts per SIMD the registers allow
+
+// LDS place of the lane's element (t, q) of its panel
+template <int TN>
+__device__ __forceinline__ int panel_at(int t, int q) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, row = 4 * q + (lane >> 4);
+  return (t * TN + w) * 256 + row * 16 + (lr ^ row);
+}
+template <int TN>
+__device__ __forceinline__ void panel_to_lds(cplx* L, const Panel<TN>& P) {
 #pragma unroll
-  for (int fi = 0; fi < FRR; ++fi)
+  for (int t = 0; t < TN; ++t)
 #pragma unroll
-    for (int fj = 0; fj < FRC; ++fj) C[fi][fj].zero();
-  double ar[2][FRR], ai[2][FRR], br[2][FRC], bi[2][FRC];  // [buffer][fragment]
-  auto load = [&](int ks, int buf) {
+    for (int q = 0; q < 4; ++q) L[panel_at<TN>(t, q)] = c_make(P.r[t][q], P.i[t][q]);
+}
+
+// Row tiles of A B for the wavefront's column panel: A in LDS, element (t,
+// q) of B from get(t, q, re, im); row tile i of the product to out(i, acc).
+template <int TN, class Get, class Out>
+__device__ __forceinline__ void panel_product(const cplx* L, Get get, Out out) {
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  int off[4];
 #pragma unroll
-    for (int f = 0; f < SW::FRM; ++f) {
-      if (f < FRR) {
-        const int ia = (4 * ks + lk) * LD + wr + f * 16 + lr;  // A[row][4 ks + lk]
-        ar[buf][f] = Ar[ia];
-        ai[buf][f] = Ai[ia];
+  for (int q = 0; q < 4; ++q) off[q] = lr * 16 + ((4 * q + lk) ^ lr);
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    Cfrag<double> acc;
+    acc.zero();
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const cplx a = L[(i * TN + t) * 256 + off[q]];
+        double br, bi;
+        get(t, q, br, bi);
+        acc.mma(a.x, a.y, br, bi);
       }
-      if (f < FRC) {
-        const int ib = (wc + f * 16 + lr) * LD + 4 * ks + lk;  // B[4 ks + lk][col]
-        br[buf][f] = Br[ib];
-        bi[buf][f] = Bi[ib];
-      }
+      // no LDS reads of later tiles ahead of the products: their registers
+      // would push the panels out
+      __builtin_amdgcn_sched_barrier(0);
     }
-  };
-  load(0, 0);
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const int cb = ks & 1;
-    if (ks + 1 < KS) load(ks + 1, cb ^ 1);
-#pragma unroll
-    for (int fi = 0; fi < FRR; ++fi)
-#pragma unroll
-      for (int fj = 0; fj < FRC; ++fj) C[fi][fj].mma(ar[cb][fi], ai[cb][fi], br[cb][fj], bi[cb][fj]);
+    out(i, acc);
   }
 }
 
-// step_gemm over the K steps num_wann needs: 12 up to 48 bands, else 16.
-// Each output fragment is the same MFMA sequence in either layout, so a
-// product's result does not depend on N.
-template <int N>
-__device__ __forceinline__ void step_gemm_n(Cfrag<double> (&C)[StepWaves<N>::FRR][StepWaves<N>::FRC],
-                                            const double* Ar, const double* Ai, const double* Br, const double* Bi,
-                                            int n) {
-  if (N > 48 && n > 48) step_gemm<16, N>(C, Ar, Ai, Br, Bi);
-  else step_gemm<12, N>(C, Ar, Ai, Br, Bi);
-}
-
-// Position (row, column) of accumulator element i of fragment (fi, fj).
-template <int N>
-__device__ __forceinline__ void step_pos(int fi, int fj, int i, int* r, int* c) {
-  typedef StepWaves<N> SW;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  *r = (w / SW::WC) * (N / SW::WR) + fi * 16 + Mfma<double>::row(lane >> 4, i);
-  *c = (w % SW::WC) * (N / SW::WC) + fj * 16 + (lane & 15);
-}
-
-// Retraction of one (problem, k) for 32 < num_wann <= 64, every matrix in
-// LDS and every product on FP64 MFMA: forms D (trial step), X = scale D,
-// E = exp(X) by the scaling and squaring of the Taylor polynomial that
-// k_step uses (same plan), and U_new = U E.  The exponential of the
+// Retraction of one (problem, k) for num_wann <= 64: forms D (trial step),
+// X = scale D, E = exp(X) and U_new = U E, one wavefront per 16 columns, TN =
+// ceil(num_wann / 16) of them.  A wavefront's columns of X, X2 and the
+// product in hand stay in its registers; only the left factor of each
+// product goes through LDS, so a product is MFMA instructions with one LDS
+// read per three of them.  ||X||_2 is bounded by ||X2||_F^(1/2) once X2 is
+// known: closer than the 1-norm of X, and it saves squarings.  exp(X) of the
 // anti-Hermitian X is the unitary internal_new_u_and_m builds from the
-// eigenvectors of i X (wannierise.F90:1662-1689, 1729-1734).  N = 48 takes
-// the items of num_wann up to 48 and N = 64 the others (a workgroup whose
-// item is the other's returns at once).
-template <int N>
-__global__ void __launch_bounds__(StepWaves<N>::NT, StepWaves<N>::MINB) k_step_mfma(const Prob* probs,
-                                                                                   const Item* items, int nitems,
-                                                                                   int mode) {
-  typedef StepWaves<N> SW;
-  constexpr int NT = SW::NT, LD = SW::LD, MAT = SW::MAT, FRR = SW::FRR, FRC = SW::FRC;
+// eigenvectors of i X (wannierise.F90:1662-1689, 1729-1734).  Workgroups of
+// items with another TN return at once.
+//
+// What bounds it: three products, the squarings and U E at the rate of the
+// FP64 MFMA pipe for 49-64 bands (four of 5 us per CU and k), the loads and
+// the search below.  Horner's form took a product per degree, 5 to 11 of
+// them, with both factors in LDS.  Measured on the same states, before -> now:
+// 16 bands, 512 k 9.9 -> 7.6 us; 27, 216 k 23.5 -> 12.9; 44, 343 k 53 -> 39;
+// 64, 800 k 180 -> 125.
+template <int TN>
+__global__ void __launch_bounds__(64 * TN, kStepWaves(TN)) k_step_panel(const Prob* probs, const Item* items,
+                                                                       int nitems, int mode) {
   if (blockIdx.x >= (unsigned)nitems) return;
   const Item it = items[blockIdx.x];
   const Prob& p = probs[it.prob];
-  if ((p.nw <= 48) != (N == 48)) return;
+  if ((p.nw + 15) / 16 != TN) return;
   const State* st = p.st;
   const int cur = gate_cur(st, mode);
   if (cur < 0) return;
   const int nw = p.nw, nw2 = p.nw2;
-  const int k = it.k;
-  const int tid = threadIdx.x;
-  extern __shared__ double lds_step[];
-  double* Xr = lds_step;
-  double* Xi = Xr + MAT;
-  double* Pr = Xi + MAT;
-  double* Pi = Pr + MAT;
-  double* red = Pi + MAT;
+  const int k = it.k, lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+  __shared__ cplx L[TN * TN * 256];
+  __shared__ double red[256];
+  __shared__ State lst;
+  const int col = 16 * w + lr;
+  // element (t, q) of the panel: row 16 t + 4 q + lk
+  auto row_of = [&](int t, int q) { return 16 * t + 4 * q + lk; };
+  // a lane's element (t, q) of a block: uniform base, offset o + 16 t + 4 q
+  const unsigned o = (unsigned)(col * nw + lk);
   cplx* Dk = p.D + (size_t)k * nw2;
-  // every G, D and U element of the thread is requested before the search
-  // and the exponential (one workgroup fills a CU's LDS, so there are no
-  // other wavefronts to cover the latency of loads issued one loop trip
-  // at a time)
-  constexpr int SL = N * N / NT;
-  static_assert(SL * NT == N * N, "whole matrix per thread slot");
-  cplx gpre[SL], dpre[SL], upre[SL];
+  // G and D are requested before the search, so their latency overlaps it
+  Panel<TN> X, G;
   {
     const cplx* Gk = p.G + (size_t)k * nw2;
-    const cplx* Uc = p.U[cur] + (size_t)k * nw2;
 #pragma unroll
-    for (int i = 0; i < SL; ++i) {
-      const int e = tid + NT * i;
-      const int r = e % N, c = e / N;
-      cplx g = c_make(0.0, 0.0), d = g, u = g;
-      if (r < nw && c < nw) {
-        const int q = r + c * nw;
-        if (mode == MODE_TRIAL) g = Gk[q];
-        d = Dk[q];
-        u = Uc[q];
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int row = row_of(t, q);
+        cplx g = c_make(0.0, 0.0), d = g;
+        if (row < nw && col < nw) {
+          if (mode == MODE_TRIAL) g = Gk[o + 16 * t + 4 * q];
+          d = Dk[o + 16 * t + 4 * q];
+        }
+        G.r[t][q] = g.x;
+        G.i[t][q] = g.y;
+        X.r[t][q] = d.x;
+        X.i[t][q] = d.y;
       }
-      gpre[i] = g;
-      dpre[i] = d;
-      upre[i] = u;
-    }
   }
-  __shared__ State lst;
   const State* ss = st;
   if (mode == MODE_TRIAL) {
     search_in_step(p, k, &lst, red);
     ss = &lst;
   }
-  const double scale = ss->scale;
-  // X = scale D (zero outside nw), D formed on the trial step, and the
-  // moduli of X for its 1-norm (into the P slot, free until the Taylor
-  // polynomial); each column is then summed in row order by lane c of
-  // wavefront 0, the maximum by lane exchange
+  const double scale = ss->scale, beta = ss->beta, sign = ss->dir_sign;
 #pragma unroll
-  for (int i = 0; i < SL; ++i) {
-    const int e = tid + NT * i;
-    const int r = e % N, c = e / N;
-    cplx x = c_make(0.0, 0.0);
-    if (r < nw && c < nw) {
-      cplx d = dpre[i];
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      cplx d = c_make(X.r[t][q], X.i[t][q]);
       if (mode == MODE_TRIAL) {
-        d = c_scale(c_add(gpre[i], c_scale(d, ss->beta)), ss->dir_sign);
-        st_stream(&Dk[r + c * nw], d);
+        d = c_scale(c_add(c_make(G.r[t][q], G.i[t][q]), c_scale(d, beta)), sign);
+        const int row = row_of(t, q);
+        if (row < nw && col < nw) Dk[o + 16 * t + 4 * q] = d;
       }
-      x = c_scale(d, scale);
+      X.r[t][q] = d.x * scale;
+      X.i[t][q] = d.y * scale;
     }
-    Xr[c * LD + r] = x.x;
-    Xi[c * LD + r] = x.y;
-    Pr[c * LD + r] = sqrt(c_abs2(x));
-  }
+  panel_to_lds<TN>(L, X);
   __syncthreads();
-  double cs = 0.0;
-  if (tid < 64) {
-    if (tid < nw) {
-#pragma unroll 4
-      for (int r = 0; r < nw; ++r) cs += Pr[tid * LD + r];
-    }
+  Panel<TN> Y;  // X2
+  double f2 = 0.0;
+  panel_product<TN>(
+      L, [&](int t, int q, double& br, double& bi) { br = X.r[t][q]; bi = X.i[t][q]; },
+      [&](int i, const Cfrag<double>& acc) {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) cs = fmax(cs, __shfl_xor(cs, o));
-    if (tid == 0) red[0] = cs;
-  }
-  __syncthreads();
-  cs = red[0];
-  int sq, m;
-  taylor_plan(cs, &sq, &m);
-  const double f = ldexp(1.0, -sq);
-  const double invm = 1.0 / (double)m;
-  for (int e = tid; e < N * N; e += NT) {
-    const int r = e % N, c = e / N;
-    const int q = c * LD + r;
-    const double xr = Xr[q] * f, xi = Xi[q] * f;
-    Xr[q] = xr;
-    Xi[q] = xi;
-    Pr[q] = xr * invm + (r == c ? 1.0 : 0.0);
-    Pi[q] = xi * invm;
-  }
-  __syncthreads();
-  Cfrag<double> C[FRR][FRC];
-  // Horner: P <- I + X P / j
-  for (int j = m - 1; j >= 1; --j) {
-    step_gemm_n<N>(C, Xr, Xi, Pr, Pi, nw);
-    __syncthreads();
-    const double invj = 1.0 / (double)j;
-#pragma unroll
-    for (int fi = 0; fi < FRR; ++fi)
-#pragma unroll
-      for (int fj = 0; fj < FRC; ++fj)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          int r, c;
-          step_pos<N>(fi, fj, i, &r, &c);
-          const int q = c * LD + r;
-          Pr[q] = C[fi][fj].re(i) * invj + (r == c ? 1.0 : 0.0);
-          Pi[q] = C[fi][fj].im(i) * invj;
+        for (int q = 0; q < 4; ++q) {
+          const double a = acc.re(q), b = acc.im(q);
+          Y.r[i][q] = a;
+          Y.i[i][q] = b;
+          f2 = fma(a, a, fma(b, b, f2));
         }
-    __syncthreads();
-  }
-  // squarings: P <- P P
+      });
+  // ||X2||_F^2 over the wavefronts in order; every read of X in LDS is done
+  f2 = wave_sum(f2);
+  if (lane == 0) red[w] = f2;
+  __syncthreads();
+  f2 = 0.0;
+#pragma unroll
+  for (int v = 0; v < TN; ++v) f2 += red[v];
+  const int sq = squarings(sqrt(sqrt(f2)));
+  const double f = ldexp(1.0, -sq), ff = f * f;
+#pragma unroll
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      X.r[t][q] *= f;
+      X.i[t][q] *= f;
+      Y.r[t][q] *= ff;
+      Y.i[t][q] *= ff;
+    }
+  panel_to_lds<TN>(L, Y);
+  __syncthreads();
+  Panel<TN> A;  // A4; the panel of X2 is read back from LDS (three panels and
+                // the accumulators do not fit the registers at TN = 4)
+  panel_product<TN>(
+      L,
+      [&](int t, int q, double& br, double& bi) {
+        const cplx y = L[panel_at<TN>(t, q)];
+        br = fma(kT8x2, y.x, kT8x1 * X.r[t][q]);
+        bi = fma(kT8x2, y.y, kT8x1 * X.i[t][q]);
+      },
+      [&](int i, const Cfrag<double>& acc) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          A.r[i][q] = acc.re(q);
+          A.i[i][q] = acc.im(q);
+        }
+      });
+#pragma unroll
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const cplx y = L[panel_at<TN>(t, q)];
+      Y.r[t][q] = y.x;
+      Y.i[t][q] = y.y;
+    }
+  __syncthreads();
+  // the factors of the last product, and 1 + X + y2 X2 into X
+#pragma unroll
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const double one = row_of(t, q) == col ? 1.0 : 0.0;
+      const double xr = X.r[t][q], xi = X.i[t][q], yr = Y.r[t][q], yi = Y.i[t][q], ar = A.r[t][q], ai = A.i[t][q];
+      L[panel_at<TN>(t, q)] = c_make(fma(kT8x3, yr, ar), fma(kT8x3, yi, ai));
+      Y.r[t][q] = fma(kT8x7, ar, fma(kT8x6, yr, fma(kT8x5, xr, kT8x4 * one)));
+      Y.i[t][q] = fma(kT8x7, ai, fma(kT8x6, yi, kT8x5 * xi));
+      X.r[t][q] = one + fma(kT8y2, yr, xr);
+      X.i[t][q] = fma(kT8y2, yi, xi);
+    }
+  __syncthreads();
+  panel_product<TN>(
+      L, [&](int t, int q, double& br, double& bi) { br = Y.r[t][q]; bi = Y.i[t][q]; },
+      [&](int i, const Cfrag<double>& acc) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          X.r[i][q] += acc.re(q);
+          X.i[i][q] += acc.im(q);
+        }
+      });
   for (int s = 0; s < sq; ++s) {
-    step_gemm_n<N>(C, Pr, Pi, Pr, Pi, nw);
     __syncthreads();
-#pragma unroll
-    for (int fi = 0; fi < FRR; ++fi)
-#pragma unroll
-      for (int fj = 0; fj < FRC; ++fj)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          int r, c;
-          step_pos<N>(fi, fj, i, &r, &c);
-          const int q = c * LD + r;
-          Pr[q] = C[fi][fj].re(i);
-          Pi[q] = C[fi][fj].im(i);
-        }
+    panel_to_lds<TN>(L, X);
     __syncthreads();
+    panel_product<TN>(
+        L, [&](int t, int q, double& br, double& bi) { br = X.r[t][q]; bi = X.i[t][q]; },
+        [&](int i, const Cfrag<double>& acc) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            Y.r[i][q] = acc.re(q);
+            Y.i[i][q] = acc.im(q);
+          }
+        });
+    X = Y;
   }
-  // E = P to global, and its transpose ET (rows of E, for the rotation's
-  // operand loads); U into the X slot (zero outside nw)
-  cplx* Ek = p.E + (size_t)k * nw2;
-  cplx* ETk = p.ET + (size_t)k * nw2;
+  // E (and E^T where the rotation reads its operands from it), and U into LDS
+  const cplx* Uc = p.U[cur] + (size_t)k * nw2;
 #pragma unroll
-  for (int i = 0; i < SL; ++i) {
-    const int e = tid + NT * i;
-    const int r = e % N, c = e / N;
-    const int q = c * LD + r;
-    if (r < nw && c < nw) {
-      st_stream(&Ek[r + c * nw], c_make(Pr[q], Pi[q]));
-      const int qt = r * LD + c;  // E[c][r]
-      st_stream(&ETk[r + c * nw], c_make(Pr[qt], Pi[qt]));
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int row = row_of(t, q);
+      cplx u = c_make(0.0, 0.0);
+      if (row < nw && col < nw) u = Uc[o + 16 * t + 4 * q];
+      Y.r[t][q] = u.x;
+      Y.i[t][q] = u.y;
     }
-    Xr[q] = upre[i].x;
-    Xi[q] = upre[i].y;
-  }
-  __syncthreads();
-  step_gemm_n<N>(C, Xr, Xi, Pr, Pi, nw);
-  cplx* Un = p.U[1 - cur] + (size_t)k * nw2;
+  cplx* Ek = p.E + (size_t)k * nw2;
 #pragma unroll
-  for (int fi = 0; fi < FRR; ++fi)
+  for (int t = 0; t < TN; ++t)
 #pragma unroll
-    for (int fj = 0; fj < FRC; ++fj)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        int r, c;
-        step_pos<N>(fi, fj, i, &r, &c);
-        if (r < nw && c < nw) st_stream(&Un[r + c * nw], c_make(C[fi][fj].re(i), C[fi][fj].im(i)));
+    for (int q = 0; q < 4; ++q) {
+      const int row = row_of(t, q);
+      if (row < nw && col < nw) {
+        const cplx e = c_make(X.r[t][q], X.i[t][q]);
+        Ek[o + 16 * t + 4 * q] = e;
+        if (p.want_et) p.ET[(size_t)k * nw2 + col + (size_t)row * nw] = e;
       }
+    }
+  __syncthreads();
+  panel_to_lds<TN>(L, Y);
+  __syncthreads();
+  cplx* Un = p.U[1 - cur] + (size_t)k * nw2;
+  panel_product<TN>(
+      L, [&](int t, int q, double& br, double& bi) { br = X.r[t][q]; bi = X.i[t][q]; },
+      [&](int i, const Cfrag<double>& acc) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int row = row_of(i, q);
+          if (row < nw && col < nw) Un[o + 16 * i + 4 * q] = c_make(acc.re(q), acc.im(q));
+        }
+      });
 }
 
 // C = A B for n x n column-major complex matrices in global memory, held by
