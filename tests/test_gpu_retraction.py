@@ -47,3 +47,31 @@ def test_retraction_matches_eigenvectors(ctx, nw):
             k2 = p.kmesh.nnlist[:, b] - 1
             mk = np.conj(np.transpose(e, (0, 2, 1))) @ np.transpose(m0[:, :, b, :], (2, 0, 1)) @ e[k2]
             assert np.abs(np.transpose(m[:, :, b, :], (2, 0, 1)) - mk).max() <= tol
+
+
+@pytest.mark.parametrize("nw", [1, 3, 16, 17, 32, 33, 48, 49, 64, 65, 90])
+def test_projection_matches_svd(ctx, nw):
+    """overlap_project at the edges of the panels: singular values in [0.3,
+    1.3], so the polar factor is known to a few nw eps (1e-12); a singular or
+    non-finite A is refused."""
+    from wannier90_amd import capi, synth
+
+    print(f"[projection] nw {nw}", flush=True)
+    p = synth.make_problem(77 + nw, kind="sc", nw=nw, mp=(2, 2, 2), decay=2.0)
+    rng = np.random.default_rng(nw)
+    a = rng.normal(size=(8, nw, nw)) + 1j * rng.normal(size=(8, nw, nw))
+    z, _, vh = np.linalg.svd(a)
+    a = (z * rng.uniform(0.3, 1.3, size=(8, 1, nw))) @ vh
+    ref = z @ vh
+    af = np.asfortranarray(np.transpose(a, (1, 2, 0)))
+    m = np.array(p.m_orig, order="F")
+    u = ctx.project(p.kmesh, af, m)
+    assert np.abs(np.transpose(u, (2, 0, 1)) - ref).max() <= 1e-12
+    k2 = p.kmesh.nnlist[:, 0] - 1
+    mk = np.conj(np.transpose(ref, (0, 2, 1))) @ np.transpose(p.m_orig[:, :, 0, :], (2, 0, 1)) @ ref[k2]
+    assert np.abs(np.transpose(m[:, :, 0, :], (2, 0, 1)) - mk).max() <= 1e-11
+    for bad in (0.0, np.nan, np.inf):
+        b = af.copy(order="F")
+        b[:, 0, 3] = bad
+        with pytest.raises(capi.W90Error):
+            ctx.project(p.kmesh, b, np.array(p.m_orig, order="F"))

@@ -1083,7 +1083,11 @@ int launch_step(Engine* E, const Lists& L, int mode) {
     hipLaunchKernelGGL(k_step_panel<3>, dim3(c.n), dim3(192), 0, s, E->d_probs, L.items + c.off, c.n, mode);
   if (c.n && c.nwmax > 48)
     hipLaunchKernelGGL(k_step_panel<4>, dim3(c.n), dim3(256), 0, s, E->d_probs, L.items + c.off, c.n, mode);
-  if (d.n)
+  if (d.n && d.nwmin <= 80)
+    hipLaunchKernelGGL(k_step_panel<5>, dim3(d.n), dim3(320), 0, s, E->d_probs, L.items + d.off, d.n, mode);
+  if (d.n && d.nwmin <= 96 && d.nwmax > 80)
+    hipLaunchKernelGGL(k_step_panel<6>, dim3(d.n), dim3(384), 0, s, E->d_probs, L.items + d.off, d.n, mode);
+  if (d.n && d.nwmax > 96)
     hipLaunchKernelGGL(k_step, dim3(d.n), dim3(W90_STEP_NT), 0, s, E->d_probs, L.items + d.off, d.n, mode);
   HIPCHK(E->ctx, hipGetLastError());
   return W90GPU_OK;
@@ -2310,7 +2314,12 @@ int w90gpu_project(w90gpu_ctx* ctx, const w90gpu_problem* prob, const double* a_
     HIPCHK(ctx, hipMemcpyAsync(m->p.G, a_matrix, ub, hipMemcpyHostToDevice, E->stream));
     HIPCHK(ctx, hipMemcpyAsync(m->p.M[0], m_matrix, mb, hipMemcpyHostToDevice, E->stream));
     hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, E->stream, E->d_probs, L.plist, 1);
-    hipLaunchKernelGGL(k_polar, dim3(n), dim3(W90_NT), 0, E->stream, E->d_probs, L.items, n);
+    const int tn = (m->nw + 15) / 16;
+    if (tn == 1) hipLaunchKernelGGL(k_polar_panel<1>, dim3(n), dim3(64), 0, E->stream, E->d_probs, L.items, n);
+    else if (tn == 2) hipLaunchKernelGGL(k_polar_panel<2>, dim3(n), dim3(128), 0, E->stream, E->d_probs, L.items, n);
+    else if (tn == 3) hipLaunchKernelGGL(k_polar_panel<3>, dim3(n), dim3(192), 0, E->stream, E->d_probs, L.items, n);
+    else if (tn == 4) hipLaunchKernelGGL(k_polar_panel<4>, dim3(n), dim3(256), 0, E->stream, E->d_probs, L.items, n);
+    else hipLaunchKernelGGL(k_polar, dim3(n), dim3(W90_STEP_NT), 0, E->stream, E->d_probs, L.items, n);
     HIPCHK(ctx, hipGetLastError());
     hipLaunchKernelGGL(k_transpose_e, dim3(n), dim3(W90_NT), 0, E->stream, E->d_probs, L.items, n);
     HIPCHK(ctx, hipGetLastError());

@@ -42,7 +42,8 @@
 typedef double2 cplx;
 
 #define W90_NT 256          // threads per workgroup of the per-k kernels
-#define W90_STEP_NT 1024    // threads of the global-memory retraction (above 64 bands)
+#define W90_STEP_NT 1024    // threads of the global-memory retraction (above W90_PANEL_MAX bands)
+#define W90_PANEL_MAX 96    // most bands whose matrix fits a workgroup's LDS (k_step_panel)
 #define W90_FINAL_NT 1024   // threads of the per-problem omega kernel
 #define W90_MAX_GROUPS 32   // k-ranges of the first omega reduction level
 #define W90_MIXED_RTOL 1e-8 // relative FP32 noise floor of Omega differences in the bulk phase
@@ -1488,54 +1489,33 @@ __device__ void search_in_step(const Prob& p, int k, State* lst, double* red) {
 
 // ---------------------------------------------------------- retraction
 
-// Degree and squarings of the Taylor approximant of exp(X) for ||X||_1 = nrm:
-// X is scaled by 2^-sq to norm <= 1/8, and the degree m is the smallest with
-// (nrm/2^sq)^(m+1)/(m+1)! < 1e-18, far below the FP64 rounding of the
-// result (the exponential of an anti-Hermitian matrix is unitary, norm 1).
-__device__ __forceinline__ void taylor_plan(double nrm, int* sq_out, int* m_out) {
-  if (!isfinite(nrm)) nrm = 0.0;  // a non-finite step yields a non-finite U
-  int sq = 0;
-  while (nrm > 0.125 && sq < 64) {
-    nrm *= 0.5;
-    ++sq;
+// exp(X) as its Taylor polynomial of degree 8 in three products (Bader,
+// Blanes and Casas, Mathematics 7 (2019) 1174, eq. 11):
+//   A4 = X2 (x1 X + x2 X2), X2 = X X,
+//   T8 = 1 + X + y2 X2 + (x3 X2 + A4)(x4 + x5 X + x6 X2 + x7 A4).
+// The remainder is at most r^9 / 9! for ||X||_2 <= r (X is anti-Hermitian, so
+// the scalar bound holds on its spectrum): kTayl8 is the r where that is
+// 1e-18, far below the FP64 rounding of the result, a unitary matrix.
+constexpr double kT8x1 = 0.10836465678522780852, kT8x2 = 0.027091164196306952131, kT8x3 = 0.66666666666666666667,
+                 kT8x4 = 0.54676145797072405251, kT8x5 = 0.16112557339541759283, kT8x6 = 0.014090917158378207731,
+                 kT8x7 = 0.033792797010870504140, kT8y2 = 0.13549236135285063166;
+constexpr double kTayl8 = 0.0414;
+
+// Squarings of exp(X) for ||X||_2 <= r: X is scaled by 2^-s to r <= kTayl8.
+__device__ __forceinline__ int squarings(double r) {
+  if (!isfinite(r)) return 0;  // a non-finite step yields a non-finite U
+  int s = 0;
+  while (r > kTayl8 && s < 64) {
+    r *= 0.5;
+    ++s;
   }
-  int m = 1;
-  double term = nrm;
-  while (m < 24) {
-    term = term * nrm / (double)(m + 1);
-    if (term < 1e-18) break;
-    ++m;
-  }
-  *sq_out = sq;
-  *m_out = m;
+  return s;
 }
 
-// C = A * B for n x n column-major complex matrices held by one workgroup.
-__device__ void wg_gemm(cplx* C, const cplx* A, const cplx* B, int n) {
-  const int n2 = n * n;
-  for (int e = threadIdx.x; e < n2; e += blockDim.x) {
-    const int i = e % n, j = e / n;
-    const cplx* bc = B + (size_t)j * n;
-    cplx acc = c_make(0.0, 0.0);
-    for (int l = 0; l < n; ++l) acc = c_add(acc, c_mul(A[i + (size_t)l * n], bc[l]));
-    C[e] = acc;
-  }
-  __syncthreads();
-}
-
-// C = A^+ B for n x n column-major complex matrices held by one workgroup.
-__device__ void wg_gemm_cn(cplx* C, const cplx* A, const cplx* B, int n) {
-  const int n2 = n * n;
-  for (int e = threadIdx.x; e < n2; e += blockDim.x) {
-    const int i = e % n, j = e / n;
-    const cplx* ac = A + (size_t)i * n;
-    const cplx* bc = B + (size_t)j * n;
-    cplx acc = c_make(0.0, 0.0);
-    for (int l = 0; l < n; ++l) acc = c_add(acc, c_cmul(ac[l], bc[l]));
-    C[e] = acc;
-  }
-  __syncthreads();
-}
+// C = A B or (adj) A^+ B on FP64 MFMA for matrices in global memory, by one
+// workgroup (w90gpu_mfma.h).
+__device__ void wg_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, double scale = 1.0,
+                             bool ident = false, bool adj = false);
 
 // ET(k) = E(k)^T for one k by one workgroup (E written by this workgroup
 // before; the caller synchronised it): coalesced writes, reads along rows.
@@ -1555,7 +1535,7 @@ __global__ void __launch_bounds__(W90_NT) k_delta_u(const Prob* probs, const Ite
   const State* st = p.st;
   if (!gate(st, MODE_REMIX)) return;
   const size_t o = (size_t)it.k * p.nw2;
-  wg_gemm_cn(p.E + o, p.U0 + o, p.U[st->cur] + o, p.nw);
+  wg_gemm_mfma(p.E + o, p.U0 + o, p.U[st->cur] + o, p.nw, 1.0, false, true);
   wg_transpose_e(p, it.k);
 }
 
@@ -1567,22 +1547,16 @@ __global__ void __launch_bounds__(W90_NT) k_transpose_e(const Prob* probs, const
   wg_transpose_e(probs[it.prob], it.k);
 }
 
-// C = A * B (with ident: I + scale A B) on FP64 MFMA for matrices in global
-// memory (w90gpu_mfma.h).
-__device__ void wg_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, double scale = 1.0,
-                             bool ident = false);
-
 // Retraction of one (problem, k) with workspaces in global memory (num_wann
 // above the LDS kernels): forms the search direction D (trial step only), X = scale * D,
-// E = exp(X) by scaling and squaring of a Taylor polynomial, and U_new = U E.
-// X is anti-Hermitian, so exp(X) is the same unitary that
-// internal_new_u_and_m builds from the eigenvectors of i X
-// (wannierise.F90:1662-1689, 1729-1734).
+// E = exp(X) as in k_step_panel, and U_new = U E (128 bands, 125 k: 694 ->
+// 394 us against Horner's form of a Taylor polynomial).
 __global__ void __launch_bounds__(W90_STEP_NT) k_step(const Prob* probs, const Item* items, int nitems, int mode) {
   if (blockIdx.x >= (unsigned)nitems) return;
   const Item it = items[blockIdx.x];
   const Prob& p = probs[it.prob];
   const State* st = p.st;
+  if (p.nw <= W90_PANEL_MAX) return;  // k_step_panel
   const int cur = gate_cur(st, mode);
   if (cur < 0) return;
   const int nw = p.nw, nw2 = p.nw2;
@@ -1611,37 +1585,36 @@ __global__ void __launch_bounds__(W90_STEP_NT) k_step(const Prob* probs, const I
     for (int e = threadIdx.x; e < nw2; e += blockDim.x) X[e] = c_scale(Dk[e], scale);
   }
   __syncthreads();
-  double cs = 0.0;
-  for (int j = threadIdx.x; j < nw; j += blockDim.x) {
-    double s = 0.0;
-    for (int i = 0; i < nw; ++i) s += sqrt(c_abs2(X[i + (size_t)j * nw]));
-    cs = fmax(cs, s);
-  }
-  int sq, m;
-  taylor_plan(block_max(cs, red), &sq, &m);
-  if (sq > 0) {
-    const double f = ldexp(1.0, -sq);
-    for (int e = threadIdx.x; e < nw2; e += blockDim.x) X[e] = c_scale(X[e], f);
-  }
-  __syncthreads();
-  const double invm = 1.0 / (double)m;
+  // X2 (into P), its scaling, x1 X + x2 X2 (into E) and A4 (into the buffer of
+  // the new U, written last)
+  wg_gemm_mfma(P, X, X, nw);
+  double f2 = 0.0;
+  for (int e = threadIdx.x; e < nw2; e += blockDim.x) f2 += c_abs2(P[e]);
+  const int sq = squarings(sqrt(sqrt(block_sum(f2, red))));
+  const double f = ldexp(1.0, -sq), ff = f * f;
   for (int e = threadIdx.x; e < nw2; e += blockDim.x) {
-    cplx v = c_scale(X[e], invm);
-    if (e % nw == e / nw) v.x += 1.0;
-    P[e] = v;
+    const cplx x = c_scale(X[e], f), y = c_scale(P[e], ff);
+    X[e] = x;
+    P[e] = y;
+    Ek[e] = c_add(c_scale(x, kT8x1), c_scale(y, kT8x2));
   }
   __syncthreads();
-  // Horner: P <- I + X P / j, the scale and the identity applied as each
-  // product is stored; P and E take turns holding the polynomial
-  cplx* pc = P;
-  cplx* pn = Ek;
-  for (int j = m - 1; j >= 1; --j) {
-    wg_gemm_mfma(pn, X, pc, nw, 1.0 / (double)j, true);
-    cplx* t = pc;
-    pc = pn;
-    pn = t;
+  cplx* A4 = p.U[1 - cur] + (size_t)k * nw2;
+  wg_gemm_mfma(A4, P, Ek, nw);
+  // the factors of the last product into P and A4, 1 + X + y2 X2 into X
+  for (int e = threadIdx.x; e < nw2; e += blockDim.x) {
+    const cplx x = X[e], y = P[e], q = A4[e];
+    const double one = e % nw == e / nw ? 1.0 : 0.0;
+    P[e] = c_add(c_scale(y, kT8x3), q);
+    A4[e] = c_make(fma(kT8x7, q.x, fma(kT8x6, y.x, fma(kT8x5, x.x, kT8x4 * one))),
+                   fma(kT8x7, q.y, fma(kT8x6, y.y, kT8x5 * x.y)));
+    X[e] = c_make(one + fma(kT8y2, y.x, x.x), fma(kT8y2, y.y, x.y));
   }
-  cplx* a = pc;
+  __syncthreads();
+  wg_gemm_mfma(Ek, P, A4, nw);
+  for (int e = threadIdx.x; e < nw2; e += blockDim.x) Ek[e] = c_add(Ek[e], X[e]);
+  __syncthreads();
+  cplx* a = Ek;
   cplx* b = X;
   for (int s = 0; s < sq; ++s) {
     wg_gemm_mfma(b, a, a, nw);
@@ -1649,83 +1622,8 @@ __global__ void __launch_bounds__(W90_STEP_NT) k_step(const Prob* probs, const I
     a = b;
     b = t;
   }
-  for (int e = threadIdx.x; e < nw2; e += blockDim.x) Ek[e] = a[e];
+  if (a != Ek)
+    for (int e = threadIdx.x; e < nw2; e += blockDim.x) Ek[e] = a[e];
   __syncthreads();
   wg_gemm_mfma(p.U[1 - cur] + (size_t)k * nw2, p.U[cur] + (size_t)k * nw2, Ek, nw);
-}
-
-// ---------------------------------------------------------- projection
-
-// Lowdin orthonormalisation of overlap_project (src/overlap.F90:758-952)
-// for num_bands = num_wann: the unitary polar factor U = A (A^+ A)^-1/2 of
-// A(k) (staged in G), which is the Z V^+ built there from the SVD
-// A = Z S V^+.  Newton-Schulz iteration X <- X (3 - X^+ X)/2 from
-// X = A/||A||_F (all singular values in (0,1]) converges to it for
-// non-singular A, quadratically near the end: once X^+ X = 1 to 1e-12 one
-// more step reaches rounding level and the iteration stops (at most 200
-// steps).  Writes U(k) to E.
-__global__ void __launch_bounds__(W90_NT) k_polar(const Prob* probs, const Item* items, int nitems) {
-  if (blockIdx.x >= (unsigned)nitems) return;
-  const Item it = items[blockIdx.x];
-  const Prob& p = probs[it.prob];
-  const int nw = p.nw, nw2 = p.nw2;
-  const int k = it.k;
-  cplx* X = p.E + (size_t)k * nw2;
-  cplx* Y = p.W1 + (size_t)k * nw2;
-  cplx* Z = p.W2 + (size_t)k * nw2;
-  __shared__ double red[W90_NT];
-  const cplx* Ak = p.G + (size_t)k * nw2;
-  double fro = 0.0;
-  for (int e = threadIdx.x; e < nw2; e += blockDim.x) fro += c_abs2(Ak[e]);
-  fro = sqrt(block_sum(fro, red));
-  const double inv = (fro > 0.0 && isfinite(fro)) ? 1.0 / fro : 0.0;
-  for (int e = threadIdx.x; e < nw2; e += blockDim.x) X[e] = c_scale(Ak[e], inv);
-  __syncthreads();
-  for (int iter = 0; iter < 200; ++iter) {
-    wg_gemm_cn(Y, X, X, nw);
-    double dev = 0.0;
-    for (int e = threadIdx.x; e < nw2; e += blockDim.x) {
-      cplx y = Y[e];
-      if (e % nw == e / nw) y.x -= 1.0;
-      dev = fmax(dev, sqrt(c_abs2(y)));
-      // 3 - X^+ X, halved below
-      Y[e] = c_make(-Y[e].x + ((e % nw == e / nw) ? 3.0 : 0.0), -Y[e].y);
-    }
-    dev = block_max(dev, red);
-    if (!(dev == dev)) break;  // non-finite input: left to the unitarity check
-    wg_gemm(Z, X, Y, nw);
-    for (int e = threadIdx.x; e < nw2; e += blockDim.x) X[e] = c_scale(Z[e], 0.5);
-    __syncthreads();
-    if (dev < 1e-12) break;
-  }
-}
-
-// wann_check_unitarity (wannierise.F90:2594-2661): per-k maximum deviation
-// of U U^+ and U^+ U from the identity (NaN-propagating).
-__global__ void __launch_bounds__(W90_NT) k_unitarity(const Prob* probs, const Item* items, int nitems) {
-  if (blockIdx.x >= (unsigned)nitems) return;
-  const Item it = items[blockIdx.x];
-  const Prob& p = probs[it.prob];
-  const int nw = p.nw, nw2 = p.nw2;
-  const int k = it.k;
-  const cplx* U = p.U[p.st->cur] + (size_t)k * nw2;
-  __shared__ double red[W90_NT];
-  double dev = 0.0;
-  for (int e = threadIdx.x; e < nw2; e += blockDim.x) {
-    const int i = e % nw, j = e / nw;
-    cplx c1 = c_make(0, 0), c2 = c_make(0, 0);
-    for (int m = 0; m < nw; ++m) {
-      c1 = c_add(c1, c_mul(U[i + m * nw], c_conj(U[j + m * nw])));
-      c2 = c_add(c2, c_mul(U[m + j * nw], c_conj(U[m + i * nw])));
-    }
-    if (i == j) {
-      c1.x -= 1.0;
-      c2.x -= 1.0;
-    }
-    const double v = fmax(sqrt(c_abs2(c1)), sqrt(c_abs2(c2)));
-    if (!(v <= dev)) dev = isnan(v) ? INFINITY : fmax(v, dev);
-    if (isnan(c1.x) || isnan(c1.y) || isnan(c2.x) || isnan(c2.y)) dev = INFINITY;
-  }
-  dev = block_max(dev, red);
-  if (threadIdx.x == 0) p.unit[k] = dev;
 }

@@ -831,29 +831,6 @@ __global__ void __launch_bounds__(256) k_reduce_tiles(const Prob* probs, const I
 
 #define W90_STEP_N 64
 
-// exp(X) as its Taylor polynomial of degree 8 in three products (Bader,
-// Blanes and Casas, Mathematics 7 (2019) 1174, eq. 11):
-//   A4 = X2 (x1 X + x2 X2), X2 = X X,
-//   T8 = 1 + X + y2 X2 + (x3 X2 + A4)(x4 + x5 X + x6 X2 + x7 A4).
-// The remainder is at most r^9 / 9! for ||X||_2 <= r (X is anti-Hermitian, so
-// the scalar bound holds on its spectrum): kTayl8 is the r where that is
-// 1e-18, far below the FP64 rounding of the result, a unitary matrix.
-constexpr double kT8x1 = 0.10836465678522780852, kT8x2 = 0.027091164196306952131, kT8x3 = 0.66666666666666666667,
-                 kT8x4 = 0.54676145797072405251, kT8x5 = 0.16112557339541759283, kT8x6 = 0.014090917158378207731,
-                 kT8x7 = 0.033792797010870504140, kT8y2 = 0.13549236135285063166;
-constexpr double kTayl8 = 0.0414;
-
-// Squarings of exp(X) for ||X||_2 <= r: X is scaled by 2^-s to r <= kTayl8.
-__device__ __forceinline__ int squarings(double r) {
-  if (!isfinite(r)) return 0;  // a non-finite step yields a non-finite U
-  int s = 0;
-  while (r > kTayl8 && s < 64) {
-    r *= 0.5;
-    ++s;
-  }
-  return s;
-}
-
 // Matrices of 16 TN x 16 TN in k_step_panel: column panel w (16 columns) is
 // held by wavefront w in the result layout of the MFMA, element q of row
 // tile t = row 16 t + 4 q + l / 16, column 16 w + l % 16, which is also the
@@ -881,14 +858,15 @@ __device__ __forceinline__ void panel_to_lds(cplx* L, const Panel<TN>& P) {
     for (int q = 0; q < 4; ++q) L[panel_at<TN>(t, q)] = c_make(P.r[t][q], P.i[t][q]);
 }
 
-// Row tiles of A B for the wavefront's column panel: A in LDS, element (t,
-// q) of B from get(t, q, re, im); row tile i of the product to out(i, acc).
-template <int TN, class Get, class Out>
+// Row tiles of A B (ADJ: A^+ B) for the wavefront's column panel: A in LDS,
+// element (t, q) of B from get(t, q, re, im); row tile i of the product to
+// out(i, acc).
+template <int TN, bool ADJ = false, class Get, class Out>
 __device__ __forceinline__ void panel_product(const cplx* L, Get get, Out out) {
   const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
-  int off[4];
+  int off[4];  // A[l % 16][4 q + l / 16] of a tile, or (ADJ) A[4 q + l / 16][l % 16]
 #pragma unroll
-  for (int q = 0; q < 4; ++q) off[q] = lr * 16 + ((4 * q + lk) ^ lr);
+  for (int q = 0; q < 4; ++q) off[q] = ADJ ? (4 * q + lk) * 16 + (lr ^ (4 * q + lk)) : lr * 16 + ((4 * q + lk) ^ lr);
 #pragma unroll
   for (int i = 0; i < TN; ++i) {
     Cfrag<double> acc;
@@ -897,10 +875,10 @@ __device__ __forceinline__ void panel_product(const cplx* L, Get get, Out out) {
     for (int t = 0; t < TN; ++t) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const cplx a = L[(i * TN + t) * 256 + off[q]];
+        const cplx a = L[(ADJ ? t * TN + i : i * TN + t) * 256 + off[q]];
         double br, bi;
         get(t, q, br, bi);
-        acc.mma(a.x, a.y, br, bi);
+        acc.mma(a.x, ADJ ? -a.y : a.y, br, bi);
       }
       // no LDS reads of later tiles ahead of the products: their registers
       // would push the panels out
@@ -910,7 +888,7 @@ __device__ __forceinline__ void panel_product(const cplx* L, Get get, Out out) {
   }
 }
 
-// Retraction of one (problem, k) for num_wann <= 64: forms D (trial step),
+// Retraction of one (problem, k) for num_wann <= W90_PANEL_MAX: forms D (trial step),
 // X = scale D, E = exp(X) and U_new = U E, one wavefront per 16 columns, TN =
 // ceil(num_wann / 16) of them.  A wavefront's columns of X, X2 and the
 // product in hand stay in its registers; only the left factor of each
@@ -926,7 +904,8 @@ __device__ __forceinline__ void panel_product(const cplx* L, Get get, Out out) {
 // the search below.  Horner's form took a product per degree, 5 to 11 of
 // them, with both factors in LDS.  Measured on the same states, before -> now:
 // 16 bands, 512 k 9.9 -> 7.6 us; 27, 216 k 23.5 -> 12.9; 44, 343 k 53 -> 39;
-// 64, 800 k 180 -> 125.
+// 64, 800 k 180 -> 125; 91, 216 k 360 -> 168 (from k_step's form, all operands
+// in the caches).
 template <int TN>
 __global__ void __launch_bounds__(64 * TN, kStepWaves(TN)) k_step_panel(const Prob* probs, const Item* items,
                                                                        int nitems, int mode) {
@@ -1130,9 +1109,9 @@ __global__ void __launch_bounds__(64 * TN, kStepWaves(TN)) k_step_panel(const Pr
 // fragments loaded straight from memory (the matrices of one k stay in the
 // caches: A fragments read along a column, B fragments reuse cache lines
 // over consecutive K steps).  With ident, C = I + scale A B (one Taylor
-// step, applied as the product is stored).  Used by the retraction above
-// num_wann 64.
-__device__ void wg_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, double scale, bool ident) {
+// step, applied as the product is stored); with adj, A^+ for A.  Used above
+// num_wann 64 and by the one-time kernels.
+__device__ void wg_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, double scale, bool ident, bool adj) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nwv = blockDim.x >> 6;
   const int lr = lane & 15, lk = lane >> 4;
   const int nt = (n + 15) / 16;
@@ -1153,9 +1132,9 @@ __device__ void wg_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, doubl
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const int r = i0[u] + lr, c = j0[u] + lr;
-        const cplx a = (r < n && kk < n) ? A[r + (size_t)kk * n] : c_make(0.0, 0.0);
+        const cplx a = (r < n && kk < n) ? A[adj ? kk + (size_t)r * n : r + (size_t)kk * n] : c_make(0.0, 0.0);
         const cplx b = (kk < n && c < n) ? B[kk + (size_t)c * n] : c_make(0.0, 0.0);
-        cc[u].mma(a.x, a.y, b.x, b.y);
+        cc[u].mma(a.x, adj ? -a.y : a.y, b.x, b.y);
       }
     }
 #pragma unroll
@@ -1176,6 +1155,208 @@ __device__ void wg_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, doubl
     }
   }
   __syncthreads();
+}
+
+// ---------------------------------------------------------- projection
+
+// Lowdin orthonormalisation of overlap_project (src/overlap.F90:758-952)
+// for num_bands = num_wann: the unitary polar factor U = A (A^+ A)^-1/2 of
+// A(k) (staged in G), which is the Z V^+ built there from the SVD
+// A = Z S V^+.  Newton-Schulz iteration X <- X (3 - X^+ X)/2 from
+// X = A/||A||_F (all singular values in (0,1]) converges to it for
+// non-singular A, quadratically near the end: once X^+ X = 1 to 1e-12 one
+// more step reaches rounding level and the iteration stops (at most
+// kPolarSteps).  Writes U(k) to E.
+constexpr int kPolarSteps = 200;
+
+// Above 64 bands: matrices in global memory, one workgroup per k.
+__global__ void __launch_bounds__(W90_STEP_NT) k_polar(const Prob* probs, const Item* items, int nitems) {
+  if (blockIdx.x >= (unsigned)nitems) return;
+  const Item it = items[blockIdx.x];
+  const Prob& p = probs[it.prob];
+  const int nw = p.nw, nw2 = p.nw2;
+  const int k = it.k;
+  cplx* X = p.E + (size_t)k * nw2;
+  cplx* Y = p.W1 + (size_t)k * nw2;
+  cplx* Z = p.W2 + (size_t)k * nw2;
+  __shared__ double red[W90_NT];
+  const cplx* Ak = p.G + (size_t)k * nw2;
+  double fro = 0.0;
+  for (int e = threadIdx.x; e < nw2; e += blockDim.x) fro += c_abs2(Ak[e]);
+  fro = sqrt(block_sum(fro, red));
+  const double inv = (fro > 0.0 && isfinite(fro)) ? 1.0 / fro : 0.0;
+  for (int e = threadIdx.x; e < nw2; e += blockDim.x) X[e] = c_scale(Ak[e], inv);
+  __syncthreads();
+  for (int iter = 0; iter < kPolarSteps; ++iter) {
+    wg_gemm_mfma(Y, X, X, nw, 1.0, false, true);
+    double dev = 0.0;
+    bool bad = false;
+    for (int e = threadIdx.x; e < nw2; e += blockDim.x) {
+      cplx y = Y[e];
+      const bool diag = e % nw == e / nw;
+      const cplx d = c_make(y.x - (diag ? 1.0 : 0.0), y.y);
+      const double v = sqrt(c_abs2(d));
+      bad |= v != v;
+      dev = fmax(dev, v);
+      // 3 - X^+ X, halved below
+      Y[e] = c_make(-y.x + (diag ? 3.0 : 0.0), -y.y);
+    }
+    dev = block_max(dev, red);
+    if (__syncthreads_or(bad)) break;  // non-finite input: left to the unitarity check
+    wg_gemm_mfma(Z, X, Y, nw);
+    for (int e = threadIdx.x; e < nw2; e += blockDim.x) X[e] = c_scale(Z[e], 0.5);
+    __syncthreads();
+    if (dev < 1e-12) break;
+  }
+}
+
+// Up to 64 bands: X in LDS as the A operand and the panels of the products in
+// registers, as in k_step_panel.  32 bands, 216 k: 387 -> 54 us against
+// scalar products from global memory.
+template <int TN>
+__global__ void __launch_bounds__(64 * TN, kStepWaves(TN)) k_polar_panel(const Prob* probs, const Item* items,
+                                                                        int nitems) {
+  if (blockIdx.x >= (unsigned)nitems) return;
+  const Item it = items[blockIdx.x];
+  const Prob& p = probs[it.prob];
+  if ((p.nw + 15) / 16 != TN) return;
+  const int nw = p.nw, nw2 = p.nw2;
+  const int k = it.k, lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+  __shared__ cplx L[TN * TN * 256];
+  __shared__ double red[2 * TN];
+  const int col = 16 * w + lr;
+  const unsigned o = (unsigned)(col * nw + lk);
+  auto row_of = [&](int t, int q) { return 16 * t + 4 * q + lk; };
+  const cplx* Ak = p.G + (size_t)k * nw2;
+  Panel<TN> X, Y;
+  double fro = 0.0;
+#pragma unroll
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      cplx a = c_make(0.0, 0.0);
+      if (row_of(t, q) < nw && col < nw) a = Ak[o + 16 * t + 4 * q];
+      X.r[t][q] = a.x;
+      X.i[t][q] = a.y;
+      fro += c_abs2(a);
+    }
+  fro = wave_sum(fro);
+  if (lane == 0) red[w] = fro;
+  __syncthreads();
+  fro = 0.0;
+#pragma unroll
+  for (int v = 0; v < TN; ++v) fro += red[v];
+  fro = sqrt(fro);
+  const double inv = (fro > 0.0 && isfinite(fro)) ? 1.0 / fro : 0.0;
+#pragma unroll
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      X.r[t][q] *= inv;
+      X.i[t][q] *= inv;
+    }
+  for (int iter = 0; iter < kPolarSteps; ++iter) {
+    __syncthreads();
+    panel_to_lds<TN>(L, X);
+    __syncthreads();
+    // Y = (3 - X^+ X) / 2 and the largest |X^+ X - 1| (NaN kept: the sum below
+    // carries it)
+    double dev = 0.0, nan = 0.0;
+    panel_product<TN, true>(
+        L, [&](int t, int q, double& br, double& bi) { br = X.r[t][q]; bi = X.i[t][q]; },
+        [&](int i, const Cfrag<double>& acc) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const double one = row_of(i, q) == col && col < nw ? 1.0 : 0.0;
+            const double a = acc.re(q), b = acc.im(q);
+            const double v = sqrt((a - one) * (a - one) + b * b);
+            dev = fmax(dev, v);
+            nan += v - v;
+            Y.r[i][q] = 0.5 * (3.0 * one - a);
+            Y.i[i][q] = -0.5 * b;
+          }
+        });
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      dev = fmax(dev, __shfl_xor(dev, off, 64));
+      nan += __shfl_xor(nan, off, 64);
+    }
+    if (lane == 0) {
+      red[w] = dev;
+      red[TN + w] = nan;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < TN; ++v) {
+      dev = fmax(dev, red[v]);
+      nan += red[TN + v];
+    }
+    if (nan != nan) break;  // non-finite input: left to the unitarity check
+    panel_product<TN>(
+        L, [&](int t, int q, double& br, double& bi) { br = Y.r[t][q]; bi = Y.i[t][q]; },
+        [&](int i, const Cfrag<double>& acc) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            X.r[i][q] = acc.re(q);
+            X.i[i][q] = acc.im(q);
+          }
+        });
+    if (dev < 1e-12) break;
+  }
+  cplx* Ek = p.E + (size_t)k * nw2;
+#pragma unroll
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (row_of(t, q) < nw && col < nw) Ek[o + 16 * t + 4 * q] = c_make(X.r[t][q], X.i[t][q]);
+}
+
+// wann_check_unitarity (wannierise.F90:2594-2661): per-k maximum deviation
+// of U U^+ and U^+ U from the identity (NaN gives infinity).  Both are
+// Hermitian: a wavefront forms tiles of their upper triangles on FP64 MFMA,
+// operands from the caches (64 bands, 800 k: 875 -> 135 us against scalar
+// dot products of every element).
+__global__ void __launch_bounds__(W90_NT) k_unitarity(const Prob* probs, const Item* items, int nitems) {
+  if (blockIdx.x >= (unsigned)nitems) return;
+  const Item it = items[blockIdx.x];
+  const Prob& p = probs[it.prob];
+  const int n = p.nw;
+  const int k = it.k;
+  const cplx* U = p.U[p.st->cur] + (size_t)k * p.nw2;
+  __shared__ double red[W90_NT];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nwv = blockDim.x >> 6;
+  const int lr = lane & 15, lk = lane >> 4;
+  const int nt = (n + 15) / 16;
+  double dev = 0.0;
+  for (int x = w; x < nt * nt; x += nwv) {
+    const int ti = x % nt, tj = x / nt;
+    if (ti > tj) continue;
+    const int r = 16 * ti + lr, c = 16 * tj + lr;
+    Cfrag<double> c1, c2;
+    c1.zero();
+    c2.zero();
+    for (int ks = 0; ks < n; ks += 4) {
+      const int kk = ks + lk;
+      const bool vr = r < n && kk < n, vc = c < n && kk < n;
+      const cplx z = c_make(0.0, 0.0);
+      const cplx a1 = vr ? U[r + (size_t)kk * n] : z, b1 = vc ? U[c + (size_t)kk * n] : z;
+      const cplx a2 = vr ? U[kk + (size_t)r * n] : z, b2 = vc ? U[kk + (size_t)c * n] : z;
+      c1.mma(a1.x, a1.y, b1.x, -b1.y);
+      c2.mma(a2.x, -a2.y, b2.x, b2.y);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 16 * ti + Mfma<double>::row(lk, i);
+      if (row >= n || c >= n) continue;
+      const double one = row == c ? 1.0 : 0.0;
+      const double x1 = c1.re(i) - one, y1 = c1.im(i), x2 = c2.re(i) - one, y2 = c2.im(i);
+      const double v1 = sqrt(x1 * x1 + y1 * y1), v2 = sqrt(x2 * x2 + y2 * y2);
+      if (v1 != v1 || v2 != v2) dev = INFINITY;
+      dev = fmax(dev, fmax(v1, v2));
+    }
+  }
+  dev = block_max(dev, red);
+  if (threadIdx.x == 0) p.unit[k] = dev;
 }
 
 // ---------------------------------------------------------- small blocks
