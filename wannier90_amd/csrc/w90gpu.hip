@@ -147,7 +147,7 @@ int rot_panels(int rk, int nw) {
   return t * t;
 }
 static_assert(((W90GPU_MAX_WANN + 31) / 32) * ((W90GPU_MAX_WANN + 31) / 32) <= W90_MAX_PANELS,
-              "k_kpart stages every tile sum of a block");
+              "the tiles of a block");
 
 // partial-sum slots per block in a problem's arena: the most that any
 // candidate of its class writes
@@ -172,9 +172,9 @@ struct Lists {
   const Item* items = nullptr;
   const int* plist = nullptr;
   int np = 0;
+  int orange = 0, nrange = 0;  // the k-ranges of the omega reduction, in items behind the others
   Seg seg[kGroups][2];  // [group][0: FP64, 1: FP32]
   bool any_second = false;
-  bool any_group = false;  // some problem uses the two-level omega reduction
 };
 
 // Lists over n items of one group and precision (the segments before it
@@ -315,6 +315,15 @@ double now_s() {
 
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// k-ranges of a problem's omega reduction: ranges of 16 k and more up to 16
+// bands (one row of sums per k: a few loads), of 4 and more above (two values
+// per band and neighbour), so that the ranges of a mesh run on their own CUs
+// and the last workgroup still adds few rows.
+int omega_groups(int nw, int nk) {
+  const int per = wann_class(nw) == 0 ? 16 : 4, most = wann_class(nw) == 0 ? 32 : W90_MAX_GROUPS;
+  return nk <= 64 && wann_class(nw) == 0 ? 1 : std::max(1, std::min(most, nk / per));
+}
+
 // Arena of one problem: offsets in a fixed order that member_bind mirrors.
 struct Layout {
   size_t off[40];
@@ -333,7 +342,7 @@ size_t problem_layout(int nw, int nk, int nn, int num_iter, Layout& lay, bool pa
   const size_t mb = nw2 * nn * nk * sizeof(cplx);
   const size_t ub = nw2 * nk * sizeof(cplx);
   const size_t lnb = (size_t)nk * nn * nw * sizeof(double);
-  const size_t psz = 8 * (size_t)nw + 8;
+  const size_t psz = 8 * (size_t)nw + 2;
   lay.add(mb);   // M[0]
   lay.add(mb);   // M[1] (holds the two FP32 buffers of the mixed bulk phase)
   lay.add(mb);   // M0
@@ -351,8 +360,8 @@ size_t problem_layout(int nw, int nk, int nn, int num_iter, Layout& lay, bool pa
   lay.add(wann_class(nw) >= 3 ? mb : 256);                  // Tm (two-stage rotation scratch)
   lay.add((size_t)nk * nn * max_panels(nw) * sizeof(double));  // part_od
   lay.add((size_t)nk * nn * max_panels(nw) * sizeof(double));  // part_all
-  lay.add((size_t)nk * psz * sizeof(double));               // kpart
-  lay.add((size_t)W90_MAX_GROUPS * psz * sizeof(double));   // gpart
+  lay.add(wann_class(nw) == 0 ? (size_t)nk * psz * sizeof(double) : 0);  // kpart
+  lay.add((size_t)omega_groups(nw, nk) * psz * sizeof(double));         // gpart
   lay.add((size_t)nk * sizeof(double));                     // part_gg
   lay.add((size_t)nk * sizeof(double));                     // part_gd
   lay.add(3 * (size_t)nw * sizeof(double));                 // rave[0]
@@ -363,6 +372,7 @@ size_t problem_layout(int nw, int nk, int nn, int num_iter, Layout& lay, bool pa
   lay.add(4 * (size_t)(num_iter + 2) * sizeof(double));     // log
   lay.add(sizeof(State));                                   // state
   lay.add(sizeof(State));                                   // state template
+  lay.add(6 * sizeof(double) + sizeof(int));                // bsum, tick
   lay.add((size_t)nk * nn * sizeof(int));                   // nnl
   lay.add((size_t)nk * nn * 3 * sizeof(double));            // bk
   lay.add((size_t)nn * sizeof(double));                     // wb
@@ -563,13 +573,8 @@ void member_bind(Member* m, char* a, const Layout& lay) {
   p.nn = m->nn;
   p.nw2 = m->nw * m->nw;
   p.npan = rot_panels(m->rk, m->nw);
-  p.psz = 8 * m->nw + 8;
-  // two reduction levels only where one workgroup summing all per-k
-  // vectors would be slow (over 128 Ki values)
-  // meshes above 64 k-points reduce in two levels (32 k-ranges, then their
-  // sums): one workgroup alone reads the nk vectors at the bandwidth of one
-  // CU
-  p.ngroup = (m->nk <= 64) ? 0 : std::min(m->nk, W90_MAX_GROUPS);
+  p.psz = 8 * m->nw + 2;
+  p.ngroup = omega_groups(m->nw, m->nk);
   p.M[0] = (cplx*)(a + lay.off[i++]);
   p.M[1] = (cplx*)(a + lay.off[i++]);
   m->M0 = (cplx*)(a + lay.off[i++]);
@@ -607,6 +612,8 @@ void member_bind(Member* m, char* a, const Layout& lay) {
   p.st = (State*)(a + lay.off[i++]);
   m->st_init = (State*)(a + lay.off[i++]);
   p.st_init = m->st_init;
+  p.bsum = (const double*)(a + lay.off[i]);
+  p.tick = (int*)(a + lay.off[i++] + 6 * sizeof(double));
   p.nnl = (const int*)(a + lay.off[i++]);
   p.bk = (const double*)(a + lay.off[i++]);
   p.wb = (const double*)(a + lay.off[i++]);
@@ -617,6 +624,18 @@ void member_bind(Member* m, char* a, const Layout& lay) {
     p.mate = (const int*)(a + lay.off[i++]);
     m->pair_flag = (int*)(a + lay.off[i++]);
   }
+}
+
+// sum over k and b of wb b b^T (xx, yy, zz, xy, yz, zx), bk as [k][b][3].
+void b_matrix(int nk, int nn, const double* bk, const double* wb, double* b6) {
+  for (int u = 0; u < 6; ++u) b6[u] = 0.0;
+  for (int k = 0; k < nk; ++k)
+    for (int b = 0; b < nn; ++b) {
+      const double* v = bk + 3 * ((size_t)k * nn + b);
+      const double w = wb[b];
+      const double t[6] = {v[0] * v[0], v[1] * v[1], v[2] * v[2], v[0] * v[1], v[1] * v[2], v[2] * v[0]};
+      for (int u = 0; u < 6; ++u) b6[u] += w * t[u];
+    }
 }
 
 // Pairs of the k-mesh for the rotation by pairs: mate[k][b] = k' nn + b'
@@ -832,6 +851,9 @@ int engine_add(Engine* E, const w90gpu_problem* prob, const w90gpu_control* ctl,
   auto put = [&](const void* dst, const void* src, size_t n) { std::memcpy(img.data() + ((const char*)dst - t0), src, n); };
   put(m->p.st, &s, sizeof(State));
   put(m->st_init, &s, sizeof(State));
+  double b6[6];
+  b_matrix(m->nk, m->nn, prob->bk, prob->wb, b6);
+  put(m->p.bsum, b6, sizeof(b6));  // (the ticket behind it is zero)
   put(m->p.nnl, hn.data(), hn.size() * sizeof(int));
   put(m->p.bk, prob->bk, (size_t)m->nk * m->nn * 3 * sizeof(double));
   put(m->p.wb, prob->wb, (size_t)m->nn * sizeof(double));
@@ -907,11 +929,13 @@ void build_lists(const std::vector<Member*>& ms, F prec_of, std::vector<Item>& i
         }
         s.n = (int)items.size() - s.off;
       }
+  L.orange = (int)items.size();
   for (Member* m : ms) {
     plist.push_back(m->slot);
     if (!m->ctl.lfixstep) L.any_second = true;
-    if (m->p.ngroup > 0) L.any_group = true;
+    for (int g = 0; g < m->p.ngroup; ++g) items.push_back(Item{m->slot, g});
   }
+  L.nrange = (int)items.size() - L.orange;
   L.np = (int)plist.size();
 }
 
@@ -934,7 +958,7 @@ int upload_lists(Engine* E, const std::vector<Item>& items, const std::vector<in
 // bulk phase), as in the run lists.
 int aux_lists(Engine* E, const std::vector<Member*>& ms, Lists& L, bool by_phase = false) {
   int nitems = 0;
-  for (Member* m : ms) nitems += m->nk;
+  for (Member* m : ms) nitems += m->nk + m->p.ngroup;
   int rc = grow_tables(E, (int)E->slots.size(), nitems);
   if (rc) return rc;
   std::vector<Item> items;
@@ -1028,8 +1052,8 @@ void launch_rot_kernel(hipStream_t s, const Prob* P, const Item* it, const Seg& 
   }
 }
 
-// The rotation of M and the reduction of its diagonal into the per-k
-// partial sums of wann_omega, over every group and precision of the lists.
+// The rotation of M with its phases and sums of |M|^2, over every group and
+// precision of the lists.
 int launch_rotate(Engine* E, const Lists& L, int mode) {
   hipStream_t s = E->stream;
   const Prob* P = E->d_probs;
@@ -1042,25 +1066,13 @@ int launch_rotate(Engine* E, const Lists& L, int mode) {
       else launch_rot_kernel<float2>(s, P, it, sg, kGroupRot[g], mode);
       HIPCHK(E->ctx, hipGetLastError());
     }
-  // per-k partial vectors of the MFMA classes
-  const Seg gk = class_range(L, 1, kClasses - 1);
-  if (gk.n) {
-    hipLaunchKernelGGL(k_kpart, dim3(gk.n), dim3(W90_NT), 0, s, P, L.items + gk.off, gk.n, mode);
-    HIPCHK(E->ctx, hipGetLastError());
-  }
   return W90GPU_OK;
 }
 
-// The reduction of the per-k partial vectors over k, with the control
-// logic that follows each wann_omega.
+// The reduction of wann_omega over k, with the control logic that follows it.
 int launch_reduce(Engine* E, const Lists& L, int mode, int lean = 0) {
-  if (L.any_group) {
-    hipLaunchKernelGGL(k_omega_group, dim3(L.np * W90_MAX_GROUPS), dim3(W90_NT), 0, E->stream, E->d_probs,
-                       L.plist, L.np, mode);
-    HIPCHK(E->ctx, hipGetLastError());
-  }
-  hipLaunchKernelGGL(k_omega_final, dim3(L.np), dim3(W90_FINAL_NT), 0, E->stream, E->d_probs, L.plist, L.np, mode,
-                     lean);
+  hipLaunchKernelGGL(k_omega, dim3(L.nrange), dim3(W90_OMEGA_NT), 0, E->stream, E->d_probs, L.items + L.orange,
+                     L.nrange, mode, lean);
   HIPCHK(E->ctx, hipGetLastError());
   return W90GPU_OK;
 }
@@ -1358,7 +1370,7 @@ int build_run_lists(Engine* E) {
   for (Member* m : E->slots)
     if (m && m->stage == 2) {
       ms.push_back(m);
-      nitems += m->nk;
+      nitems += m->nk + m->p.ngroup;
     }
   int rc = grow_tables(E, (int)E->slots.size(), nitems);
   if (rc) return rc;
@@ -1638,12 +1650,14 @@ int scratch_address(int device, char** out) {
 }
 
 // Tables of the allocation-free path, built on the device: the work items
-// (problem 0, k), the problem list {0} and the neighbour table nnl[k][b]
+// (problem 0, k) and (problem 0, k-range), the problem list {0}, the ticket of
+// the omega reduction and the neighbour table nnl[k][b]
 // (0-based) from the caller's nnlist(nk, nn), 1-based, copied raw.
-__global__ void k_noalloc_tables(Item* items, int* plist, int* nnl, const int* nnlist_raw, int nk, int nn) {
+__global__ void k_noalloc_tables(Item* items, int* plist, int* nnl, int* tick, const int* nnlist_raw, int nk, int nn, int ngroup) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) plist[0] = 0;
+  if (i == 0) plist[0] = *tick = 0;
   if (i < nk) items[i] = Item{0, i};
+  if (i < ngroup) items[nk + i] = Item{0, i};
   if (i < nk * nn) {
     const int k = i / nn, b = i % nn;
     nnl[i] = nnlist_raw[k + (size_t)nk * b] - 1;
@@ -1660,7 +1674,7 @@ struct ScratchLayout {
 ScratchLayout scratch_layout(int nw, int nk, int nn, Layout& lay) {
   ScratchLayout s;
   s.items = align_up(sizeof(Prob));
-  s.plist = s.items + align_up(sizeof(Item) * (size_t)nk);
+  s.plist = s.items + align_up(sizeof(Item) * (size_t)(nk + omega_groups(nw, nk)));
   s.raw = s.plist + align_up(sizeof(int));
   s.arena = s.raw + align_up(sizeof(int) * (size_t)nk * nn);
   s.total = s.arena + problem_layout(nw, nk, nn, 0, lay, false);
@@ -2190,11 +2204,14 @@ int w90gpu_omega_noalloc(w90gpu_ctx* ctx, const w90gpu_problem* prob, const doub
   HIPCHK(ctx, hipMemcpy(raw, prob->nnlist, sizeof(int) * (size_t)nk * nn, hipMemcpyHostToDevice));
   HIPCHK(ctx, hipMemcpy((void*)m.p.bk, prob->bk, sizeof(double) * 3 * (size_t)nk * nn, hipMemcpyHostToDevice));
   HIPCHK(ctx, hipMemcpy((void*)m.p.wb, prob->wb, sizeof(double) * (size_t)nn, hipMemcpyHostToDevice));
+  double b6[6];
+  b_matrix(nk, nn, prob->bk, prob->wb, b6);
+  HIPCHK(ctx, hipMemcpy((void*)m.p.bsum, b6, sizeof(b6), hipMemcpyHostToDevice));
   HIPCHK(ctx, hipMemcpy(m.st_init, &st0, sizeof(State), hipMemcpyHostToDevice));
   HIPCHK(ctx, hipMemcpy(m.p.M[0], m_matrix, mb, hipMemcpyHostToDevice));
   const int nt = std::max(nk * nn, nk);
   hipLaunchKernelGGL(k_noalloc_tables, dim3((nt + 255) / 256), dim3(256), 0, nullptr, items, plist, (int*)m.p.nnl,
-                     raw, nk, nn);
+                     m.p.tick, raw, nk, nn, m.p.ngroup);
   HIPCHK(ctx, hipGetLastError());
   Engine E;
   E.ctx = ctx;
@@ -2207,7 +2224,8 @@ int w90gpu_omega_noalloc(w90gpu_ctx* ctx, const w90gpu_problem* prob, const doub
   // the segments build_lists gives a single member: empty before and after
   // its group, all nk items in (group, FP64)
   one_group_lists(L, group_of(m.cls, m.rk), 0, nk, nn, rot_panels(m.rk, nw), nw);
-  L.any_group = m.p.ngroup > 0;
+  L.orange = nk;
+  L.nrange = m.p.ngroup;
   hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, nullptr, E.d_probs, L.plist, 1);
   hipLaunchKernelGGL(k_zero, dim3((unsigned)std::min<size_t>(1024, (nd + 255) / 256)), dim3(256), 0, nullptr,
                      m.p.U[0], nd);

@@ -44,8 +44,8 @@ typedef double2 cplx;
 #define W90_NT 256          // threads per workgroup of the per-k kernels
 #define W90_STEP_NT 1024    // threads of the global-memory retraction (above W90_PANEL_MAX bands)
 #define W90_PANEL_MAX 96    // most bands whose matrix fits a workgroup's LDS (k_step_panel)
-#define W90_FINAL_NT 1024   // threads of the per-problem omega kernel
-#define W90_MAX_GROUPS 32   // k-ranges of the first omega reduction level
+#define W90_OMEGA_NT 512    // threads of the omega reduction
+#define W90_MAX_GROUPS 64   // most k-ranges (workgroups) of a problem's omega reduction
 #define W90_MIXED_RTOL 1e-8 // relative FP32 noise floor of Omega differences in the bulk phase
 #ifndef W90_BULK_STALLS
 #define W90_BULK_STALLS 2   // rejected bulk steps in a row that end the bulk phase
@@ -214,9 +214,8 @@ struct State {
 // Device view of one problem: sizes and pointers into its HBM arena.
 struct Prob {
   int nw, nk, nn, npan;
-  int psz, nw2, ngroup, want_et;  // psz: per-k partial vector length; ngroup: first-level k-ranges
-                                  // (0: the final reduction sums the per-k vectors itself);
-                                  // want_et: the rotation kernel reads ET
+  int psz, nw2, ngroup, want_et;  // psz: partial vector length; ngroup: k-ranges of the omega
+                                  // reduction; want_et: the rotation kernel reads ET
   // npan: tiles of the MFMA rotation per block M(k,b) (num_wann > 16)
   const int* nnl;     // [k][b] 0-based neighbour
   // FP64 rotation by pairs (see rot_pairs): npair blocks (k, b) per k are
@@ -245,8 +244,11 @@ struct Prob {
   double* part_od;    // [k][b][tile] (MFMA path)
   double* part_all;   // [k][b][tile] (MFMA path)
   void* Tm;           // [k][b][nw*nw] E_k^+ M(k,b) of the MFMA path, storage precision
-  double* kpart;      // [k][psz] per-k partial sums of wann_omega (DiagAcc layout)
+  double* kpart;      // [k][psz] per-k partial sums of wann_omega (DiagAcc layout; up to 16 bands,
+                      // written by the rotation)
   double* gpart;      // [ngroup][psz] sums over contiguous k-ranges
+  const double* bsum; // [6] sum over k and b of wb b b^T (xx, yy, zz, xy, yz, zx)
+  int* tick;          // workgroups of the omega reduction that have stored their range
   double* part_gg;    // [k]
   double* part_gd;    // [k]
   double* rave[2];    // [3][nw] per buffer (Fortran rave(3,nw): ind fastest)
@@ -441,9 +443,8 @@ __global__ void __launch_bounds__(W90_NT) k_gather_final(const Prob* probs, cons
 // and the scalars
 //   [8*nw + 0]     S_od      = sum_b wb sum_{m!=n} |M_mn|^2
 //   [8*nw + 1]     S_i       = sum_b wb (nw - sum_mn |M_mn|^2)
-//   [8*nw + 2..7]  B         = sum_b wb b b^T  (xx, yy, zz, xy, yz, zx)
 // with ln_n = Im ln M_nn and r0 the centres of the source buffer.  With
-// d = rave - r0, Omega_D = (1/nk) sum_n [A + 2 d.V + d^T B d] is exact
+// d = rave - r0 and B = sum_b wb b b^T, Omega_D = (1/nk) sum_n [A + 2 d.V + d^T B d] is exact
 // algebra for (1/nk) sum wb (ln + b.rave)^2 (wannierise.F90:2260-2275), and
 // r0 close to rave keeps it free of cancellation, so no second pass over ln
 // is needed once rave is known.
@@ -473,23 +474,6 @@ __device__ __forceinline__ void diag_store(double* out, int nw, int n, const Dia
   out[5 * nw + n] = d.v[0];
   out[6 * nw + n] = d.v[1];
   out[7 * nw + n] = d.v[2];
-}
-
-// Scalars of the per-k vector that depend only on the k-mesh: B = sum wb b b^T
-// from the weights wb[b] and the vectors bk[3 b + i] of the k.
-__device__ void kpart_bmat(const double* wb, const double* bk, int nn, double* out) {
-  double b6[6] = {0, 0, 0, 0, 0, 0};
-  for (int b = 0; b < nn; ++b) {
-    const double w = wb[b];
-    const double* bv = bk + b * 3;
-    b6[0] += w * bv[0] * bv[0];
-    b6[1] += w * bv[1] * bv[1];
-    b6[2] += w * bv[2] * bv[2];
-    b6[3] += w * bv[0] * bv[1];
-    b6[4] += w * bv[1] * bv[2];
-    b6[5] += w * bv[2] * bv[0];
-  }
-  for (int u = 0; u < 6; ++u) out[2 + u] = b6[u];
 }
 
 // The weights wb and the vectors bk(:,:,k) of one k staged in LDS by
@@ -602,70 +586,6 @@ __global__ void __launch_bounds__(W90_NT) k_check_pairs(Prob p, int npair, int* 
 // Tiles per block M(k,b) of the MFMA rotation at most: 32 x 32 panels over
 // 256 bands.
 #define W90_MAX_PANELS 64
-static_assert(W90GPU_MAX_WANN <= W90_NT, "k_kpart: one thread per Wannier function");
-
-// Per-k partial vector from the per-tile outputs of the MFMA rotation
-// (num_wann above the LDS kernels): diagonal phases and |M_nn|^2, and the
-// tile sums of |M_mn|^2.
-__global__ void __launch_bounds__(W90_NT) k_kpart(const Prob* probs, const Item* items, int nitems, int mode) {
-  if (blockIdx.x >= (unsigned)nitems) return;
-  const Item it = items[blockIdx.x];
-  const Prob& p = probs[it.prob];
-  const State* st = p.st;
-  const int cur = gate_cur(st, mode);
-  if (cur < 0) return;
-  const int nw = p.nw, nn = p.nn;
-  const int k = it.k;
-  const int dst = dst_buf(mode, cur);
-  const double* ln = p.ln[dst];
-  double* out = p.kpart + (size_t)k * p.psz;
-  const int npan = p.npan;
-  // every input of the k is loaded in one round: the mesh tables and the
-  // tile sums into LDS, the diagonal phases and moduli into registers
-  __shared__ double wbL[W90GPU_NUM_NNMAX], bkL[3 * W90GPU_NUM_NNMAX];
-  __shared__ double podL[W90GPU_NUM_NNMAX * W90_MAX_PANELS], pallL[W90GPU_NUM_NNMAX * W90_MAX_PANELS];
-  kmesh_stage(p, k, wbL, bkL);
-  for (int t = threadIdx.x; t < nn * npan; t += blockDim.x) {
-    podL[t] = p.part_od[(size_t)k * nn * npan + t];
-    pallL[t] = p.part_all[(size_t)k * nn * npan + t];
-  }
-  double lnv[W90GPU_NUM_NNMAX], d2v[W90GPU_NUM_NNMAX], r0[3];
-  const int n0 = threadIdx.x;
-  if (n0 < nw) {
-    ref_centre(p, mode, cur, n0, r0);
-#pragma unroll
-    for (int b = 0; b < W90GPU_NUM_NNMAX; ++b) {
-      if (b < nn) {
-        const size_t kb = (size_t)k * nn + b;
-        lnv[b] = ln[kb * nw + n0];
-        d2v[b] = p.d2[kb * nw + n0];
-      }
-    }
-  }
-  __syncthreads();
-  if (n0 < nw) {
-    DiagAcc d = {};
-#pragma unroll
-    for (int b = 0; b < W90GPU_NUM_NNMAX; ++b)
-      if (b < nn) diag_add(d, wbL[b], bkL + b * 3, lnv[b], d2v[b], r0[0], r0[1], r0[2]);
-    diag_store(out, nw, n0, d);
-  }
-  if (threadIdx.x == 0) {
-    double sod = 0.0, si = 0.0;
-    for (int b = 0; b < nn; ++b) {
-      double od = 0.0, al = 0.0;
-      for (int q = 0; q < npan; ++q) {
-        od += podL[b * npan + q];
-        al += pallL[b * npan + q];
-      }
-      sod += wbL[b] * od;
-      si += wbL[b] * ((double)nw - al);
-    }
-    out[8 * nw + 0] = sod;
-    out[8 * nw + 1] = si;
-    kpart_bmat(wbL, bkL, nn, out + 8 * nw);
-  }
-}
 
 // ---------------------------------------------------------- omega / control
 
@@ -733,38 +653,6 @@ __device__ void accept_step(State* st, const Spread& sp, int dst, double* logrow
   conv_step(st, logrow, st->gcnorm1);
 }
 
-// First level of the omega reduction: workgroup (problem, g) sums the per-k
-// vectors of a contiguous k-range, in k order (rows read coalesced, 16 rows
-// loaded at once and then added in order).
-__global__ void __launch_bounds__(W90_NT) k_omega_group(const Prob* probs, const int* plist, int np, int mode) {
-  const int pi = blockIdx.x / W90_MAX_GROUPS;
-  const int g = blockIdx.x % W90_MAX_GROUPS;
-  if (pi >= np) return;
-  const Prob& p = probs[plist[pi]];
-  if (g >= p.ngroup || !gate(p.st, mode)) return;
-  const int G = p.ngroup, psz = p.psz;
-  const int k0 = (int)(((long)g * p.nk) / G), k1 = (int)(((long)(g + 1) * p.nk) / G);
-  for (int v = threadIdx.x; v < psz; v += blockDim.x) {
-    double s = 0.0;
-    // chunks of 16 rows: the loads of a chunk are issued together (rows
-    // past k1 read as zero), then added in row order
-    for (int k = k0; k < k1; k += 16) {
-      double x[16];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) x[u] = (k + u < k1) ? p.kpart[(size_t)(k + u) * psz + v] : 0.0;
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (k + u < k1) s += x[u];
-    }
-    p.gpart[(size_t)g * psz + v] = s;
-  }
-}
-
-// Final reduction of wann_omega (one workgroup per problem) fused with the
-// control logic that follows each wann_omega call in wann_main: initial
-// state (:452-470), internal_optimal_step (:1528-1596) after the trial step
-// and the acceptance of the trial or parabolic step (:660-701).  MODE_REMIX
-// installs the FP64 rebuild of M at the end of the mixed bulk phase.
 // Control logic of wann_main after a wann_omega evaluation, run by one
 // thread on the workgroup's copy of the state: the initial state
 // (:452-470), internal_optimal_step (:1528-1596) after the trial step, the
@@ -873,104 +761,254 @@ __device__ void omega_control(State* st, const Prob& p, double sod, double si, d
   accept_step(st, sp, dst, logrow);
 }
 
-__global__ void __launch_bounds__(W90_FINAL_NT) k_omega_final(const Prob* probs, const int* plist, int np,
-                                                              int mode, int lean) {
-  if (blockIdx.x >= (unsigned)np) return;
-  const Prob& p = probs[plist[blockIdx.x]];
-  // the state is worked on in LDS: the control logic below is a chain of
-  // dependent reads and writes that would each pay a global-memory latency.
-  // Its words are requested first and stored to LDS after the row sums
-  // below have issued their loads, so the two rounds of loads overlap (the
-  // sums of a problem that the gate then skips are not used).
-  __shared__ State sst;
-  static_assert(sizeof(State) % sizeof(double) == 0, "State is copied as doubles");
-  constexpr int NSD = sizeof(State) / sizeof(double);
-  static_assert(NSD <= W90_FINAL_NT, "one state word per thread");
-  const int tid = threadIdx.x;
-  const double sword = tid < NSD ? reinterpret_cast<const double*>(p.st)[tid] : 0.0;
-  const int nw = p.nw, nk = p.nk, psz = p.psz;
-  const double rnk = (double)nk;
-  __shared__ double red[W90_FINAL_NT];
-  __shared__ double sums[8 * W90GPU_MAX_WANN + 8];
-  __shared__ double sc[8];
+struct OmegaLds {
+  double red[2 * W90_OMEGA_NT / 64];
+  double sums[8 * W90GPU_MAX_WANN + 2];
+  double slot[4 * W90_OMEGA_NT];
+  double bk[32 * 3 * W90GPU_NUM_NNMAX];
+  double wb[W90GPU_NUM_NNMAX];
+  int last;
+};
+__device__ __forceinline__ int pow2_up(int x) {
+  int r = 1;
+  while (r < x) r <<= 1;
+  return r;
+}
 
-  // sum of the group vectors (or, for problems without the group level,
-  // of the per-k vectors): VB values per pass (coalesced along a row), J
-  // lanes over rows, lanes combined in fixed order
-  const int VB = min(psz, W90_FINAL_NT);
-  const int J = W90_FINAL_NT / VB;
-  const int G = p.ngroup > 0 ? p.ngroup : nk;
-  const double* rows = p.ngroup > 0 ? p.gpart : p.kpart;
-  for (int v0 = 0; v0 < psz; v0 += VB) {
+// Partial vector of the k-range [k0, k1) from the per-(k, b) outputs of the
+// rotations above 16 bands (diagonal phases and moduli, tile sums of |M|^2)
+// into S.sums.  A thread takes one Wannier function and every slots-th k of
+// the range (slots of LW lanes), its sums run over b and those k in order,
+// and the slots are added in order.  The b-vectors and the tile sums of a
+// chunk of 32 k are requested with the first phases.
+__device__ void omega_range(const Prob& p, int cur, int dst, const double* r0, int k0, int k1, OmegaLds& S) {
+  const int tid = threadIdx.x, nw = p.nw, nn = p.nn, npan = p.npan;
+  const int LW = pow2_up(nw), slots = W90_OMEGA_NT / LW, n = tid & (LW - 1), sl = tid / LW;
+  const double* ln = p.ln[dst];
+  const double wbt = tid < nn ? p.wb[tid] : 0.0;
+  DiagAcc d = {};
+  double od = 0.0, si = 0.0;
+  double lnv[W90GPU_NUM_NNMAX], d2v[W90GPU_NUM_NNMAX];
+  auto phases = [&](int k) {
+#pragma unroll
+    for (int b = 0; b < W90GPU_NUM_NNMAX; ++b)
+      if (b < nn) {
+        const size_t kb = (size_t)k * nn + b;
+        lnv[b] = ln[kb * nw + n];
+        d2v[b] = p.d2[kb * nw + n];
+      }
+  };
+  for (int c0 = k0; c0 < k1; c0 += 32) {
+    const int c1 = min(k1, c0 + 32), nkb = (c1 - c0) * nn;
+    const bool mine = n < nw && c0 + sl < c1;
+    if (mine) phases(c0 + sl);
+    constexpr int BKS = (32 * 3 * W90GPU_NUM_NNMAX + W90_OMEGA_NT - 1) / W90_OMEGA_NT;
+    double bv[BKS];
+#pragma unroll
+    for (int i = 0; i < BKS; ++i) {
+      const int t = tid + i * W90_OMEGA_NT;
+      bv[i] = t < 3 * nkb ? p.bk[(size_t)c0 * nn * 3 + t] : 0.0;
+    }
+    static_assert(32 * W90GPU_NUM_NNMAX <= W90_OMEGA_NT, "one (k, b) of a chunk per thread");
+    double o = 0.0, a = 0.0;
+    if (tid < nkb) {
+      const double* po = p.part_od + ((size_t)c0 * nn + tid) * npan;
+      const double* pa = p.part_all + ((size_t)c0 * nn + tid) * npan;
+      for (int q = 0; q < npan; ++q) {
+        o += po[q];
+        a += pa[q];
+      }
+    }
+    if (c0 > k0) __syncthreads();  // the last chunk's b-vectors are used
+    if (tid < nn) S.wb[tid] = wbt;
+#pragma unroll
+    for (int i = 0; i < BKS; ++i) {
+      const int t = tid + i * W90_OMEGA_NT;
+      if (t < 3 * nkb) S.bk[t] = bv[i];
+    }
+    __syncthreads();
+    if (tid < nkb) {
+      const double w = S.wb[tid % nn];
+      od += w * o;
+      si += w * ((double)nw - a);
+    }
+    if (mine)
+      for (int k = c0 + sl;;) {
+#pragma unroll
+        for (int b = 0; b < W90GPU_NUM_NNMAX; ++b)
+          if (b < nn) diag_add(d, S.wb[b], S.bk + ((k - c0) * nn + b) * 3, lnv[b], d2v[b], r0[0], r0[1], r0[2]);
+        k += slots;
+        if (k >= c1) break;
+        phases(k);
+      }
+  }
+  block_sum2(od, si, S.red);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {  // four of the eight sums at a time
+    if (h) __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      S.slot[u * W90_OMEGA_NT + tid] = h ? (u == 0 ? d.a : d.v[u > 0 ? u - 1 : 0]) : (u < 3 ? d.r[u < 3 ? u : 0] : d.r2);
+    __syncthreads();
+    for (int v = tid; v < 4 * nw; v += W90_OMEGA_NT) {
+      const int u = v / nw, m = v % nw;
+      double t = 0.0;
+      for (int q = 0; q < slots; ++q) t += S.slot[u * W90_OMEGA_NT + q * LW + m];
+      S.sums[4 * h * nw + v] = t;
+    }
+  }
+  if (tid == 0) {
+    S.sums[8 * nw] = od;
+    S.sums[8 * nw + 1] = si;
+  }
+  __syncthreads();
+}
+
+// Sum of rows r0 .. r1 of 8 nw + 2 values (contiguous) into S.sums: the 8 nw
+// values VB per pass (coalesced along a row), J lanes over rows, lanes
+// combined in fixed order, while the last wavefront adds the two scalars.
+__device__ void omega_rows(const double* rows, int r0, int r1, int nw, OmegaLds& S) {
+  const int tid = threadIdx.x, psz = 8 * nw + 2, n8 = 8 * nw;
+  double s0 = 0.0, s1 = 0.0;
+  if (tid >= W90_OMEGA_NT - 64)
+    for (int g = r0 + (tid & 63); g < r1; g += 64) {
+      s0 += rows[(size_t)g * psz + n8];
+      s1 += rows[(size_t)g * psz + n8 + 1];
+    }
+  const int VB = min(n8, W90_OMEGA_NT);
+  const int J = W90_OMEGA_NT / VB;
+  for (int v0 = 0; v0 < n8; v0 += VB) {
     const int v = v0 + tid % VB;
     const int j = tid / VB;
     double s = 0.0;
-    if (j < J && v < psz) {
-      // rows j, j+J, ...: eight independent partial sums, combined in a
-      // fixed order; four rounds of eight rows are loaded at once (32 loads
-      // in flight) and added round by round, the same order as one round
-      // at a time
+    if (j < J && v < n8) {
+      // rows j, j + J, ...: eight independent partial sums, combined in a
+      // fixed order; 32 rows are loaded at once
       double a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      int g = j;
-      for (; g + 31 * J < G; g += 32 * J) {
+      int g = r0 + j;
+      for (; g + 31 * J < r1; g += 32 * J) {
         double x[32];
 #pragma unroll
         for (int u = 0; u < 32; ++u) x[u] = rows[(size_t)(g + u * J) * psz + v];
 #pragma unroll
         for (int u = 0; u < 32; ++u) a[u % 8] += x[u];
       }
-      for (; g + 7 * J < G; g += 8 * J) {
+      for (; g + 7 * J < r1; g += 8 * J) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) a[u] += rows[(size_t)(g + u * J) * psz + v];
       }
-      for (int u = 0; g < G; g += J, ++u) a[u] += rows[(size_t)g * psz + v];
+#pragma unroll
+      for (int u = 0; u < 7; ++u)
+        if (g + u * J < r1) a[u] += rows[(size_t)(g + u * J) * psz + v];
       s = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
     }
-    red[tid] = s;
+    S.slot[tid] = s;
     __syncthreads();
-    if (tid < VB && v0 + tid < psz) {
+    if (tid < VB && v0 + tid < n8) {
       double t = 0.0;
-      for (int jj = 0; jj < J; ++jj) t += red[tid + jj * VB];
-      sums[v0 + tid] = t;
+      for (int jj = 0; jj < J; ++jj) t += S.slot[tid + jj * VB];
+      S.sums[v0 + tid] = t;
     }
     __syncthreads();
   }
-  if (tid < NSD) reinterpret_cast<double*>(&sst)[tid] = sword;
+  if (tid >= W90_OMEGA_NT - 64) {
+    s0 = wave_sum(s0);
+    s1 = wave_sum(s1);
+    if (tid == W90_OMEGA_NT - 64) {
+      S.sums[n8] = s0;
+      S.sums[n8 + 1] = s1;
+    }
+  }
   __syncthreads();
-  State* st = &sst;
-  const int cur = gate_cur(st, mode);
-  if (cur < 0) return;
-  const int dst = dst_buf(mode, cur);
+}
 
+// The reduction of wann_omega over k, in one launch: workgroup (problem, g)
+// sums the k-range g and stores its vector; the last of a problem's workgroups
+// to arrive (an atomic ticket) adds the ranges, forms the centres and Omega
+// and runs the control logic that follows each wann_omega call in wann_main:
+// initial state (:452-470), internal_optimal_step (:1528-1596) after the trial
+// step and the acceptance of the trial or parabolic step (:660-701).
+// MODE_REMIX installs the FP64 rebuild of M at the end of the mixed bulk
+// phase.  No workgroup waits for another; the ranges are added in their order
+// whichever workgroup does it, so the result does not depend on the arrival.
+// The stored range is released to the device before the ticket is taken and
+// the last workgroup acquires before it reads (the fences of the two sides).
+//
+// It is bound by a chain of memory latencies (problem, state, phases, ticket,
+// rows), not by its few megabytes.  Three dependent launches (a vector per k
+// above 16 bands, the sums over k-ranges, the final sum with the control) paid
+// the chain three times: 64 bands, 800 k 34.5 -> 24.4 us with the launch gaps;
+// 27 bands, 216 k 24.7 -> 16.2; 16 bands, 512 k 13.1 -> 11.0.  1024 threads
+// spill (38 us at 64 bands); relaxed device-scope loads and stores in place of
+// the two fences gain 0.5 us.
+__global__ void __launch_bounds__(W90_OMEGA_NT) k_omega(const Prob* probs, const Item* ranges, int nranges, int mode,
+                                                        int lean) {
+  if (blockIdx.x >= (unsigned)nranges) return;
+  const Item it = ranges[blockIdx.x];
+  const Prob& p = probs[it.prob];
+  __shared__ OmegaLds S;
+  // the state is worked on in LDS: the control logic below is a chain of
+  // dependent reads and writes that would each pay a global-memory latency
+  __shared__ State sst;
+  static_assert(sizeof(State) % sizeof(double) == 0, "State is copied as doubles");
+  constexpr int NSD = sizeof(State) / sizeof(double);
+  static_assert(NSD <= W90_OMEGA_NT, "one state word per thread");
+  const int tid = threadIdx.x, g = it.k, G = p.ngroup;
+  const double sword = tid < NSD ? reinterpret_cast<const double*>(p.st)[tid] : 0.0;
+  const int cur = gate_cur(p.st, mode);
+  if (cur < 0) return;
+  const int nw = p.nw, nk = p.nk, psz = p.psz;
+  const double rnk = (double)nk;
+  const int dst = dst_buf(mode, cur);
+  const int k0 = (int)(((long)g * nk) / G), k1 = (int)(((long)(g + 1) * nk) / G);
+  // reference centres of this thread's Wannier function, here (tid) and in
+  // omega_range (tid mod a power of two: the same for tid < num_wann); read
+  // before rave[dst] is written (dst == cur for the rebuild)
+  double r0[3] = {0.0, 0.0, 0.0};
+  const int n0 = tid & (pow2_up(nw) - 1);
+  if (n0 < nw) ref_centre(p, mode, cur, n0, r0);
+  if (nw <= 16) omega_rows(p.kpart, k0, k1, nw, S);
+  else omega_range(p, cur, dst, r0, k0, k1, S);
+  if (G > 1) {
+    for (int v = tid; v < psz; v += W90_OMEGA_NT) p.gpart[(size_t)g * psz + v] = S.sums[v];
+    // every wavefront's stores have completed before the barrier, and one
+    // fence on each side of the ticket releases and acquires them
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      __threadfence();
+      S.last = __hip_atomic_fetch_add(p.tick, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == G - 1;
+      __threadfence();
+    }
+    __syncthreads();
+    if (!S.last) return;
+    if (tid == 0) __hip_atomic_store(p.tick, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    omega_rows(p.gpart, 0, G, nw, S);
+  }
+  if (tid < NSD) reinterpret_cast<double*>(&sst)[tid] = sword;
+  State* st = &sst;
+  const double* sums = S.sums;
   double omd_n = 0.0;
-  for (int n = tid; n < nw; n += blockDim.x) {
+  if (tid < nw) {
+    const int n = tid;
     double q[8];
     for (int u = 0; u < 8; ++u) q[u] = sums[u * nw + n];
-    double bb[6];
-    for (int u = 0; u < 6; ++u) bb[u] = sums[8 * nw + 2 + u];
-    // reference centres are read before rave[dst] is written (dst == cur
-    // for the rebuild)
-    double r0[3];
-    ref_centre(p, mode, cur, n, r0);
+    const double* bb = p.bsum;
     const double rx = -q[0] / rnk, ry = -q[1] / rnk, rz = -q[2] / rnk;
+    const double dx = rx - r0[0], dy = ry - r0[1], dz = rz - r0[2];
+    const double dbd = bb[0] * dx * dx + bb[1] * dy * dy + bb[2] * dz * dz +
+                       2.0 * (bb[3] * dx * dy + bb[4] * dy * dz + bb[5] * dz * dx);
+    omd_n = q[4] + 2.0 * (dx * q[5] + dy * q[6] + dz * q[7]) + dbd;
     p.rave[dst][0 + 3 * n] = rx;
     p.rave[dst][1 + 3 * n] = ry;
     p.rave[dst][2 + 3 * n] = rz;
     p.r2ave[dst][n] = q[3] / rnk;
-    const double dx = rx - r0[0], dy = ry - r0[1], dz = rz - r0[2];
-    const double dbd = bb[0] * dx * dx + bb[1] * dy * dy + bb[2] * dz * dz +
-                       2.0 * (bb[3] * dx * dy + bb[4] * dy * dz + bb[5] * dz * dx);
-    omd_n += q[4] + 2.0 * (dx * q[5] + dy * q[6] + dz * q[7]) + dbd;
   }
+  static_assert(W90GPU_MAX_WANN <= W90_OMEGA_NT, "one thread per Wannier function");
   // Omega_D summed over n in a fixed tree
-  const double omd = block_sum(omd_n, red);
-  if (threadIdx.x == 0) {
-    sc[0] = sums[8 * nw + 0];
-    sc[1] = sums[8 * nw + 1];
-  }
-  __syncthreads();
+  const double omd = block_sum(omd_n, S.red);
   if (mode == MODE_BENCH) return;  // timing of the reduction alone: the state stays as it is
-  if (threadIdx.x == 0) omega_control(st, p, sc[0], sc[1], omd, mode, dst, lean);
+  if (threadIdx.x == 0) omega_control(st, p, sums[8 * nw], sums[8 * nw + 1], omd, mode, dst, lean);
   __syncthreads();
   for (int i = threadIdx.x; i < NSD; i += blockDim.x)
     reinterpret_cast<double*>(p.st)[i] = reinterpret_cast<const double*>(&sst)[i];

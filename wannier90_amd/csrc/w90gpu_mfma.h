@@ -1542,6 +1542,5 @@ __global__ void __launch_bounds__(64 * W90GPU_NUM_NNMAX) k_rotate_w16(const Prob
     }
     outk[8 * nw + 0] = sod;
     outk[8 * nw + 1] = (double)nw * wsum - sall;
-    kpart_bmat(wbL, bkL, nn, outk + 8 * nw);
   }
 }
