@@ -310,8 +310,11 @@ def main():
     launches = 200 if prob.num_wann <= 32 else 20
     avg_ms = sess.rotation_time(launches)
     nk, nn, nw = prob.num_kpts, prob.kmesh.nntot, prob.num_wann
-    rot_bytes = (16.0 if prec == capi.PREC_FP64 else 8.0) * nk * nw * nw * (2 * nn + 1)  # M read + write, E once
-    rot_flops = 16.0 * nk * nn * nw ** 3               # two complex GEMMs per (k,b)
+    # generated overlaps hold M(k+b,-b) = M(k,b)^+: in FP64 above 16 bands one
+    # block of each pair is read and formed, and both are written
+    formed = nn // 2 if prec == capi.PREC_FP64 and nw > 16 else nn
+    rot_bytes = (16.0 if prec == capi.PREC_FP64 else 8.0) * nk * nw * nw * (formed + nn + 1)  # M read + write, E once
+    rot_flops = 16.0 * nk * formed * nw ** 3           # two complex GEMMs per block formed
     ai = rot_flops / rot_bytes
     peak_flops = FP64_PEAK_TFLOPS if prec == capi.PREC_FP64 else FP32_PEAK_TFLOPS
     ridge = peak_flops * 1e12 / (HBM_PEAK_GBS * 1e9)
@@ -323,8 +326,8 @@ def main():
         achieved = rot_flops / (avg_ms * 1e-3) / 1e12
         roof = dict(bound="mfma", achieved=achieved, peak=peak_flops, unit="TFLOP/s",
                     frac=achieved / peak_flops, traffic=None)
-    kname = ("k_rotate_w16" if nw <= 16 else "k_rot_fused + k_kpart" if nw <= 64
-             else "k_rot_gemm stage 1 + stage 2 + k_kpart")
+    kname = ("k_rotate_w16" if nw <= 16 else "k_rot_panel" if nw <= 48 and prec == capi.PREC_FP64
+             else "k_rot_fused" if nw <= 64 else "k_rot_gemm stage 1 + stage 2")
     roof.update(kernel=kname, avg_launch_ms=avg_ms, launches=launches,
                 algorithmic_bytes=rot_bytes, algorithmic_flops=rot_flops)
     roof["traffic"] = measured_traffic(args.config, args.precision)

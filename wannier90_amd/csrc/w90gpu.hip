@@ -101,7 +101,8 @@ int wann_class(int nw) { return nw <= 16 ? 0 : nw <= kLdsMaxWann ? 1 : nw <= W90
 //           panels: less padding for 65-96 bands, lower reuse per load)
 // The choice is made per (num_wann, nntot) by the autotuner (rot_choice,
 // tune_member) and fixed for the life of the process, so a problem is
-// rotated by the same kernel alone and in a batch.
+// rotated by the same kernel alone and in a batch.  Up to W90_ROT_PANEL_MAX
+// bands it is the choice for the FP32 phase: the FP64 rotation is k_rot_panel.
 enum RotKernel { RK_W16 = 0, RK_FUSED32, RK_FUSED64, RK_DIRECT64, RK_GEMM64, RK_GEMM32, RK_FUSED48, kRotKernels };
 const char* const kRotName[kRotKernels] = {"w16", "fused32", "fused64", "direct64", "gemm64", "gemm32", "fused48"};
 // output tile edge (the initial reduction k_reduce_tiles uses the same tiles)
@@ -139,10 +140,11 @@ int last_group(int cls) {
   return g;
 }
 
-// Tiles per block M(k,b) of a rotation kernel: the per-(k,b) partial sums
-// of its epilogue.
+// Partial sums per block M(k,b) that a problem's FP64 rotation leaves: its
+// tiles or column panels (the FP32 kernels up to 64 bands fill the first).
 int rot_panels(int rk, int nw) {
   if (rk == RK_W16) return 1;
+  if (nw <= W90_ROT_PANEL_MAX) return (nw + 15) / 16;  // one per wavefront of k_rot_panel
   const int t = (nw + kRotEdge[rk] - 1) / kRotEdge[rk];
   return t * t;
 }
@@ -767,6 +769,13 @@ void tune_refresh() {
   }
 }
 
+// The table's choice, or the class default.
+int table_rot(int nw, int nn) {
+  for (const TuneRow& r : kTuneTable)
+    if (nw >= r.nw_lo && nw <= r.nw_hi && nn >= r.nn_lo && nn <= r.nn_hi && rot_serves(r.rk, nw)) return r.rk;
+  return default_rot(wann_class(nw));
+}
+
 // The rotation kernel of a problem.  *pending (when given) is set if the
 // key is to be measured at the start of its first solve; until then the
 // class default stands.
@@ -782,9 +791,7 @@ int rot_choice(int nw, int nn, bool* pending) {
     if (pending && first_group(c) != last_group(c)) *pending = true;
     return default_rot(c);
   }
-  for (const TuneRow& r : kTuneTable)
-    if (nw >= r.nw_lo && nw <= r.nw_hi && nn >= r.nn_lo && nn <= r.nn_hi && rot_serves(r.rk, nw)) return r.rk;
-  return default_rot(c);
+  return table_rot(nw, nn);
 }
 
 // Admit a problem: pool bytes, a slot, its k-mesh tables and state template.
@@ -1007,13 +1014,19 @@ Seg class_prec_range(const Lists& L, int c, int q) {
   return r;
 }
 
+// Workgroups that k_rot_panel keeps when it takes several blocks of a k each:
+// four times what runs at once.  1024 to 4096 measure the same within 1%.
+constexpr int kRotGroups = 2048;
+
 // One rotation kernel over a segment of items in storage precision T2; for
 // MODE_INIT the tile reduction of the current M with the kernel's tiles.
 template <class T2>
 void launch_rot_kernel(hipStream_t s, const Prob* P, const Item* it, const Seg& g, int rk, int mode) {
   // MFMA GEMM tiles; gridDim.y covers b and the tiles of a block
   const int nb = mode == MODE_INIT ? g.nnmax : g.nbmax;
-  const dim3 g2(g.n, nb * g.npanmax);
+  // tiles of a block: of the two-launch kernels, or of the initial reduction
+  // (one tile up to 64 bands)
+  const dim3 g2(g.n, nb * (rk == RK_GEMM64 || rk == RK_GEMM32 ? g.npanmax : 1));
   // one tile per block: both products in one launch, XCD-aware
   // one-dimensional grid (see k_rot_fused)
   const dim3 gb((unsigned)(8 * ((g.n + 7) / 8) * nb));
@@ -1028,27 +1041,32 @@ void launch_rot_kernel(hipStream_t s, const Prob* P, const Item* it, const Seg& 
     else hipLaunchKernelGGL((k_reduce_tiles<T2, 64>), g2, dim3(256), 0, s, P, it, g.n, mode);
     return;
   }
-  switch (rk) {
-    case RK_FUSED32:
-      hipLaunchKernelGGL((k_rot_fused<T2, 32>), gb, dim3(256), 0, s, P, it, g.n, nb, mode);
-      break;
-    case RK_FUSED64:
-      hipLaunchKernelGGL((k_rot_fused<T2, 64>), gb, dim3(256), 0, s, P, it, g.n, nb, mode);
-      break;
-    case RK_FUSED48:
-      hipLaunchKernelGGL((k_rot_fused<T2, 48>), gb, dim3(FusedWaves<48>::NT), 0, s, P, it, g.n, nb, mode);
-      break;
-    case RK_DIRECT64:
-      hipLaunchKernelGGL(k_rot_direct<T2>, gb, dim3(256), 0, s, P, it, g.n, nb, mode);
-      break;
-    case RK_GEMM64:
-      hipLaunchKernelGGL((k_rot_gemm<T2, 1, 64>), g2, dim3(256), 0, s, P, it, g.n, mode);
-      hipLaunchKernelGGL((k_rot_gemm<T2, 2, 64>), g2, dim3(256), 0, s, P, it, g.n, mode);
-      break;
-    default:  // RK_GEMM32
-      hipLaunchKernelGGL((k_rot_gemm<T2, 1, 32>), g2, dim3(256), 0, s, P, it, g.n, mode);
-      hipLaunchKernelGGL((k_rot_gemm<T2, 2, 32>), g2, dim3(256), 0, s, P, it, g.n, mode);
-      break;
+  if (rk == RK_GEMM64) {
+    hipLaunchKernelGGL((k_rot_gemm<T2, 1, 64>), g2, dim3(256), 0, s, P, it, g.n, mode);
+    hipLaunchKernelGGL((k_rot_gemm<T2, 2, 64>), g2, dim3(256), 0, s, P, it, g.n, mode);
+  } else if (rk == RK_GEMM32) {
+    hipLaunchKernelGGL((k_rot_gemm<T2, 1, 32>), g2, dim3(256), 0, s, P, it, g.n, mode);
+    hipLaunchKernelGGL((k_rot_gemm<T2, 2, 32>), g2, dim3(256), 0, s, P, it, g.n, mode);
+  } else {
+    constexpr bool fp64 = std::is_same<T2, cplx>::value;
+    if constexpr (fp64) {
+      // 17-48 bands in FP64: column panels, whichever tile the FP32 phase has.
+      // Several blocks of a k to a workgroup (E_k staged once) on large sets
+      const int most = std::min(std::min(nb, W90_ROT_SLOTS), std::max(1, nb * g.n / kRotGroups));
+      const int nchunk = (nb + most - 1) / most, bchunk = (nb + nchunk - 1) / nchunk;
+      const dim3 gp((unsigned)(8 * ((g.n + 7) / 8) * nchunk));
+      if (g.nwmin <= 32)
+        hipLaunchKernelGGL(k_rot_panel<2>, gp, dim3(128), 0, s, P, it, g.n, nchunk, bchunk, mode);
+      if (g.nwmin <= 48 && g.nwmax > 32)
+        hipLaunchKernelGGL(k_rot_panel<3>, gp, dim3(192), 0, s, P, it, g.n, nchunk, bchunk, mode);
+      if (g.nwmax <= W90_ROT_PANEL_MAX) return;
+    } else {
+      if (rk == RK_FUSED32) hipLaunchKernelGGL((k_rot_fused<T2, 32>), gb, dim3(256), 0, s, P, it, g.n, nb, mode);
+      if (rk == RK_FUSED48)
+        hipLaunchKernelGGL((k_rot_fused<T2, 48>), gb, dim3(FusedWaves<48>::NT), 0, s, P, it, g.n, nb, mode);
+    }
+    if (rk == RK_FUSED64) hipLaunchKernelGGL((k_rot_fused<T2, 64>), gb, dim3(256), 0, s, P, it, g.n, nb, mode);
+    if (rk == RK_DIRECT64) hipLaunchKernelGGL(k_rot_direct<T2>, gb, dim3(256), 0, s, P, it, g.n, nb, mode);
   }
 }
 
@@ -1217,7 +1235,9 @@ int tune_member(Engine* E, Member* m) {
   for (int pass = 0; pass < 2; ++pass)
     for (size_t i = 0; i < cand.size(); ++i)
       if ((rc = time_one(cand[pass ? cand.size() - 1 - i : i]))) return rc;
-  const int d = default_rot(c);
+  // up to W90_ROT_PANEL_MAX bands every candidate rotates FP64 alike: the choice
+  // is for the FP32 phase, and the table's, unless measured otherwise
+  const int d = nw <= W90_ROT_PANEL_MAX ? table_rot(nw, m->nn) : default_rot(c);
   int pick = d;
   for (int rk : cand)
     if (t[rk] < t[pick]) pick = rk;

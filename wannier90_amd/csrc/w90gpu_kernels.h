@@ -44,6 +44,8 @@ typedef double2 cplx;
 #define W90_NT 256          // threads per workgroup of the per-k kernels
 #define W90_STEP_NT 1024    // threads of the global-memory retraction (above W90_PANEL_MAX bands)
 #define W90_PANEL_MAX 96    // most bands whose matrix fits a workgroup's LDS (k_step_panel)
+#define W90_ROT_PANEL_MAX 48 // most bands of the FP64 rotation by column panels (k_rot_panel)
+#define W90_ROT_SLOTS 12     // most blocks of a k that one of its workgroups takes
 #define W90_OMEGA_NT 512    // threads of the omega reduction
 #define W90_MAX_GROUPS 64   // most k-ranges (workgroups) of a problem's omega reduction
 #define W90_MIXED_RTOL 1e-8 // relative FP32 noise floor of Omega differences in the bulk phase

@@ -508,8 +508,8 @@ __device__ __forceinline__ void rot_fused_tile(const Prob& p, int k, int b, int 
   }
 }
 
-// The rotation for num_wann <= GT (one tile per block), both products in
-// one workgroup per (item, b) with T in LDS (rot_fused_tile).  Workgroups
+// The rotation for num_wann <= GT (one tile per block) in FP32, and in FP64 above
+// W90_ROT_PANEL_MAX bands, both products in one workgroup per (item, b) with T in LDS (rot_fused_tile).  Workgroups
 // are placed XCD-aware: a one-dimensional grid of 8 * ceil(nitems / 8) *
 // nnmax workgroups, where workgroup w runs on XCD w % 8 (round-robin
 // dispatch) and takes item 8 t + w % 8 and neighbour b with
@@ -526,6 +526,7 @@ __global__ void __launch_bounds__(FusedWaves<GT>::NT, FusedWaves<GT>::MINB) k_ro
   const Item it = items[item];
   const Prob& p = probs[it.prob];
   const State* st = p.st;
+  if (sizeof(T2) == sizeof(cplx) && p.nw <= W90_ROT_PANEL_MAX) return;  // k_rot_panel's
   const int cur = gate_cur(st, mode);
   if (cur < 0) return;
   int mate;
@@ -775,6 +776,7 @@ __global__ void __launch_bounds__(256, 2) k_rot_direct(const Prob* probs, const 
   const Item it = items[item];
   const Prob& p = probs[it.prob];
   const State* st = p.st;
+  if (sizeof(T2) == sizeof(cplx) && p.nw <= W90_ROT_PANEL_MAX) return;  // k_rot_panel's
   const int cur = gate_cur(st, mode);
   if (cur < 0) return;
   int mate;
@@ -824,6 +826,9 @@ __global__ void __launch_bounds__(256) k_reduce_tiles(const Prob* probs, const I
   if (threadIdx.x == 0) {
     p.part_od[kb * p.npan + tile] = od;
     p.part_all[kb * p.npan + tile] = all;
+    // slots that only the FP64 rotation fills (one per 16 columns)
+    if (tile == 0)
+      for (int q = ntl; q < p.npan; ++q) p.part_od[kb * p.npan + q] = p.part_all[kb * p.npan + q] = 0.0;
   }
 }
 
@@ -885,6 +890,237 @@ __device__ __forceinline__ void panel_product(const cplx* L, Get get, Out out) {
       __builtin_amdgcn_sched_barrier(0);
     }
     out(i, acc);
+  }
+}
+
+// ------------------------------------------------ rotation by column panels
+
+// The FP64 rotation for num_wann 17-48: R = E_k^+ (M(k,b) E_{k+b}) with one
+// wavefront per 16 columns, TN = ceil(num_wann / 16) of them.  E_k^+ is the A
+// operand of the second product for every b of the k: a workgroup stages it in
+// LDS once and takes up to bchunk blocks of the k.  The first product's A operand
+// is M itself, read from memory in operand order (rows along the lanes), kRotPF
+// K steps ahead, with a row tile ahead of that touched for L2; its B operand, the
+// wavefront's columns of E_{k+b}, and its result, which is the B operand of the
+// second product as it stands, stay in registers.  No barrier between the
+// products or blocks: wavefronts drift apart and cover each other's loads.  The
+// next block's columns of E and first operands of M arrive during the second
+// product.
+//
+// Epilogue: R to the other buffer (and its adjoint to the pair's block), the
+// sums of |M|^2 of the wavefront's columns (TN partial sums per block), and the
+// diagonal to LDS: Im ln M_nn and |M_nn|^2 follow at the end, for inside the loop
+// the compiler keeps atan2's constants in 40 registers over the products.
+// Items with another TN are left out.  Placement as k_rot_fused (the workgroups
+// of a k back to back on one XCD).
+//
+// Per block two products of 48 TN^3 MFMA instructions, 64 cycles each: 23 us of
+// the 61 at 44 bands; the rest are the chain of tables, E_k and first operands
+// before a workgroup's products (7 us) and, at TN = 3, three wavefronts to four
+// SIMDs.  Measured per rotation by pairs against a workgroup per block with both
+// products staged through LDS in K chunks, two barriers a chunk (k_rot_fused):
+//   27 bands, 216 k: 27.2 -> 21.8 us   32 bands, 512 k: 30.4 -> 25.2 us
+//   44 bands, 343 k: 69.0 -> 61.0 us   48 bands, 216 k: 71.0 -> 64 us
+// With four panels the two operand panels, the accumulators and the loads in
+// flight pass the 256 registers: 76 -> 76 us at 52 bands and 404 -> 382 at 64
+// with scratch traffic, so 49-64 bands stay with k_rot_fused and k_rot_direct.
+constexpr int kRotPF = 4;  // K steps of M in flight
+
+// A pointer that is the same in every lane (said to the compiler here).
+template <class T>
+__device__ __forceinline__ T* uniform(T* q) {
+  const unsigned long long u = (unsigned long long)q;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)u), hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
+  return (T*)(((unsigned long long)hi << 32) | lo);
+}
+
+// A matrix of `bytes` bytes as a buffer: offsets past it read zero, writes there
+// are dropped.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const cplx* base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)uniform(base), 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+__device__ __forceinline__ cplx buf_load(__amdgpu_buffer_rsrc_t r, unsigned byte) {
+  return __builtin_bit_cast(cplx, __builtin_amdgcn_raw_buffer_load_b128(r, byte, 0, 0));
+}
+__device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, unsigned byte, cplx v) {
+  typedef unsigned v4u __attribute__((ext_vector_type(4)));
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), r, byte, 0, 0);
+}
+
+// What the rotation reads of a problem, in scalar registers: read after a store
+// it would wait for the store.
+struct RotProb {
+  const cplx *E, *src;
+  cplx* out;
+  double *od, *all;
+  int nw, nn, npan;
+  __device__ __forceinline__ void read(const Prob& p, int mode, int cur) {
+    E = uniform((const cplx*)p.E);
+    src = uniform(rot_src<cplx>(p, mode, cur));
+    out = uniform(p.M[dst_buf(mode, cur)]);
+    od = uniform(p.part_od);
+    all = uniform(p.part_all);
+    nw = __builtin_amdgcn_readfirstlane(p.nw);
+    nn = __builtin_amdgcn_readfirstlane(p.nn);
+    npan = __builtin_amdgcn_readfirstlane(p.npan);
+  }
+};
+
+template <int TN>
+__global__ void __launch_bounds__(64 * TN, kStepWaves(TN)) k_rot_panel(const Prob* probs, const Item* items,
+                                                                      int nitems, int nchunk, int bchunk, int mode) {
+  const int wg = blockIdx.x, rr = wg >> 3;
+  const int item = 8 * (rr / nchunk) + (wg & 7);
+  if (item >= nitems) return;
+  const Item it = items[item];
+  const Prob& p = probs[it.prob];
+  if ((p.nw + 15) / 16 != TN) return;
+  const int cur = gate_cur(p.st, mode);
+  if (cur < 0) return;
+  const int j0 = (rr % nchunk) * bchunk, nu = min(bchunk, (p.npair > 0 ? p.npair : p.nn) - j0);
+  if (nu <= 0) return;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lk = lane >> 4, k = it.k;
+  __shared__ cplx L[TN * TN * 256];
+  __shared__ cplx dg[W90_ROT_SLOTS * 16 * TN];
+  __shared__ int slot_b[W90_ROT_SLOTS], slot_mate[W90_ROT_SLOTS], slot_k[W90_ROT_SLOTS];
+  if ((int)threadIdx.x < nu) {
+    int m;
+    const int b = rot_slot<cplx>(p, k, j0 + threadIdx.x, &m);
+    slot_b[threadIdx.x] = b;
+    slot_mate[threadIdx.x] = m;
+    slot_k[threadIdx.x] = p.nnl[(size_t)k * p.nn + b];
+  }
+  RotProb F;
+  F.read(p, mode, cur);
+  const int nw = F.nw, nw2 = nw * nw, bytes = 16 * nw2;
+  const unsigned ks = 64u * nw;
+  const int col = 16 * w + lr;
+  auto row_of = [&](int t, int q) { return 16 * t + 4 * q + lk; };
+  const unsigned far = 0xc0000000u;  // past any matrix, also with a tile's offset added
+  constexpr int NS = 4 * TN;         // K steps of the first product
+  auto load_panel = [&](const cplx* E, Panel<TN>& P) {
+    const auto r = buf_rsrc(E, bytes);
+    const unsigned oc = 16u * (unsigned)(col * nw + lk);
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const cplx e = buf_load(r, oc + 16u * (16 * t + 4 * q));
+        P.r[t][q] = e.x;
+        P.i[t][q] = e.y;
+      }
+  };
+  // a word of every 64 bytes of a row tile of M, the wavefront's columns: the
+  // operand loads of all wavefronts, a row tile later, then find it in L2
+  unsigned warm = 0;
+  auto touch = [&](__amdgpu_buffer_rsrc_t r, int i) {
+    warm = __builtin_amdgcn_raw_buffer_load_b32(r, 16u * (unsigned)(col * nw + 4 * lk) + 256u * i, 0, 0);
+  };
+  cplx a[kRotPF];  // M's operand of K step x % NS, row tile x / NS
+  Panel<TN> B, P;
+  load_panel(F.E + (size_t)k * nw2, P);
+  __syncthreads();
+  int b, mate;
+  // columns of E and first operands of M of slot u
+  auto begin = [&](int u) {
+    b = __builtin_amdgcn_readfirstlane(slot_b[u]);
+    mate = __builtin_amdgcn_readfirstlane(slot_mate[u]);
+    load_panel(F.E + (size_t)__builtin_amdgcn_readfirstlane(slot_k[u]) * nw2, B);
+    const auto m = buf_rsrc(F.src + ((size_t)k * F.nn + b) * nw2, bytes);
+    const unsigned of = 16u * (unsigned)(lk * nw + lr);
+#pragma unroll
+    for (int x = 0; x < kRotPF; ++x) a[x] = buf_load(m, of + x * ks);
+  };
+  begin(0);
+#pragma unroll
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (row_of(t, q) >= nw) P.r[t][q] = P.i[t][q] = 0.0;
+  panel_to_lds<TN>(L, P);
+  __syncthreads();
+  for (int u = 0; u < nu; ++u) {
+    const size_t kb = (size_t)k * F.nn + b;
+    const auto msrc = buf_rsrc(F.src + kb * nw2, bytes);
+    // offsets anew for each block: kept over the loop they take the panels' registers
+    unsigned of = 16u * (unsigned)(lk * nw + lr), oc = 16u * (unsigned)(col * nw + lk),
+             om = col < nw ? 16u * (unsigned)(lk * nw + col) : far;
+    asm volatile("" : "+v"(of), "+v"(oc), "+v"(om));
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+      Cfrag<double> acc;
+      acc.zero();
+      if (i + 1 < TN) touch(msrc, i + 1);
+#pragma unroll
+      for (int sk = 0; sk < NS; ++sk) {
+        const int x = i * NS + sk, y = x + kRotPF;
+        const cplx v = a[x % kRotPF];
+        if (y < TN * NS) a[x % kRotPF] = buf_load(msrc, of + (y % NS) * ks + 256u * (y / NS));
+        acc.mma(v.x, v.y, B.r[sk / 4][sk % 4], B.i[sk / 4][sk % 4]);
+        if (sk % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        P.r[i][q] = acc.re(q);
+        P.i[i][q] = acc.im(q);
+        // formed here: left to the compiler the three accumulators stay, half as many registers again
+        asm volatile("" : "+v"(P.r[i][q]), "+v"(P.i[i][q]));
+      }
+      asm volatile("" ::"v"(warm));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the next block's, ahead of this one's stores, which share the wait counter
+    const int part = kb * F.npan + w, matep = mate;
+    const auto out = buf_rsrc(F.out + kb * nw2, bytes);
+    const auto outm = buf_rsrc(F.out + (mate >= 0 ? (size_t)mate * nw2 : 0), mate >= 0 ? bytes : 0);
+    if (u + 1 < nu) begin(u + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    double od = 0.0, all = 0.0;
+    panel_product<TN, true>(
+        L, [&](int t, int q, double& br, double& bi) { br = P.r[t][q]; bi = P.i[t][q]; },
+        [&](int i, const Cfrag<double>& acc) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int row = row_of(i, q);
+            const cplx v = c_make(acc.re(q), acc.im(q));
+            buf_store(out, i < TN - 1 || row < nw ? oc + 16u * (16 * i + 4 * q) : far, v);
+            buf_store(outm, om + (4 * i + q) * ks, c_conj(v));
+            const double a2 = c_abs2(v);  // zero past num_wann
+            all += a2;
+            if (i == w) {  // the tile on the diagonal
+              od += 4 * q + lk != lr ? a2 : 0.0;
+              if (4 * q + lk == lr) dg[u * 16 * TN + col] = v;
+            } else {
+              od += a2;
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        });
+    od = wave_sum(od);
+    all = wave_sum(all);
+    if (lane == 0) {
+      F.od[part] = od;
+      F.all[part] = all;
+      if (matep >= 0) {
+        F.od[matep * F.npan + w] = od;
+        F.all[matep * F.npan + w] = all;
+      }
+    }
+  }
+  __syncthreads();
+  double *ln = p.ln[dst_buf(mode, cur)], *d2 = p.d2;
+  for (int e = threadIdx.x; e < nu * 16 * TN; e += 64 * TN) {
+    const int u = e / (16 * TN), n = e - u * 16 * TN, m = slot_mate[u];
+    if (n >= nw) continue;
+    const cplx z = dg[e];
+    const size_t at = ((size_t)k * F.nn + slot_b[u]) * nw + n;
+    const double l = atan2(z.y, z.x), a2 = c_abs2(z);
+    ln[at] = l;
+    d2[at] = a2;
+    if (m >= 0) {
+      ln[(size_t)m * nw + n] = -l;
+      d2[(size_t)m * nw + n] = a2;
+    }
   }
 }
 
