@@ -31,8 +31,8 @@
 // Hermitian eigenproblems (of Z, Q P Q and the subspace Hamiltonian) are
 // solved in the workgroup by a two-sided cyclic Jacobi method with
 // round-robin (tournament) ordering: n/2 disjoint complex rotations per
-// round, applied to A (by 2 x 2 blocks) and to the basis between two
-// barriers; the polar factors (of A and of U_opt^+ A) by the one-sided Jacobi
+// round, applied to A (by 2 x 2 blocks) and to the basis, one barrier a round;
+// the polar factors (of A and of U_opt^+ A) by the one-sided Jacobi
 // SVD with the same ordering.  A workgroup's matrices live in LDS up to order
 // 64 (two 64 x 65 complex blocks); up to 96 the matrix does and the basis is
 // in the workgroup's own area of global memory, which holds both above that,

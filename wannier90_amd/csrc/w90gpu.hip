@@ -78,11 +78,11 @@ struct Member {
 };
 
 // kernel classes by num_wann: the wavefront-per-neighbour MFMA rotation up
-// to 16; the one-workgroup-per-block MFMA rotation (32 x 32 tile, T in LDS)
-// with the per-k LDS retraction and gradient up to 32; the same rotation
-// with a 64 x 64 (or, up to 48 bands, 48 x 48) tile, the MFMA retraction
-// and the LDS gradient up to 64; the two-launch MFMA rotation (tiles over
-// panels) with the global-memory retraction and the tiled gradient up to
+// to 16; one-launch rotations up to 64 (FP64 to 48 bands by column panels, else
+// a workgroup per block with T in LDS), with the chunked LDS gradient up to 32
+// and the one-block LDS gradient up to 64; the two-launch MFMA rotation (tiles
+// over panels) with the tiled gradient above.  The retraction is by column
+// panels up to W90_PANEL_MAX and in global memory from there to
 // W90GPU_MAX_WANN
 constexpr int kClasses = 4;
 constexpr int kLdsMaxWann = 32;

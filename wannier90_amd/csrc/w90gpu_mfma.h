@@ -2,10 +2,11 @@
 // M(k,b) <- E_k^+ M(k,b) E_{k+b} as two complex products on
 // v_mfma_*_16x16x4 tiles (FP64 for the plain path, FP32 with FP32
 // accumulation for the mixed bulk phase), and the products of the
-// retraction (k_step_panel up to num_wann 64).
+// retraction (k_step_panel up to num_wann 96).
 //
 // num_wann <= 16 (k_rotate_w16): one 16 x 16 tile per block, one wavefront
-// per neighbour b.  num_wann 17-64 (k_rot_fused): a workgroup computes both
+// per neighbour b.  num_wann 17-48 in FP64 (k_rot_panel): a wavefront per 16
+// columns, no barriers.  num_wann 17-64 else (k_rot_fused): a workgroup computes both
 // products of one (k, b) block as one GT x GT tile (GT = 32, 48 or 64), T
 // kept in LDS between them.  num_wann 65-256 (k_rot_gemm): each product is
 // its own launch over up to 4 x 4 tiles of 64 (or 8 x 8 of 32), T through
