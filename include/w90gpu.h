@@ -245,9 +245,9 @@ int w90gpu_session_rotation_time(w90gpu_session* sess, int reps, double* avg_ms)
 /* The same for one phase of an iteration: W90GPU_PHASE_ROTATION (as
  * above), W90GPU_PHASE_GRADIENT (wann_domega: G and its per-k norms),
  * W90GPU_PHASE_RETRACTION (exp of the scaled search direction and the U
- * update of the parabolic step) or W90GPU_PHASE_REDUCTION (the final
- * reduction of wann_omega over k, without the control logic that follows
- * it).  Each launch rewrites scratch buffers only (the other M or U buffer,
+ * update of the parabolic step) or W90GPU_PHASE_REDUCTION (the per-k
+ * vectors of wann_omega and their reduction over k, without the control
+ * logic that follows it).  Each launch rewrites scratch buffers only (the other M or U buffer,
  * G, exp(dW), the other centres buffer), so the returned M, U and centres
  * of the solve are unchanged. */
 #define W90GPU_PHASE_ROTATION 0
