@@ -368,8 +368,9 @@ int w90gpu_disentangle(w90gpu_ctx* ctx, const w90gpu_problem* prob, int num_band
  * is compiled into the library, else the class default.  With the
  * environment variable W90GPU_TUNE=1 when a context or batch is created, a
  * key without a choice is measured at the start of its first solve: every
- * candidate is timed on the problem's own data, and one replaces the
- * default only if it is at least 3% faster.  W90GPU_TUNE_FILE=<path> reads
+ * candidate is timed on the problem's own buffers (up to 48 bands in FP32,
+ * the only phase that has a choice there; above in FP64), and one replaces
+ * the default only if it is at least 3% faster.  W90GPU_TUNE_FILE=<path> reads
  * choices from, and appends measurements to, a text file.  Results depend
  * on the kernel only through rounding. */
 /* Name of the kernel that a problem of this shape admitted now would use

@@ -769,13 +769,6 @@ void tune_refresh() {
   }
 }
 
-// The table's choice, or the class default.
-int table_rot(int nw, int nn) {
-  for (const TuneRow& r : kTuneTable)
-    if (nw >= r.nw_lo && nw <= r.nw_hi && nn >= r.nn_lo && nn <= r.nn_hi && rot_serves(r.rk, nw)) return r.rk;
-  return default_rot(wann_class(nw));
-}
-
 // The rotation kernel of a problem.  *pending (when given) is set if the
 // key is to be measured at the start of its first solve; until then the
 // class default stands.
@@ -791,7 +784,9 @@ int rot_choice(int nw, int nn, bool* pending) {
     if (pending && first_group(c) != last_group(c)) *pending = true;
     return default_rot(c);
   }
-  return table_rot(nw, nn);
+  for (const TuneRow& r : kTuneTable)
+    if (nw >= r.nw_lo && nw <= r.nw_hi && nn >= r.nn_lo && nn <= r.nn_hi && rot_serves(r.rk, nw)) return r.rk;
+  return default_rot(c);
 }
 
 // Admit a problem: pool bytes, a slot, its k-mesh tables and state template.
@@ -1187,9 +1182,11 @@ int enqueue_iteration(Engine* E, const Lists& L, bool lean = false) {
   return W90GPU_OK;
 }
 
-// Measure the rotation candidates of a member's class on its own data and
-// fix the choice for its (num_wann, nntot).  Each candidate runs in
-// MODE_BENCH (a trial rotation of the current buffer that writes only the
+// Measure the rotation candidates of a member's class on its own buffers and
+// fix the choice for its (num_wann, nntot).  What is timed is what the choice
+// is for: up to W90_ROT_PANEL_MAX bands the FP32 rotation (in FP64 every
+// candidate is k_rot_panel there), above it the FP64 one.  Each candidate runs
+// in MODE_BENCH (a trial rotation of the current buffer that writes only the
 // other buffer, the per-(k,b) outputs and the partial sums, all rebuilt by
 // the initial evaluation that follows) over the member's k items, repeated
 // so that one launch holds at least kTuneItems items, as in a batch; five
@@ -1212,13 +1209,14 @@ int tune_member(Engine* E, Member* m) {
   std::vector<int> cand;
   for (int g = first_group(c); g <= last_group(c); ++g)
     if (rot_serves(kGroupRot[g], nw)) cand.push_back(kGroupRot[g]);
+  const int prec = nw <= W90_ROT_PANEL_MAX ? 1 : 0;  // as in Lists: 0 FP64, 1 FP32
   double t[kRotKernels];
   for (double& x : t) x = 1e30;
   auto time_one = [&](int rk) -> int {
     m->p.npan = rot_panels(rk, nw);
     HIPCHK(E->ctx, hipMemcpyAsync(E->d_probs + m->slot, &m->p, sizeof(Prob), hipMemcpyHostToDevice, E->stream));
     Lists L;
-    one_group_lists(L, group_of(c, rk), 0, n, nn, m->p.npan, nw);
+    one_group_lists(L, group_of(c, rk), prec, n, nn, m->p.npan, nw);
     L.items = E->d_aux_items;
     int r = launch_rotate(E, L, MODE_BENCH);
     if (r) return r;
@@ -1235,9 +1233,7 @@ int tune_member(Engine* E, Member* m) {
   for (int pass = 0; pass < 2; ++pass)
     for (size_t i = 0; i < cand.size(); ++i)
       if ((rc = time_one(cand[pass ? cand.size() - 1 - i : i]))) return rc;
-  // up to W90_ROT_PANEL_MAX bands every candidate rotates FP64 alike: the choice
-  // is for the FP32 phase, and the table's, unless measured otherwise
-  const int d = nw <= W90_ROT_PANEL_MAX ? table_rot(nw, m->nn) : default_rot(c);
+  const int d = default_rot(c);
   int pick = d;
   for (int rk : cand)
     if (t[rk] < t[pick]) pick = rk;
