@@ -5,6 +5,10 @@ kernel whatever the choice), so it has to time the FP32 kernels: at 24 bands
 fused64 works on a padded 64 x 64 tile, four times the area of fused32's, and
 2.9 to 3.3 times slower by the FP64 instances of both; 1.5 times is asked for.
 Timings of one kernel under two names agree to a few percent.
+
+Above 48 bands it times the FP64 rotation as it will run: for overlaps that
+pair, half of the blocks.  At 52 bands 0.8 of the time block by block is asked
+for (0.61 at 64 bands, measured as 419 of 690 us).
 """
 import pytest
 
@@ -55,3 +59,14 @@ def test_up_to_48_bands_the_fp32_kernels_are_timed(monkeypatch, tmp_path, mixed)
     assert set(t) == {"fused32", "fused64"}
     assert t["fused64"] > 1.5 * t["fused32"]
     assert pick == "fused32"
+
+
+def test_above_48_bands_the_rotation_by_pairs_is_timed(monkeypatch, tmp_path):
+    p, u, m = problem(52)
+    _, by_pairs = tuned(monkeypatch, tmp_path / "pairs.txt", p.kmesh, 52, p.num_kpts, m, u)
+    m1 = m.copy(order="F")
+    m1[51, 0, 0, 0] += 1e-3
+    _, by_block = tuned(monkeypatch, tmp_path / "blocks.txt", p.kmesh, 52, p.num_kpts, m1, u)
+    assert set(by_pairs) == set(by_block) == {"fused64", "direct64"}
+    for k in by_pairs:
+        assert by_pairs[k] < 0.8 * by_block[k]

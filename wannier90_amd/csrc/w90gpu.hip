@@ -179,16 +179,19 @@ struct Lists {
   bool any_second = false;
 };
 
-// Lists over n items of one group and precision (the segments before it
-// empty at 0, those after it empty at n).
-void one_group_lists(Lists& L, int g0, int q0, int n, int nn, int npan, int nw) {
+// Blocks per k that a problem's rotation forms in a precision (0 FP64, 1 FP32).
+int formed_blocks(const Prob& p, int q) { return q == 0 && p.npair > 0 ? p.npair : p.nn; }
+
+// Lists over n items of one problem, group and precision (the segments before
+// it empty at 0, those after it empty at n).
+void one_group_lists(Lists& L, int g0, int q0, int n, const Prob& p) {
   for (int c = 0; c < kClasses; ++c)
     for (int q = 0; q < 2; ++q)
       for (int g = first_group(c); g <= last_group(c); ++g) {
         const bool after = c > kGroupClass[g0] || (c == kGroupClass[g0] && (q > q0 || (q == q0 && g > g0)));
         L.seg[g][q] = Seg{after ? n : 0, 0, 0, 0};
       }
-  L.seg[g0][q0] = Seg{0, n, nn, npan, nn, nw, nw};
+  L.seg[g0][q0] = Seg{0, n, p.nn, p.npan, formed_blocks(p, q0), p.nw, p.nw};
 }
 
 struct Pool {
@@ -925,7 +928,7 @@ void build_lists(const std::vector<Member*>& ms, F prec_of, std::vector<Item>& i
           for (int k = 0; k < m->nk; ++k) items.push_back(Item{m->slot, k});
           s.nnmax = std::max(s.nnmax, m->nn);
           s.npanmax = std::max(s.npanmax, rot_panels(m->rk, m->nw));
-          s.nbmax = std::max(s.nbmax, q == 0 && m->p.npair > 0 ? m->p.npair : m->nn);
+          s.nbmax = std::max(s.nbmax, formed_blocks(m->p, q));
           s.nwmin = s.nwmin ? std::min(s.nwmin, m->nw) : m->nw;
           s.nwmax = std::max(s.nwmax, m->nw);
         }
@@ -1185,7 +1188,8 @@ int enqueue_iteration(Engine* E, const Lists& L, bool lean = false) {
 // Measure the rotation candidates of a member's class on its own buffers and
 // fix the choice for its (num_wann, nntot).  What is timed is what the choice
 // is for: up to W90_ROT_PANEL_MAX bands the FP32 rotation (in FP64 every
-// candidate is k_rot_panel there), above it the FP64 one.  Each candidate runs
+// candidate is k_rot_panel there), above it the FP64 one, by pairs if the
+// member's overlaps pair.  Each candidate runs
 // in MODE_BENCH (a trial rotation of the current buffer that writes only the
 // other buffer, the per-(k,b) outputs and the partial sums, all rebuilt by
 // the initial evaluation that follows) over the member's k items, repeated
@@ -1216,7 +1220,7 @@ int tune_member(Engine* E, Member* m) {
     m->p.npan = rot_panels(rk, nw);
     HIPCHK(E->ctx, hipMemcpyAsync(E->d_probs + m->slot, &m->p, sizeof(Prob), hipMemcpyHostToDevice, E->stream));
     Lists L;
-    one_group_lists(L, group_of(c, rk), prec, n, nn, m->p.npan, nw);
+    one_group_lists(L, group_of(c, rk), prec, n, m->p);
     L.items = E->d_aux_items;
     int r = launch_rotate(E, L, MODE_BENCH);
     if (r) return r;
@@ -1285,15 +1289,16 @@ int tune_pending(Engine* E, const std::vector<Member*>& ms) {
 // the initial wann_omega in FP64, and the FP32 copy of M for the mixed
 // bulk phase.
 int enqueue_start(Engine* E, const std::vector<Member*>& ms) {
-  int rc = tune_pending(E, ms);
-  if (rc) return rc;
-  // rotation by pairs or block by block, as the loaded overlaps allow
+  // rotation by pairs or block by block, as the loaded overlaps allow (before
+  // the tuner, which times what will run)
   for (Member* m : ms) {
     const int np = m->paired ? m->pairs : 0;
     if (np == m->p.npair) continue;
     m->p.npair = np;
     HIPCHK(E->ctx, hipMemcpyAsync(E->d_probs + m->slot, &m->p, sizeof(Prob), hipMemcpyHostToDevice, E->stream));
   }
+  int rc = tune_pending(E, ms);
+  if (rc) return rc;
   Lists L;
   rc = aux_lists(E, ms, L);
   if (rc) return rc;
@@ -2239,7 +2244,7 @@ int w90gpu_omega_noalloc(w90gpu_ctx* ctx, const w90gpu_problem* prob, const doub
   L.np = 1;
   // the segments build_lists gives a single member: empty before and after
   // its group, all nk items in (group, FP64)
-  one_group_lists(L, group_of(m.cls, m.rk), 0, nk, nn, rot_panels(m.rk, nw), nw);
+  one_group_lists(L, group_of(m.cls, m.rk), 0, nk, m.p);
   L.orange = nk;
   L.nrange = m.p.ngroup;
   hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, nullptr, E.d_probs, L.plist, 1);
