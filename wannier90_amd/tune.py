@@ -2,8 +2,9 @@
 
 The autotuner lives in the engine (w90gpu.hip: rot_choice, tune_member): with
 W90GPU_TUNE=1 the first solve of each (num_wann, nntot) times every rotation
-kernel of its num_wann class on the problem's own resident data and keeps a
-candidate only if it is at least 3% faster than the class default; with
+kernel of its num_wann class on the problem's own buffers (up to 48 bands in
+FP32, where the choice is that of the FP32 phase only, above in FP64) and keeps
+a candidate only if it is at least 3% faster than the class default; with
 W90GPU_TUNE_FILE set, each choice is appended to that file as
 
     num_wann nntot kernel candidate=microseconds ... items=N
