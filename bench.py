@@ -54,7 +54,6 @@ sys.path.insert(0, ROOT)
 METRIC = "MLWF solves/s at ΔΩ≤1e-8 Å² vs FP64; p50/p99 latency; mixed vs plain GPU"
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
-FP32_PEAK_TFLOPS = 157.3
 
 
 def parse():
@@ -198,6 +197,29 @@ WORKLOADS = {
 PROFILE_STEM = {1: "sc4_64k", 2: "fcc16_512k", 3: "triclinic64_800k"}
 
 
+def rotation_roofline(sess, nw, nk, nn, launches):
+    """Duration of the FP64 rotation and its rate against the bound that its
+    arithmetic intensity gives.  Where the overlaps pair one block of each pair
+    is read and formed, and both are written."""
+    avg_ms = sess.rotation_time(launches)
+    formed = sess.formed_blocks()
+    rot_bytes = 16.0 * nk * nw * nw * (formed + nn + 1)  # M read + write, E once
+    rot_flops = 16.0 * nk * formed * nw ** 3             # two complex GEMMs per block formed
+    if rot_flops / rot_bytes < FP64_PEAK_TFLOPS * 1e12 / (HBM_PEAK_GBS * 1e9):
+        achieved = rot_bytes / (avg_ms * 1e-3) / 1e9
+        roof = dict(bound="hbm", achieved=achieved, peak=HBM_PEAK_GBS, unit="GB/s",
+                    frac=achieved / HBM_PEAK_GBS, traffic=None)
+    else:
+        achieved = rot_flops / (avg_ms * 1e-3) / 1e12
+        roof = dict(bound="mfma", achieved=achieved, peak=FP64_PEAK_TFLOPS, unit="TFLOP/s",
+                    frac=achieved / FP64_PEAK_TFLOPS, traffic=None)
+    kname = ("k_rotate_w16" if nw <= 16 else "k_rot_panel" if nw <= 48
+             else "k_rot_fused" if nw <= 64 else "k_rot_gemm stage 1 + stage 2")
+    roof.update(kernel=kname, avg_launch_ms=avg_ms, launches=launches,
+                algorithmic_bytes=rot_bytes, algorithmic_flops=rot_flops)
+    return roof
+
+
 def measured_traffic(config, precision):
     """HBM bytes per launch of the rotation kernel from the committed PMC
     summary of the same workload (profiles/*_pmc.json: FETCH_SIZE and
@@ -308,30 +330,11 @@ def main():
     # the dominant kernel (M rotation with the fused omega partial sums):
     # HIP events around back-to-back launches on the final state
     launches = 200 if prob.num_wann <= 32 else 20
-    avg_ms = sess.rotation_time(launches)
-    nk, nn, nw = prob.num_kpts, prob.kmesh.nntot, prob.num_wann
-    # generated overlaps hold M(k+b,-b) = M(k,b)^+: in FP64 above 16 bands one
-    # block of each pair is read and formed, and both are written
-    formed = nn // 2 if prec == capi.PREC_FP64 and nw > 16 else nn
-    rot_bytes = (16.0 if prec == capi.PREC_FP64 else 8.0) * nk * nw * nw * (formed + nn + 1)  # M read + write, E once
-    rot_flops = 16.0 * nk * formed * nw ** 3           # two complex GEMMs per block formed
-    ai = rot_flops / rot_bytes
-    peak_flops = FP64_PEAK_TFLOPS if prec == capi.PREC_FP64 else FP32_PEAK_TFLOPS
-    ridge = peak_flops * 1e12 / (HBM_PEAK_GBS * 1e9)
-    if ai < ridge:
-        achieved = rot_bytes / (avg_ms * 1e-3) / 1e9
-        roof = dict(bound="hbm", achieved=achieved, peak=HBM_PEAK_GBS, unit="GB/s",
-                    frac=achieved / HBM_PEAK_GBS, traffic=None)
-    else:
-        achieved = rot_flops / (avg_ms * 1e-3) / 1e12
-        roof = dict(bound="mfma", achieved=achieved, peak=peak_flops, unit="TFLOP/s",
-                    frac=achieved / peak_flops, traffic=None)
-    kname = ("k_rotate_w16" if nw <= 16 else "k_rot_panel" if nw <= 48 and prec == capi.PREC_FP64
-             else "k_rot_fused" if nw <= 64 else "k_rot_gemm stage 1 + stage 2")
-    roof.update(kernel=kname, avg_launch_ms=avg_ms, launches=launches,
-                algorithmic_bytes=rot_bytes, algorithmic_flops=rot_flops)
-    roof["traffic"] = measured_traffic(args.config, args.precision)
-    log(f"[bench] k_rotate: {launches} launches, avg {avg_ms * 1e3:.1f} us, AI={ai:.2f} flop/B")
+    roof = rotation_roofline(sess, prob.num_wann, prob.num_kpts, prob.kmesh.nntot, launches)
+    avg_ms = roof["avg_launch_ms"]
+    roof["traffic"] = measured_traffic(args.config, "fp64")
+    log(f"[bench] k_rotate: {launches} launches, avg {avg_ms * 1e3:.1f} us, "
+        f"AI={roof['algorithmic_flops'] / roof['algorithmic_bytes']:.2f} flop/B")
     # the other phases of an iteration, timed the same way (the omega
     # reductions and control are the remainder of the per-iteration time)
     phase_us = {"rotation": avg_ms * 1e3,
@@ -355,7 +358,7 @@ def main():
         "dtype": "f64" if prec == capi.PREC_FP64 else "f32+f64",
         "data": "synthetic",
         "config": {
-            "workload": WORKLOADS[args.config] + f", nntot={nn}, num_iter=500, conv_tol=1e-10, "
+            "workload": WORKLOADS[args.config] + f", nntot={prob.kmesh.nntot}, num_iter=500, conv_tol=1e-10, "
                         "conv_window=3, one problem per launch",
             "precision": args.precision,
             "iterations": its,

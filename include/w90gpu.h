@@ -233,6 +233,11 @@ int w90gpu_session_fetch(w90gpu_session* sess, double* m_matrix, double* u_matri
  * (src/wannierise.F90:703-756).  Writes min(rows, iterations+1) rows;
  * returns the number written or a negative status. */
 int w90gpu_session_history(w90gpu_session* sess, double* out, int rows);
+/* Blocks M(k,b) per k that the FP64 rotation of the loaded problem forms:
+ * nntot/2 where it works by adjoint pairs (above 16 bands, on a mesh whose
+ * blocks pair and overlaps that hold M(k+b,-b) = M(k,b)^+ to rounding), else
+ * nntot. */
+int w90gpu_session_formed_blocks(w90gpu_session* sess, int* blocks);
 /* Device bytes held by a session of this problem shape. */
 size_t w90gpu_session_bytes(int num_wann, int num_kpts, int nntot);
 /* Kernel timing: the M-rotation kernel of this problem (the fused rotation

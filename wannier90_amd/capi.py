@@ -117,6 +117,7 @@ SIGNATURES = [
     ("w90gpu_session_fetch", C.c_int, [_vp, _dp, _dp, _dp, _dp]),
     ("w90gpu_session_bytes", C.c_size_t, [C.c_int, C.c_int, C.c_int]),
     ("w90gpu_session_history", C.c_int, [_vp, _dp, C.c_int]),
+    ("w90gpu_session_formed_blocks", C.c_int, [_vp, _ip]),
     ("w90gpu_session_rotation_time", C.c_int, [_vp, C.c_int, _dp]),
     ("w90gpu_session_phase_time", C.c_int, [_vp, C.c_int, C.c_int, _dp]),
     ("w90gpu_problem_bytes", C.c_size_t, [C.c_int, C.c_int, C.c_int, C.c_int]),
@@ -509,8 +510,15 @@ class Session:
             raise W90Error(-n, self.ctx.error())
         return out[:n]
 
+    def formed_blocks(self):
+        """Blocks M(k,b) per k that the FP64 rotation of the loaded overlaps
+        forms: nntot/2 by adjoint pairs, else nntot."""
+        n = C.c_int(0)
+        self.ctx._check(self.lib.w90gpu_session_formed_blocks(self.h, C.byref(n)))
+        return n.value
+
     def rotation_time(self, reps=50):
-        """Average duration (ms) of the M-rotation kernel, `reps` launches
+        """Average duration (ms) of the FP64 M-rotation kernel, `reps` launches
         back to back on the final state of the last solve."""
         ms = C.c_double(0.0)
         self.ctx._check(self.lib.w90gpu_session_rotation_time(self.h, reps, C.byref(ms)))

@@ -1930,6 +1930,16 @@ int w90gpu_session_history(w90gpu_session* s, double* out, int rows) {
   return n;
 }
 
+int w90gpu_session_formed_blocks(w90gpu_session* s, int* blocks) {
+  if (!s || !blocks) return W90GPU_ERR_INPUT;
+  if (!s->loaded) {
+    set_error(s->eng->ctx, "formed_blocks needs a loaded session");
+    return W90GPU_ERR_INPUT;
+  }
+  *blocks = s->m->paired ? s->m->pairs : s->m->nn;
+  return W90GPU_OK;
+}
+
 int w90gpu_session_phase_time(w90gpu_session* s, int phase, int reps, double* avg_ms) {
   if (!s || reps < 1 || !avg_ms) return W90GPU_ERR_INPUT;
   if (phase < W90GPU_PHASE_ROTATION || phase > W90GPU_PHASE_REDUCTION) return W90GPU_ERR_INPUT;
