@@ -683,15 +683,21 @@ __device__ void zgemm_herm(int N, int K, const zd* A, int lda, const zd* B, int 
 
 // Eigenvalues (the diagonal of A after jacobi_run) into J.lam, their
 // ascending order into J.perm (ties by index) and its inverse into J.rank.
+// NaN sorts as +infinity: compared as it is, it would leave entries of J.perm
+// unset, and they index columns.
 template <class JL>
 __device__ __forceinline__ void eig_order(const zd* A, int n, int ld, JL& J) {
   const int t = threadIdx.x;
   if (t < n) J.lam[t] = A[t + t * ld].x;
   __syncthreads();
   if (t < n) {
-    const double l = J.lam[t];
+    auto key = [&](int j) { return J.lam[j] == J.lam[j] ? J.lam[j] : INFINITY; };
+    const double l = key(t);
     int rank = 0;
-    for (int j = 0; j < n; ++j) rank += (J.lam[j] < l || (J.lam[j] == l && j < t)) ? 1 : 0;
+    for (int j = 0; j < n; ++j) {
+      const double x = key(j);
+      rank += (x < l || (x == l && j < t)) ? 1 : 0;
+    }
     J.perm[rank] = t;
     J.rank[t] = rank;
   }
