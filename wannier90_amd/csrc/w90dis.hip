@@ -1410,7 +1410,8 @@ int windows(w90gpu_ctx* ctx, int nb, int nw, int nk, const w90gpu_dis_control* c
       }
       if (e[i - 1] <= c->win_max) imax = i;
     }
-    const int ndim = imax - imin + 1;
+    // (imin 0: the window lies between two bands of this k)
+    const int ndim = imin > 0 ? imax - imin + 1 : 0;
     if (ndim < nw) {
       w90gpu_set_error(ctx,
                        "dis_windows: Energy window contains fewer states than number of target WFs (k-point %d, "
