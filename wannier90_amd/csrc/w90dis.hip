@@ -63,10 +63,6 @@ __device__ __forceinline__ zd zmk(double r, double i) { return make_double2(r, i
 __device__ __forceinline__ zd zadd(zd a, zd b) { return make_double2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ zd zsub(zd a, zd b) { return make_double2(a.x - b.x, a.y - b.y); }
 __device__ __forceinline__ zd zmul(zd a, zd b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
-// conj(a) * b
-__device__ __forceinline__ zd zcmul(zd a, zd b) { return make_double2(a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x); }
-// a * conj(b)
-__device__ __forceinline__ zd zmulc(zd a, zd b) { return make_double2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y); }
 __device__ __forceinline__ zd zconj(zd a) { return make_double2(a.x, -a.y); }
 __device__ __forceinline__ zd zscale(zd a, double s) { return make_double2(a.x * s, a.y * s); }
 __device__ __forceinline__ double zabs2(zd a) { return a.x * a.x + a.y * a.y; }

@@ -63,10 +63,6 @@ __device__ __forceinline__ cplx c_conj(cplx a) { return make_double2(a.x, -a.y);
 __device__ __forceinline__ cplx c_mul(cplx a, cplx b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
-// conj(a) * b
-__device__ __forceinline__ cplx c_cmul(cplx a, cplx b) {
-  return make_double2(a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x);
-}
 __device__ __forceinline__ cplx c_div(cplx a, cplx b) {
   const double d = b.x * b.x + b.y * b.y;
   return make_double2((a.x * b.x + a.y * b.y) / d, (a.y * b.x - a.x * b.y) / d);
@@ -80,13 +76,6 @@ __device__ __forceinline__ float2 c_mul(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
-template <class T2>
-__device__ __forceinline__ T2 c_zero() {
-  T2 z;
-  z.x = 0;
-  z.y = 0;
-  return z;
-}
 // storage -> FP64 and FP64 -> storage
 __device__ __forceinline__ cplx c_wide(cplx a) { return a; }
 __device__ __forceinline__ cplx c_wide(float2 a) { return make_double2((double)a.x, (double)a.y); }
@@ -509,7 +498,6 @@ __device__ __forceinline__ const T2* rot_src(const Prob& p, int mode, int cur) {
   }
   return mbuf<T2>(p, cur);
 }
-__device__ __forceinline__ const cplx* rot_factor(const Prob& p, int, int) { return p.E; }
 
 // --------------------------------------------------------- M rotation
 
@@ -1554,8 +1542,7 @@ __device__ __forceinline__ int squarings(double r) {
 
 // C = A B or (adj) A^+ B on FP64 MFMA for matrices in global memory, by one
 // workgroup (w90gpu_mfma.h).
-__device__ void wg_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, double scale = 1.0,
-                             bool ident = false, bool adj = false);
+__device__ void wg_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, bool adj = false);
 
 // ET(k) = E(k)^T for one k by one workgroup (E written by this workgroup
 // before; the caller synchronised it): coalesced writes, reads along rows.
@@ -1575,7 +1562,7 @@ __global__ void __launch_bounds__(W90_NT) k_delta_u(const Prob* probs, const Ite
   const State* st = p.st;
   if (!gate(st, MODE_REMIX)) return;
   const size_t o = (size_t)it.k * p.nw2;
-  wg_gemm_mfma(p.E + o, p.U0 + o, p.U[st->cur] + o, p.nw, 1.0, false, true);
+  wg_gemm_mfma(p.E + o, p.U0 + o, p.U[st->cur] + o, p.nw, true);
   wg_transpose_e(p, it.k);
 }
 

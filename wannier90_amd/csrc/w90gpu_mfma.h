@@ -93,15 +93,6 @@ struct Real<float2> {
 };
 
 
-// output tile edge of a workgroup: 32 up to num_wann 32, 64 above
-__host__ __device__ __forceinline__ int gemm_edge(int nw) { return nw <= 32 ? 32 : 64; }
-
-// GEMM tiles per block M(k,b)
-__host__ __device__ __forceinline__ int gemm_tiles(int nw) {
-  const int t = (nw + gemm_edge(nw) - 1) / gemm_edge(nw);
-  return t * t;
-}
-
 // One GT x GT output tile (row0, col0) of one stage of the rotation of
 // block (k, b) by the workgroup (256 threads): operands and scratch as in
 // k_rot_gemm, LDS passed in.
@@ -1345,10 +1336,9 @@ __global__ void __launch_bounds__(64 * TN, kStepWaves(TN)) k_step_panel(const Pr
 // a time (independent accumulator chains), on FP64 MFMA with the operand
 // fragments loaded straight from memory (the matrices of one k stay in the
 // caches: A fragments read along a column, B fragments reuse cache lines
-// over consecutive K steps).  With ident, C = I + scale A B (one Taylor
-// step, applied as the product is stored); with adj, A^+ for A.  Used above
-// num_wann 64 and by the one-time kernels.
-__device__ void wg_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, double scale, bool ident, bool adj) {
+// over consecutive K steps).  With adj, A^+ for A.  Used by the retraction
+// above W90_PANEL_MAX bands and by the one-time kernels.
+__device__ void wg_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, bool adj) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nwv = blockDim.x >> 6;
   const int lr = lane & 15, lk = lane >> 4;
   const int nt = (n + 15) / 16;
@@ -1380,14 +1370,7 @@ __device__ void wg_gemm_mfma(cplx* C, const cplx* A, const cplx* B, int n, doubl
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r = i0[u] + Mfma<double>::row(lk, i), c = j0[u] + lr;
-        if (r < n && c < n) {
-          cplx v = c_make(cc[u].re(i), cc[u].im(i));
-          if (ident) {
-            v = c_scale(v, scale);
-            if (r == c) v.x += 1.0;
-          }
-          C[r + (size_t)c * n] = v;
-        }
+        if (r < n && c < n) C[r + (size_t)c * n] = c_make(cc[u].re(i), cc[u].im(i));
       }
     }
   }
@@ -1425,7 +1408,7 @@ __global__ void __launch_bounds__(W90_STEP_NT) k_polar(const Prob* probs, const 
   for (int e = threadIdx.x; e < nw2; e += blockDim.x) X[e] = c_scale(Ak[e], inv);
   __syncthreads();
   for (int iter = 0; iter < kPolarSteps; ++iter) {
-    wg_gemm_mfma(Y, X, X, nw, 1.0, false, true);
+    wg_gemm_mfma(Y, X, X, nw, true);
     double dev = 0.0;
     bool bad = false;
     for (int e = threadIdx.x; e < nw2; e += blockDim.x) {
