@@ -384,14 +384,18 @@ __device__ __forceinline__ void jacobi_item(int x, int half, int& r1, int& r2) {
 // one workgroup, 0.85 us at order 11; the LDS traffic of the blocks and rows
 // with two per CU, 1.1 us at order 39 (1.66 us when the rotations had a pass
 // of their own between two barriers and every wavefront did both parts).
-// k_dis_update per launch, before -> now: 48 bands to 24, 11 frozen, 512 k
-// 385 -> 250 us; 12 to 8, 64 k 68 -> 43 us; 80 to 40, 64 k, whose matrices
-// were both in global memory, 4.34 -> 0.87 ms.
+// k_dis_update per launch (average over a call, the cold first one with it),
+// before -> now: 48 bands to 24, 11 frozen, 512 k 384 -> 262 us; 12 to 8, 64 k 68
+// -> 42 us; 80 to 40, 64 k, whose matrices were both in global memory, 4.35 ->
+// 1.01 ms.
 //
 // theta false: sweeps until no pair rotates.  theta true: sweeps until every
 // angle left is at most 5e-9, where the rest of the method is the first-order
-// step E (1 + T), T_ij = a_ij / (a_jj - a_ii), to rounding (products of two
-// angles are below 2.5e-17); the caller applies it with its own product.  The
+// step E (1 + T), T_ij = a_ij / (a_jj - a_ii), to rounding: a product of two
+// angles is below 2.5e-17, and an entry of T^2, the first term left out, a sum
+// of at most n of them (1.6e-15 at order 64, 6.4e-15 at 256; what it takes from
+// E's orthonormality the next iteration's Newton-Schulz step puts back).  The
+// caller applies it with its own product.  The
 // sweeps are checked in one parallel pass before each.  Returns the number
 // of sweeps, or -1 if kMaxSweeps were not enough.  A warm start (a nearly
 // diagonal A) leaves off-diagonal entries just below the skip bounds, so they

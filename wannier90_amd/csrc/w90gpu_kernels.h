@@ -508,9 +508,15 @@ __device__ __forceinline__ const T2* rot_src(const Prob& p, int mode, int cur) {
 // the second time conjugate-transposed with its phases negated: half of the
 // MFMA products, which bound the kernel, and half of the reads of M.
 // Measured per rotation, every block formed -> by pairs: 64 bands, 800 k,
-// nntot 12 690 -> 419 us; 44, 343 k, 8 115 -> 78; 27, 216 k, 12 49 -> 38; 91,
-// 216 k, 6 372 -> 220.  FP32 storage (the mixed bulk phase) rotates every
-// block; up to 16 bands one workgroup forms all blocks of a k and its sums.
+// nntot 12 687 -> 412 us; 44, 384 k, 8 110 -> 64; 27, 216 k, 12 35 -> 21.7; 91,
+// 216 k, 6 370 -> 213; 128, 125 k, 6 483 -> 275.  FP32 storage (the mixed bulk
+// phase) rotates every block; up to 16 bands one workgroup forms all blocks of a
+// k and its sums.
+//
+// It is all blocks of a problem or none, so overlaps that went through text of
+// 12 decimals seldom qualify: one element whose two copies were rounded to
+// different last digits (1e-12, a hundred times the bound) is enough.  So is a
+// state that block-by-block rotations have moved for some hundred iterations.
 template <class T2>
 __device__ __forceinline__ int rot_pairs(const Prob& p) {
   return std::is_same<T2, cplx>::value ? p.npair : 0;
@@ -534,7 +540,7 @@ __device__ __forceinline__ int rot_slot(const Prob& p, int k, int j, int* mate) 
 // the products that formed the overlaps and of one rotation (so taking one
 // block of the pair for the other moves the result no more than a rotation
 // does).  NaN fails the test.  One pass over M0 through 32 x 32 tiles (the
-// transposed element of each comes from LDS): 0.2 ms for 64 bands, 800 k,
+// transposed element of each comes from LDS): 0.14 ms for 64 bands, 800 k,
 // nntot 12, once per load.
 __global__ void __launch_bounds__(W90_NT) k_check_pairs(Prob p, int npair, int* flag) {
   constexpr int TS = 32, RS = W90_NT / TS;
@@ -1470,9 +1476,9 @@ __device__ void search_control(State* st, double gg, double gd) {
 __device__ void search_in_step(const Prob& p, int k, State* lst, double* red) {
   constexpr int NSD = sizeof(State) / sizeof(double);
   // the partial sums are requested first, the state copy overlaps them;
-  // the k range is split over W90_NT lanes whatever the workgroup size
-  // (lanes beyond add exact zeros), so every retraction kernel forms the
-  // same sums
+  // the k range is split over the workgroup's lanes, at most W90_NT (lanes
+  // beyond add exact zeros): the sums' order is that of the kernel, and so of
+  // num_wann
   double gg = 0.0, gd = 0.0;
   const int nsplit = min((int)blockDim.x, W90_NT);
   const int per = (p.nk + nsplit - 1) / nsplit;

@@ -911,8 +911,8 @@ __device__ __forceinline__ void panel_product(const cplx* L, Get get, Out out) {
 // before a workgroup's products (7 us) and, at TN = 3, three wavefronts to four
 // SIMDs.  Measured per rotation by pairs against a workgroup per block with both
 // products staged through LDS in K chunks, two barriers a chunk (k_rot_fused):
-//   27 bands, 216 k: 27.2 -> 21.8 us   32 bands, 512 k: 30.4 -> 25.2 us
-//   44 bands, 343 k: 69.0 -> 61.0 us   48 bands, 216 k: 71.0 -> 64 us
+//   27 bands, 216 k, nntot 12: 27.2 -> 21.8 us   32, 512 k, 6: 30.4 -> 25.2 us
+//   44 bands, 343 k, nntot 8: 69.0 -> 61.0 us    48, 216 k, 12: 71.0 -> 64 us
 // With four panels the two operand panels, the accumulators and the loads in
 // flight pass the 256 registers: 76 -> 76 us at 52 bands and 404 -> 382 at 64
 // with scratch traffic, so 49-64 bands stay with k_rot_fused and k_rot_direct.
@@ -1130,10 +1130,11 @@ __global__ void __launch_bounds__(64 * TN, kStepWaves(TN)) k_rot_panel(const Pro
 // What bounds it: three products, the squarings and U E at the rate of the
 // FP64 MFMA pipe for 49-64 bands (four of 5 us per CU and k), the loads and
 // the search below.  Horner's form took a product per degree, 5 to 11 of
-// them, with both factors in LDS.  Measured on the same states, before -> now:
-// 16 bands, 512 k 9.9 -> 7.6 us; 27, 216 k 23.5 -> 12.9; 44, 343 k 53 -> 39;
-// 64, 800 k 180 -> 125; 91, 216 k 360 -> 168 (from k_step's form, all operands
-// in the caches).
+// them, with both factors in LDS.  Averages over the launches of a solve, before
+// -> now: 16 bands, 512 k 12.7 -> 10.6 us; 27, 216 k 26.2 -> 16.4; 44, 384 k 70
+// -> 47; 64, 800 k 205 -> 159; 91, 216 k 422 -> 200 (from k_step's form, all
+// operands in the caches).  Alone, without the search, the read of G and the
+// store of D, it takes 6.5, 12.7, 39, 126 and 167 us at these sizes.
 template <int TN>
 __global__ void __launch_bounds__(64 * TN, kStepWaves(TN)) k_step_panel(const Prob* probs, const Item* items,
                                                                        int nitems, int mode) {
